@@ -100,15 +100,12 @@ struct PcgGraph {
     }
 };
 
-// Linear BVH over surface primitives (lbvh.hip)
-struct LbvhTree {
-    int m = 0;
-    DBuf<char> leaf, scene, nodes, nbox, sort_tmp;  // boxes / nodes as raw bytes (types private to lbvh.hip)
-    DBuf<unsigned> code, idx, flags;
-    DBuf<unsigned long long> key;
-};
+// Linear BVHs over the surface triangles and edges (lbvh.hip), one after the
+// other in shared arrays
 struct Lbvh {
-    LbvhTree tri, edge;
+    DBuf<char> leaf, part, seg, nodes, sort_tmp;  // boxes and nodes as raw bytes (types private to lbvh.hip)
+    DBuf<unsigned> code, idx, hits;
+    DBuf<unsigned long long> key;
     DBuf<int> cnt, off, err;
 };
 

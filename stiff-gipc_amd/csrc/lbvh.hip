@@ -11,25 +11,36 @@
 // _reduct_max_box (:1062-1145), Morton keys _calcMChash (:1206-1225, 10 bits
 // per axis of the box centre in the scene box, original index in the low
 // 32 bits), Karras internal nodes _calcInternalNodes with determine_range /
-// find_split (:126-227, :1247-1267), bottom-up boxes _calcInternalAABB
+// find_split (:126-227, :1247-1267), internal boxes _calcInternalAABB
 // (:1269-1296), self queries _selfQuery_vf (:1306-1406) and _selfQuery_ee
 // (:1509-1632) with the reference's filters (point not in the face, edges
 // sharing no vertex and obj > self, not all four vertices of btype >= 2,
 // different bodies or body id -1) and box test `overlap` (:33-42).
+//
+// Both trees are built and queried by the same launches: their leaves are
+// sorted together (one tree bit above the 30-bit codes), and every kernel's
+// first workgroups take the triangles, the rest the edges.
+//
 // Differences: the reference appends pairs with an atomic counter while it
-// traverses; here each query counts its hits, an exclusive scan places
-// them, and a second traversal writes them, so the candidate order is
-// (query index, traversal order) -- deterministic.  The key sort is
-// rocPRIM's radix sort of the 30-bit codes with the leaf index as value
-// (stable), which orders exactly as the reference's 64-bit keys.
+// traverses; here each query counts its hits (and keeps the first kHits of
+// them), an exclusive scan places them, and a second launch writes them, so
+// the candidate order is (query index, traversal order) -- deterministic.
+// The reference climbs the tree with per-node arrival counters to merge the
+// boxes; a node of a Karras tree covers a contiguous range of the sorted
+// leaves, so here its box is a range query on a segment tree of leaf boxes:
+// no atomics, no release / acquire between XCDs per tree level.
 #include "context.hpp"
 #include <rocprim/device/device_radix_sort.hpp>
 
 namespace sgipc {
 namespace {
 
-constexpr unsigned kNone = 0xFFFFFFFFu;
+constexpr unsigned kLeaf = 0x80000000u;   // child code: kLeaf | primitive, else internal node
 constexpr int kStack = 64;
+constexpr int kQT = 64;                   // queries per workgroup (one wavefront)
+constexpr int kHits = 32;                 // hits per query kept by the counting pass
+constexpr int kPartBoxes = 256;           // partial scene boxes per tree, at most
+constexpr unsigned kCodeMask = (1u << 30) - 1u;
 
 struct Box {
     double lx, ly, lz, ux, uy, uz;
@@ -65,33 +76,100 @@ __device__ inline bool near(const Box& a, const Box& b, double gap) {
     return true;
 }
 
-struct Node {
-    unsigned left, right, parent, elem;
-};
 
-template <int K>
-__global__ void k_leaf_boxes(int m, const unsigned* __restrict__ prim, const double* __restrict__ x,
-                             const double* __restrict__ dir, double alpha, Box* __restrict__ box) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= m) return;
-    Box b = empty_box();
-#pragma unroll
-    for (int k = 0; k < K; ++k) grow_swept(b, x, dir, alpha, prim[K * (size_t)i + k]);
-    box[i] = b;
+// FP32 boxes rounded outward, for the internal nodes: a query box widened by
+// the gap and rounded outward too never misses a node that the FP64 test
+// would visit, and the leaves are tested in FP64, so the hits and their
+// order are those of FP64 boxes throughout.  They halve a node (both
+// children's boxes and codes in one 64-byte line: one load per visit).
+struct FBox {
+    float lx, ly, lz, ux, uy, uz;
+};
+__device__ inline float round_down(double d) {
+    const float f = (float)d;
+    return (double)f > d ? nextafterf(f, -INFINITY) : f;
+}
+__device__ inline float round_up(double d) {
+    const float f = (float)d;
+    return (double)f < d ? nextafterf(f, INFINITY) : f;
+}
+__device__ inline FBox empty_fbox() {
+    return FBox{INFINITY, INFINITY, INFINITY, -INFINITY, -INFINITY, -INFINITY};
+}
+__device__ inline FBox outward(const Box& b) {
+    return FBox{round_down(b.lx), round_down(b.ly), round_down(b.lz), round_up(b.ux), round_up(b.uy), round_up(b.uz)};
+}
+// the query box widened by gap, one more step outward for the rounding of the sums
+__device__ inline FBox query_box(const Box& b, double gap) {
+    return FBox{nextafterf(round_down(b.lx - gap), -INFINITY), nextafterf(round_down(b.ly - gap), -INFINITY),
+                nextafterf(round_down(b.lz - gap), -INFINITY), nextafterf(round_up(b.ux + gap), INFINITY),
+                nextafterf(round_up(b.uy + gap), INFINITY),   nextafterf(round_up(b.uz + gap), INFINITY)};
+}
+__device__ inline FBox merge(const FBox& a, const FBox& b) {
+    return FBox{fminf(a.lx, b.lx), fminf(a.ly, b.ly), fminf(a.lz, b.lz), fmaxf(a.ux, b.ux), fmaxf(a.uy, b.uy),
+                fmaxf(a.uz, b.uz)};
+}
+__device__ inline bool apart(const FBox& q, float lx, float ly, float lz, float ux, float uy, float uz) {
+    return lx > q.ux || ux < q.lx || ly > q.uy || uy < q.ly || lz > q.uz || uz < q.lz;
 }
 
-// scene box: per-block partial boxes, then one block merges them
-__global__ void __launch_bounds__(256) k_box_reduce(int m, const Box* __restrict__ in, Box* __restrict__ out) {
-    __shared__ Box sh[256];
-    Box b = empty_box();
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < m; i += gridDim.x * blockDim.x) b = merge(b, in[i]);
-    sh[threadIdx.x] = b;
-    __syncthreads();
-    for (int s = 128; s > 0; s >>= 1) {
-        if (threadIdx.x < s) sh[threadIdx.x] = merge(sh[threadIdx.x], sh[threadIdx.x + s]);
-        __syncthreads();
+struct alignas(64) QNode {
+    float4 a, b, c;       // left box (lx ly lz ux | uy uz), right box (lx ly | lz ux uy uz)
+    unsigned left, right; // child codes
+    unsigned pad[2];
+};
+
+// one tree's part of the shared arrays: m primitives from position base
+struct Tree {
+    int m, base;
+    const unsigned* prim;  // K vertex ids per primitive
+    int K;
+};
+struct Trees {
+    Tree t[2];   // triangles, edges
+    int nb0;     // workgroups of tree 0 in this launch
+    __device__ const Tree& mine(int& block) const {
+        block = (int)blockIdx.x;
+        if (block < nb0) return t[0];
+        block -= nb0;
+        return t[1];
     }
-    if (threadIdx.x == 0) out[blockIdx.x] = sh[0];
+};
+
+template <int NW>
+__device__ inline Box block_box(Box b, Box* sh) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        b.lx = fmin(b.lx, __shfl_xor(b.lx, off)); b.ly = fmin(b.ly, __shfl_xor(b.ly, off));
+        b.lz = fmin(b.lz, __shfl_xor(b.lz, off)); b.ux = fmax(b.ux, __shfl_xor(b.ux, off));
+        b.uy = fmax(b.uy, __shfl_xor(b.uy, off)); b.uz = fmax(b.uz, __shfl_xor(b.uz, off));
+    }
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = b;
+    __syncthreads();
+    b = sh[0];
+#pragma unroll
+    for (int w = 1; w < NW; ++w) b = merge(b, sh[w]);
+    return b;
+}
+
+// leaf boxes (FP64, in primitive order) and one partial scene box per workgroup
+__global__ void __launch_bounds__(256) k_leaf_boxes(Trees T, int stride0, int stride1, const double* __restrict__ x,
+                                                    const double* __restrict__ dir, double alpha,
+                                                    Box* __restrict__ leaf, Box* __restrict__ part) {
+    __shared__ Box sh[4];
+    int blk;
+    const Tree& t = T.mine(blk);
+    const bool tri = &t == &T.t[0];
+    const int stride = 256 * (tri ? stride0 : stride1);
+    Box all = empty_box();
+    for (int i = blk * 256 + (int)threadIdx.x; i < t.m; i += stride) {
+        Box b = empty_box();
+        for (int k = 0; k < t.K; ++k) grow_swept(b, x, dir, alpha, t.prim[t.K * (size_t)i + k]);
+        leaf[t.base + (size_t)i] = b;
+        all = merge(all, b);
+    }
+    all = block_box<4>(all, sh);
+    if (threadIdx.x == 0) part[(tri ? 0 : kPartBoxes) + blk] = all;
 }
 
 __device__ inline unsigned spread10(unsigned v) {
@@ -106,35 +184,97 @@ __device__ inline unsigned cell10(double t) {
     return (unsigned)t;
 }
 
-__global__ void k_morton(int m, const Box* __restrict__ box, const Box* __restrict__ scene, unsigned* __restrict__ code,
-                         unsigned* __restrict__ idx) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= m) return;
-    const Box S = *scene, b = box[i];
+// 30-bit Morton code of every leaf box's centre in its tree's scene box
+// (merged here from the partials), the tree bit above it
+__global__ void __launch_bounds__(256) k_morton(Trees T, int np0, int np1, const Box* __restrict__ leaf,
+                                                const Box* __restrict__ part, unsigned* __restrict__ code,
+                                                unsigned* __restrict__ idx) {
+    __shared__ Box sh[4];
+    int blk;
+    const Tree& t = T.mine(blk);
+    const bool tri = &t == &T.t[0];
+    const int np = tri ? np0 : np1;
+    const Box S = block_box<4>((int)threadIdx.x < np ? part[(tri ? 0 : kPartBoxes) + threadIdx.x] : empty_box(), sh);
+    const int i = blk * 256 + (int)threadIdx.x;
+    if (i >= t.m) return;
+    const Box b = leaf[t.base + (size_t)i];
     // a flat scene axis maps every centre to cell 0 on it
     double sx = S.ux - S.lx, sy = S.uy - S.ly, sz = S.uz - S.lz;
     double cx = 0.5 * (b.lx + b.ux) - S.lx, cy = 0.5 * (b.ly + b.uy) - S.ly, cz = 0.5 * (b.lz + b.uz) - S.lz;
     unsigned xx = spread10(sx > 0.0 ? cell10(cx / sx) : 0u);
     unsigned yy = spread10(sy > 0.0 ? cell10(cy / sy) : 0u);
     unsigned zz = spread10(sz > 0.0 ? cell10(cz / sz) : 0u);
-    code[i] = (xx << 2) + (yy << 1) + zz;
-    idx[i] = (unsigned)i;
+    code[t.base + (size_t)i] = ((xx << 2) + (yy << 1) + zz) | (tri ? 0u : kCodeMask + 1u);
+    idx[t.base + (size_t)i] = (unsigned)i;
 }
 
-// leaves at m-1 .. 2m-2 in sorted order; internal nodes 0 .. m-2
-__global__ void k_leaves(int m, const unsigned* __restrict__ sidx, const unsigned* __restrict__ scode,
-                         const Box* __restrict__ box, Node* __restrict__ nodes, Box* __restrict__ nbox,
-                         unsigned long long* __restrict__ key, unsigned* __restrict__ flags) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= m) return;
-    const unsigned e = sidx[i];
-    nodes[m - 1 + i] = Node{kNone, kNone, kNone, e};
-    nbox[m - 1 + i] = box[e];
-    key[i] = ((unsigned long long)scode[i] << 32) | e;
-    if (i < m - 1) {
-        nodes[i] = Node{kNone, kNone, kNone, kNone};
-        flags[i] = 0u;
+// Segment tree over a tree's sorted leaf boxes: level k holds the merged
+// boxes of aligned runs of 2^k leaves, ceil(m / 2^k) of them; a tree's
+// levels lie one after the other from 2 * base + 64 * tree.
+__device__ inline size_t seg_base(const Tree& t, bool tri) { return 2 * (size_t)t.base + (tri ? 0 : 64); }
+__device__ inline int seg_count(int m, int k) { return (int)(((long long)m + (1ll << k) - 1) >> k); }
+
+// sorted leaves: keys, level 0 of the segment tree, and its levels 1 to 8 (a
+// workgroup's 256 leaves are one run of level 8)
+__global__ void __launch_bounds__(256) k_leaves(Trees T, const unsigned* __restrict__ sidx,
+                                                const unsigned* __restrict__ scode, const Box* __restrict__ leaf,
+                                                FBox* __restrict__ seg, unsigned long long* __restrict__ key) {
+    __shared__ FBox sh[256];
+    int blk;
+    const Tree& t = T.mine(blk);
+    const bool tri = &t == &T.t[0];
+    const int tid = (int)threadIdx.x, i = blk * 256 + tid;
+    FBox b = empty_fbox();
+    FBox* lv = seg + seg_base(t, tri);
+    if (i < t.m) {
+        const unsigned e = sidx[t.base + (size_t)i];
+        key[t.base + (size_t)i] = ((unsigned long long)(scode[t.base + (size_t)i] & kCodeMask) << 32) | e;
+        b = outward(leaf[t.base + (size_t)e]);
+        lv[i] = b;
     }
+    sh[tid] = b;
+#pragma unroll
+    for (int k = 1; k <= 8; ++k) {
+        lv += seg_count(t.m, k - 1);
+        __syncthreads();
+        if (tid < (256 >> k)) b = merge(sh[2 * tid], sh[2 * tid + 1]);
+        __syncthreads();
+        if (tid < (256 >> k)) {
+            sh[tid] = b;
+            const int q = blk * (256 >> k) + tid;
+            if (q < seg_count(t.m, k)) lv[q] = b;
+        }
+    }
+}
+
+// levels 9 and up, one workgroup per tree
+__global__ void __launch_bounds__(1024) k_seg_top(Trees T, FBox* __restrict__ seg) {
+    int blk;
+    const Tree& t = T.mine(blk);
+    const FBox* lo = seg + seg_base(t, &t == &T.t[0]);
+    for (int k = 0; k < 8; ++k) lo += seg_count(t.m, k);
+    for (int k = 9; seg_count(t.m, k - 1) > 1; ++k) {
+        const int below = seg_count(t.m, k - 1), n = seg_count(t.m, k);
+        FBox* hi = const_cast<FBox*>(lo) + below;
+        for (int q = (int)threadIdx.x; q < n; q += 1024)
+            hi[q] = 2 * q + 1 < below ? merge(lo[2 * q], lo[2 * q + 1]) : lo[2 * q];
+        __syncthreads();  // this workgroup's stores are read by its next level
+        lo = hi;
+    }
+}
+
+// merged box of the sorted leaves lo .. hi
+__device__ inline FBox range_box(const FBox* __restrict__ lv, int m, int lo, int hi) {
+    FBox b = empty_fbox();
+    int l = lo, r = hi + 1;
+    for (int k = 0; l < r; ++k) {
+        if (l & 1) b = merge(b, lv[l++]);
+        if (r & 1) b = merge(b, lv[--r]);
+        lv += seg_count(m, k);
+        l >>= 1;
+        r >>= 1;
+    }
+    return b;
 }
 
 __device__ inline int prefix(const unsigned long long* __restrict__ key, int m, int i, int j) {
@@ -142,10 +282,17 @@ __device__ inline int prefix(const unsigned long long* __restrict__ key, int m, 
     return __clzll(key[i] ^ key[j]);
 }
 
-// Karras (2012) radix-tree construction over the unique sorted keys
-__global__ void k_internal(int m, const unsigned long long* __restrict__ key, Node* __restrict__ nodes) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
+// Karras (2012) radix-tree construction over the unique sorted keys: internal
+// node i covers the leaves lo .. hi split after gamma; its two children's
+// boxes come from the segment tree
+__global__ void __launch_bounds__(256) k_internal(Trees T, const unsigned long long* __restrict__ keys,
+                                                  const unsigned* __restrict__ sidx, const FBox* __restrict__ seg,
+                                                  QNode* __restrict__ nodes) {
+    int blk;
+    const Tree& tr = T.mine(blk);
+    const int m = tr.m, i = blk * 256 + (int)threadIdx.x;
     if (i >= m - 1) return;
+    const unsigned long long* key = keys + tr.base;
     const int d = (prefix(key, m, i, i + 1) - prefix(key, m, i, i - 1)) > 0 ? 1 : -1;
     const int dmin = prefix(key, m, i, i - d);
     int lmax = 2;
@@ -162,63 +309,56 @@ __global__ void k_internal(int m, const unsigned long long* __restrict__ key, No
     } while (t > 1);
     const int gamma = i + s * d + min(d, 0);
     const int lo = min(i, j), hi = max(i, j);
-    const unsigned left = (lo == gamma) ? (unsigned)(gamma + m - 1) : (unsigned)gamma;
-    const unsigned right = (hi == gamma + 1) ? (unsigned)(gamma + 1 + m - 1) : (unsigned)(gamma + 1);
-    nodes[i].left = left;
-    nodes[i].right = right;
-    nodes[left].parent = (unsigned)i;
-    nodes[right].parent = (unsigned)i;
+    const FBox* lv = seg + seg_base(tr, &tr == &T.t[0]);
+    const FBox L = range_box(lv, m, lo, gamma), R = range_box(lv, m, gamma + 1, hi);
+    QNode n;
+    n.a = make_float4(L.lx, L.ly, L.lz, L.ux);
+    n.b = make_float4(L.uy, L.uz, R.lx, R.ly);
+    n.c = make_float4(R.lz, R.ux, R.uy, R.uz);
+    n.left = lo == gamma ? (kLeaf | sidx[tr.base + (size_t)gamma]) : (unsigned)gamma;
+    n.right = hi == gamma + 1 ? (kLeaf | sidx[tr.base + (size_t)gamma + 1]) : (unsigned)(gamma + 1);
+    n.pad[0] = n.pad[1] = 0u;
+    nodes[tr.base + (size_t)i] = n;
 }
 
-// bottom-up boxes: the second child to arrive at a parent merges it
-__global__ void k_internal_boxes(int m, const Node* __restrict__ nodes, Box* __restrict__ nbox,
-                                 unsigned* __restrict__ flags) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= m) return;
-    unsigned p = nodes[m - 1 + i].parent;
-    while (p != kNone) {
-        __threadfence();
-        if (atomicAdd(flags + p, 1u) == 0u) return;  // the sibling's thread finishes this parent
-        __threadfence();
-        const Node n = nodes[p];
-        nbox[p] = merge(nbox[n.left], nbox[n.right]);
-        p = n.parent;
-    }
-}
-
-struct QueryCtx {
-    const Node* nodes;
-    const Box* box;
-    int m;
-    double gap;
-};
-
-// visit every leaf whose box is near q (root 0; a single leaf when m == 1)
+// visit every leaf whose FP32 box is near the query, depth first: a leaf
+// child at once, of two internal children the right one first.  stk: this
+// lane's column of the wavefront's LDS stack.
 template <typename F>
-__device__ inline bool traverse(const QueryCtx& Q, const Box& q, F&& on_leaf) {
-    if (Q.m == 1) {
-        if (near(q, Q.box[0], Q.gap)) on_leaf(Q.nodes[0].elem);
+__device__ inline bool traverse(const QNode* __restrict__ nodes, int m, unsigned only, const FBox& q, unsigned* stk,
+                                F&& on_leaf) {
+    if (m == 1) {
+        on_leaf(only);
         return true;
     }
-    unsigned stack[kStack];
     int sp = 0;
-    stack[sp++] = 0;
-    while (sp > 0) {
-        const Node n = Q.nodes[stack[--sp]];
-        const unsigned ch[2] = {n.left, n.right};
-#pragma unroll
-        for (int c = 0; c < 2; ++c) {
-            if (!near(q, Q.box[ch[c]], Q.gap)) continue;
-            const unsigned e = Q.nodes[ch[c]].elem;
-            if (e != kNone) {
-                on_leaf(e);
+    unsigned cur = 0;
+    for (;;) {
+        const QNode n = nodes[cur];
+        const bool hl = !apart(q, n.a.x, n.a.y, n.a.z, n.a.w, n.b.x, n.b.y);
+        const bool hr = !apart(q, n.b.z, n.b.w, n.c.x, n.c.y, n.c.z, n.c.w);
+        unsigned next = kLeaf;  // none
+        if (hl) {
+            if (n.left & kLeaf) on_leaf(n.left & ~kLeaf);
+            else next = n.left;
+        }
+        if (hr) {
+            if (n.right & kLeaf) {
+                on_leaf(n.right & ~kLeaf);
             } else {
-                if (sp >= kStack) return false;
-                stack[sp++] = ch[c];
+                if (next != kLeaf) {
+                    if (sp >= kStack) return false;
+                    stk[kQT * sp++] = next;
+                }
+                next = n.right;
             }
         }
+        if (next == kLeaf) {
+            if (sp == 0) return true;
+            next = stk[kQT * --sp];
+        }
+        cur = next;
     }
-    return true;
 }
 
 __device__ inline bool all_static(const int* __restrict__ bt, unsigned a, unsigned b, unsigned c, unsigned d) {
@@ -228,155 +368,161 @@ __device__ inline bool other_body(const int* __restrict__ body, unsigned a, unsi
     return !body || body[a] == -1 || body[a] != body[b];
 }
 
-// pass 0 counts hits per query, pass 1 writes them at the scanned offsets
-template <int PASS>
-__global__ void k_query_vf(int nq, const unsigned* __restrict__ sv, const unsigned* __restrict__ faces,
-                           const double* __restrict__ x, const double* __restrict__ dir, double alpha, QueryCtx Q,
-                           const int* __restrict__ bt,
-                           const int* __restrict__ body, int* __restrict__ cnt, const int* __restrict__ off,
-                           int4* __restrict__ out, int cap, int* __restrict__ err) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nq) return;
-    const unsigned p = sv[i];
-    Box q = empty_box();
-    grow_swept(q, x, dir, alpha, p);
-    int k = 0;
-    const int base = PASS ? off[i] : 0;
-    bool ok = traverse(Q, q, [&](unsigned f) {
-        const unsigned a = faces[3 * (size_t)f], b = faces[3 * (size_t)f + 1], c = faces[3 * (size_t)f + 2];
-        if (p == a || p == b || p == c) return;
-        if (!other_body(body, p, a) || all_static(bt, p, a, b, c)) return;
-        if (PASS && base + k < cap) out[base + k] = make_int4((int)p, (int)a, (int)b, (int)c);
-        ++k;
-    });
-    if (!ok) atomicOr(err, 1);
-    if (!PASS) cnt[i] = k;
-}
+struct Query {
+    int nsv, nbv;                // point queries and their workgroups (before the edges' ones)
+    const unsigned* sv;
+    const double *x, *dir;
+    double alpha, gap;
+    const Box* leaf;
+    const QNode* nodes;
+    const unsigned* sidx;        // sorted primitive ids
+    const int *bt, *body;
+    int* cnt;                    // hits per query: points, then edges
+    const int* off;              // their exclusive scan (pass 1)
+    unsigned* hits;              // kHits per query slot, slot fastest
+    int4 *pt_out, *ee_out;       // pass 1: null when the list does not fit
+    int pt_cap, ee_cap;
+    int* err;
+};
 
+// Pass 0 counts the hits of every query and keeps the first kHits; pass 1
+// writes them at the scanned offsets and traverses again only for a query
+// with more.  The edge queries run in sorted (Morton) order, so the lanes of
+// a wavefront walk nearby parts of the tree; counts and output are by edge.
 template <int PASS>
-__global__ void k_query_ee(int ne, const unsigned* __restrict__ edges, const Box* __restrict__ ebox, QueryCtx Q,
-                           const int* __restrict__ bt, const int* __restrict__ body, int* __restrict__ cnt,
-                           const int* __restrict__ off, int4* __restrict__ out, int cap, int* __restrict__ err) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= ne) return;
-    const unsigned a0 = edges[2 * (size_t)i], a1 = edges[2 * (size_t)i + 1];
-    const Box q = ebox[i];  // edge i's own box (leaf boxes are kept in edge order)
+__global__ void __launch_bounds__(kQT) k_query(Trees T, Query Q) {
+    __shared__ unsigned stack[kStack * kQT];
+    unsigned* stk = stack + threadIdx.x;
+    const size_t slot = (size_t)blockIdx.x * kQT + threadIdx.x, nslots = (size_t)gridDim.x * kQT;
+    const bool vf = (int)blockIdx.x < Q.nbv;
+    const Tree& t = vf ? T.t[0] : T.t[1];
+    const unsigned* prim = t.prim;
+    int i = (int)slot - (vf ? 0 : Q.nbv * kQT);
+    if (i >= (vf ? Q.nsv : t.m)) return;
+    if (!vf) i = (int)Q.sidx[t.base + (size_t)i];
+    int4* out = vf ? Q.pt_out : Q.ee_out;
+    if (PASS && !out) return;
+    const int cap = vf ? Q.pt_cap : Q.ee_cap, qi = vf ? i : Q.nsv + i;
+    // the query's vertices: the point, or the edge's ends
+    const unsigned a0 = vf ? Q.sv[i] : prim[2 * (size_t)i], a1 = vf ? a0 : prim[2 * (size_t)i + 1];
+    auto emit = [&](int pos, unsigned e) {
+        if (pos >= cap) return;
+        if (vf) out[pos] = make_int4((int)a0, (int)prim[3 * (size_t)e], (int)prim[3 * (size_t)e + 1], (int)prim[3 * (size_t)e + 2]);
+        else out[pos] = make_int4((int)a0, (int)a1, (int)prim[2 * (size_t)e], (int)prim[2 * (size_t)e + 1]);
+    };
+    int base = 0, total = 0;
+    if (PASS) {
+        base = Q.off[qi] - (vf ? 0 : Q.off[Q.nsv]);
+        total = Q.cnt[qi];
+        for (int k = 0; k < min(total, kHits); ++k) emit(base + k, Q.hits[(size_t)k * nslots + slot]);
+        if (total <= kHits) return;
+    }
+    Box q = empty_box();
+    if (vf) grow_swept(q, Q.x, Q.dir, Q.alpha, a0);
+    else q = Q.leaf[t.base + (size_t)i];  // edge i's own box (leaf boxes are kept in edge order)
     int k = 0;
-    const int base = PASS ? off[i] : 0;
-    bool ok = traverse(Q, q, [&](unsigned o) {
-        if (o <= (unsigned)i) return;
-        const unsigned b0 = edges[2 * (size_t)o], b1 = edges[2 * (size_t)o + 1];
-        if (a0 == b0 || a0 == b1 || a1 == b0 || a1 == b1) return;
-        if (!other_body(body, a0, b0) || all_static(bt, a0, a1, b0, b1)) return;
-        if (PASS && base + k < cap) out[base + k] = make_int4((int)a0, (int)a1, (int)b0, (int)b1);
+    const bool ok = traverse(Q.nodes + t.base, t.m, t.m == 1 ? Q.sidx[t.base] : 0u, query_box(q, Q.gap), stk,
+                             [&](unsigned e) {
+        if (!vf && e <= (unsigned)i) return;
+        if (!near(q, Q.leaf[t.base + (size_t)e], Q.gap)) return;
+        if (vf) {
+            const unsigned a = prim[3 * (size_t)e], b = prim[3 * (size_t)e + 1], c = prim[3 * (size_t)e + 2];
+            if (a0 == a || a0 == b || a0 == c) return;
+            if (!other_body(Q.body, a0, a) || all_static(Q.bt, a0, a, b, c)) return;
+        } else {
+            const unsigned b0 = prim[2 * (size_t)e], b1 = prim[2 * (size_t)e + 1];
+            if (a0 == b0 || a0 == b1 || a1 == b0 || a1 == b1) return;
+            if (!other_body(Q.body, a0, b0) || all_static(Q.bt, a0, a1, b0, b1)) return;
+        }
+        if (!PASS) {
+            if (k < kHits) Q.hits[(size_t)k * nslots + slot] = e;
+        } else if (k >= kHits) {
+            emit(base + k, e);
+        }
         ++k;
     });
-    if (!ok) atomicOr(err, 1);
-    if (!PASS) cnt[i] = k;
+    if (!ok) atomicOr(Q.err, 1);
+    if (!PASS) Q.cnt[qi] = k;
 }
 
 }  // namespace
-
-// Builds the tree over m primitives of K vertices into t (boxes, nodes).
-template <int K>
-static void lbvh_build(Ctx& c, LbvhTree& t, int m, const unsigned* prim, const double* x, const double* dir,
-                       double alpha) {
-    hipStream_t s = c.stream;
-    t.m = m;
-    if (m <= 0) return;
-    Box* leaf = (Box*)t.leaf.reserve((size_t)m * sizeof(Box));
-    hipLaunchKernelGGL(k_leaf_boxes<K>, dim3(div_up(m, 256)), dim3(256), 0, s, m, prim, x, dir, alpha, leaf);
-    SGIPC_LAUNCH_CHECK();
-    const int gb = std::max(1, std::min(256, (int)div_up(m, 256)));
-    Box* part = (Box*)t.scene.reserve((size_t)(gb + 1) * sizeof(Box));
-    hipLaunchKernelGGL(k_box_reduce, dim3(gb), dim3(256), 0, s, m, (const Box*)leaf, part);
-    SGIPC_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_box_reduce, dim3(1), dim3(256), 0, s, gb, (const Box*)part, part + gb);
-    SGIPC_LAUNCH_CHECK();
-    unsigned* code = t.code.reserve(2 * (size_t)m);
-    unsigned* idx = t.idx.reserve(2 * (size_t)m);
-    hipLaunchKernelGGL(k_morton, dim3(div_up(m, 256)), dim3(256), 0, s, m, (const Box*)leaf,
-                       (const Box*)(part + gb), code, idx);
-    SGIPC_LAUNCH_CHECK();
-    if (c.sort_impl == SORT_OWN) {
-        radix_sort_pairs(c, code, code + m, (const int*)idx, 0, (int*)(idx + m), m, 30, s);
-    } else {  // rocPRIM as the cross-check
-        size_t bytes = 0;
-        SGIPC_HIP(rocprim::radix_sort_pairs(nullptr, bytes, code, code + m, idx, idx + m, (unsigned)m, 0, 30, s));
-        void* tmp = t.sort_tmp.reserve(bytes + 1);
-        SGIPC_HIP(rocprim::radix_sort_pairs(tmp, bytes, code, code + m, idx, idx + m, (unsigned)m, 0, 30, s));
-    }
-    Node* nodes = (Node*)t.nodes.reserve((size_t)(2 * m - 1) * sizeof(Node));
-    Box* nbox = (Box*)t.nbox.reserve((size_t)(2 * m - 1) * sizeof(Box));
-    unsigned long long* key = t.key.reserve((size_t)m);
-    unsigned* flags = t.flags.reserve((size_t)m);
-    hipLaunchKernelGGL(k_leaves, dim3(div_up(m, 256)), dim3(256), 0, s, m, (const unsigned*)(idx + m),
-                       (const unsigned*)(code + m), (const Box*)leaf, nodes, nbox, key, flags);
-    SGIPC_LAUNCH_CHECK();
-    if (m > 1) {
-        hipLaunchKernelGGL(k_internal, dim3(div_up(m - 1, 256)), dim3(256), 0, s, m,
-                           (const unsigned long long*)key, nodes);
-        SGIPC_LAUNCH_CHECK();
-        hipLaunchKernelGGL(k_internal_boxes, dim3(div_up(m, 256)), dim3(256), 0, s, m, (const Node*)nodes, nbox,
-                           flags);
-        SGIPC_LAUNCH_CHECK();
-    }
-}
 
 void broad_phase(Ctx& c, int nsv, const unsigned* sv, int nf, const unsigned* faces, int ne, const unsigned* edges,
                  const double* x, const int* btype, const int* body, double dhat, int* pt_out, int pt_cap, int& n_pt,
                  int* ee_out, int ee_cap, int& n_ee, const double* dir, double alpha) {
     if (!(dhat > 0.0)) throw arg_error("broad_phase: dhat must be positive");
     hipStream_t s = c.stream;
-    const double gap = sqrt(dhat);
     Lbvh& B = c.lbvh;
+    n_pt = n_ee = 0;
+    const bool pt = nsv > 0 && nf > 0, ee = ne > 1;
+    if (!pt) nsv = 0;
+    const int mt = pt ? nf : 0, me = ee ? ne : 0, M = mt + me;
+    if (M == 0) return;
+    Trees T{{Tree{mt, 0, faces, 3}, Tree{me, mt, edges, 2}}, 0};
+    auto blocks = [&](int per) {  // workgroups of `per` leaves, triangles first
+        T.nb0 = (int)div_up(mt, per);
+        return dim3((unsigned)(T.nb0 + (int)div_up(me, per)));
+    };
     int* err = B.err.reserve(1);
     fill<int>(err, 0, 1, s);
-    n_pt = n_ee = 0;
-    int hcount[2] = {0, 0};
-    // point - triangle
-    if (nsv > 0 && nf > 0) {
-        lbvh_build<3>(c, B.tri, nf, faces, x, dir, alpha);
-        QueryCtx Q{(const Node*)B.tri.nodes.p, (const Box*)B.tri.nbox.p, nf, gap};
-        int* cnt = B.cnt.reserve((size_t)nsv + 1);
-        int* off = B.off.reserve((size_t)nsv + 1);
-        hipLaunchKernelGGL(k_query_vf<0>, dim3(div_up(nsv, 128)), dim3(128), 0, s, nsv, sv, faces, x, dir, alpha, Q,
-                           btype, body, cnt, (const int*)nullptr, (int4*)nullptr, 0, err);
-        SGIPC_LAUNCH_CHECK();
-        exclusive_scan(c, cnt, off, nsv, nullptr, s);
-        SGIPC_HIP(hipMemcpyAsync(&hcount[0], off + nsv, sizeof(int), hipMemcpyDeviceToHost, s));
-        SGIPC_HIP(hipStreamSynchronize(s));
-        if (hcount[0] <= pt_cap && hcount[0] > 0) {
-            hipLaunchKernelGGL(k_query_vf<1>, dim3(div_up(nsv, 128)), dim3(128), 0, s, nsv, sv, faces, x, dir, alpha,
-                               Q, btype, body, cnt, (const int*)off, (int4*)pt_out, pt_cap, err);
-            SGIPC_LAUNCH_CHECK();
-        }
+    Box* leaf = (Box*)B.leaf.reserve((size_t)M * sizeof(Box));
+    Box* part = (Box*)B.part.reserve(2 * kPartBoxes * sizeof(Box));
+    unsigned* code = B.code.reserve(2 * (size_t)M);
+    unsigned* idx = B.idx.reserve(2 * (size_t)M);
+    unsigned long long* key = B.key.reserve((size_t)M);
+    FBox* seg = (FBox*)B.seg.reserve((2 * (size_t)M + 128) * sizeof(FBox));
+    QNode* nodes = (QNode*)B.nodes.reserve((size_t)M * sizeof(QNode));
+    const int np0 = std::min(kPartBoxes, (int)div_up(mt, 256)), np1 = std::min(kPartBoxes, (int)div_up(me, 256));
+    T.nb0 = np0;
+    hipLaunchKernelGGL(k_leaf_boxes, dim3(np0 + np1), dim3(256), 0, s, T, np0, np1, x, dir, alpha, leaf, part);
+    SGIPC_LAUNCH_CHECK();
+    const dim3 g256 = blocks(256);
+    hipLaunchKernelGGL(k_morton, g256, dim3(256), 0, s, T, np0, np1, (const Box*)leaf, (const Box*)part, code, idx);
+    SGIPC_LAUNCH_CHECK();
+    if (c.sort_impl == SORT_OWN) {
+        radix_sort_pairs(c, code, code + M, (const int*)idx, 0, (int*)(idx + M), M, 31, s);
+    } else {  // rocPRIM as the cross-check
+        size_t bytes = 0;
+        SGIPC_HIP(rocprim::radix_sort_pairs(nullptr, bytes, code, code + M, idx, idx + M, (unsigned)M, 0, 31, s));
+        void* tmp = B.sort_tmp.reserve(bytes + 1);
+        SGIPC_HIP(rocprim::radix_sort_pairs(tmp, bytes, code, code + M, idx, idx + M, (unsigned)M, 0, 31, s));
     }
-    // edge - edge
-    if (ne > 1) {
-        lbvh_build<2>(c, B.edge, ne, edges, x, dir, alpha);
-        const Box* ebox = (const Box*)B.edge.leaf.p;  // leaf boxes in edge order
-        QueryCtx Q{(const Node*)B.edge.nodes.p, (const Box*)B.edge.nbox.p, ne, gap};
-        int* cnt = B.cnt.reserve((size_t)ne + 1);
-        int* off = B.off.reserve((size_t)ne + 1);
-        hipLaunchKernelGGL(k_query_ee<0>, dim3(div_up(ne, 128)), dim3(128), 0, s, ne, edges, ebox, Q, btype, body,
-                           cnt, (const int*)nullptr, (int4*)nullptr, 0, err);
+    const unsigned* sidx = idx + M;
+    hipLaunchKernelGGL(k_leaves, g256, dim3(256), 0, s, T, sidx, (const unsigned*)(code + M), (const Box*)leaf, seg,
+                       key);
+    SGIPC_LAUNCH_CHECK();
+    if (std::max(mt, me) > 256) {
+        T.nb0 = mt > 0 ? 1 : 0;
+        hipLaunchKernelGGL(k_seg_top, dim3(T.nb0 + (me > 0 ? 1 : 0)), dim3(1024), 0, s, T, seg);
         SGIPC_LAUNCH_CHECK();
-        exclusive_scan(c, cnt, off, ne, nullptr, s);
-        SGIPC_HIP(hipMemcpyAsync(&hcount[1], off + ne, sizeof(int), hipMemcpyDeviceToHost, s));
-        SGIPC_HIP(hipStreamSynchronize(s));
-        if (hcount[1] <= ee_cap && hcount[1] > 0) {
-            hipLaunchKernelGGL(k_query_ee<1>, dim3(div_up(ne, 128)), dim3(128), 0, s, ne, edges, ebox, Q, btype,
-                               body, cnt, (const int*)off, (int4*)ee_out, ee_cap, err);
-            SGIPC_LAUNCH_CHECK();
-        }
     }
-    int herr = 0;
-    SGIPC_HIP(hipMemcpyAsync(&herr, err, sizeof(int), hipMemcpyDeviceToHost, s));
+    (void)blocks(256);
+    hipLaunchKernelGGL(k_internal, g256, dim3(256), 0, s, T, (const unsigned long long*)key, sidx, (const FBox*)seg,
+                       nodes);
+    SGIPC_LAUNCH_CHECK();
+    const int nq = nsv + me, nbv = (int)div_up(nsv, kQT), nbq = nbv + (int)div_up(me, kQT);
+    int* cnt = B.cnt.reserve((size_t)nq + 1);
+    int* off = B.off.reserve((size_t)nq + 1);
+    Query Q{nsv, nbv, sv, x, dir, alpha, sqrt(dhat), leaf, nodes, sidx, btype, body, cnt, off,
+            B.hits.reserve((size_t)kHits * nbq * kQT), nullptr, nullptr, pt_cap, ee_cap, err};
+    hipLaunchKernelGGL(k_query<0>, dim3(nbq), dim3(kQT), 0, s, T, Q);
+    SGIPC_LAUNCH_CHECK();
+    exclusive_scan(c, cnt, off, nq, nullptr, s);
+    int h[3] = {0, 0, 0};  // point-triangle hits, all hits, traversal error
+    SGIPC_HIP(hipMemcpyAsync(&h[0], off + nsv, sizeof(int), hipMemcpyDeviceToHost, s));
+    SGIPC_HIP(hipMemcpyAsync(&h[1], off + nq, sizeof(int), hipMemcpyDeviceToHost, s));
+    SGIPC_HIP(hipMemcpyAsync(&h[2], err, sizeof(int), hipMemcpyDeviceToHost, s));
     SGIPC_HIP(hipStreamSynchronize(s));
-    if (herr) throw state_error("broad_phase: BVH traversal stack exceeded");
-    n_pt = hcount[0];
-    n_ee = hcount[1];
+    if (h[2]) throw state_error("broad_phase: BVH traversal stack exceeded");
+    n_pt = h[0];
+    n_ee = h[1] - h[0];
+    Q.pt_out = n_pt > 0 && n_pt <= pt_cap ? (int4*)pt_out : nullptr;
+    Q.ee_out = n_ee > 0 && n_ee <= ee_cap ? (int4*)ee_out : nullptr;
+    if (Q.pt_out || Q.ee_out) {
+        hipLaunchKernelGGL(k_query<1>, dim3(nbq), dim3(kQT), 0, s, T, Q);
+        SGIPC_LAUNCH_CHECK();
+        SGIPC_HIP(hipStreamSynchronize(s));
+    }
 }
 
 }  // namespace sgipc

@@ -139,3 +139,30 @@ def test_ccd_candidates_and_step_bound(torch_cuda, oracle, twobox8):
     for q in een[:: max(1, len(een) // 400)]:
         d0 = _seg_seg_d(*x0[q])
         assert _seg_seg_d(*x1[q]) >= 0.04 * d0 * (1 - 1e-9)
+
+
+@pytest.mark.parametrize("nf,ne,nsv,scale", [(1, 2, 5, 1.0), (0, 3, 4, 400.0), (2, 1, 9, 400.0), (255, 257, 65, 1.0),
+                                             (256, 256, 64, 1e4), (257, 513, 63, 4e4), (None, None, None, 1e5)])
+def test_tree_sizes_and_many_hits(torch_cuda, twobox8, nf, ne, nsv, scale):
+    """Tree sizes around a workgroup's run of leaves, one tree only, and gaps
+    so wide that queries have more hits than the counting pass keeps; lists
+    and order are compared with the brute force (order: by query)."""
+    from broad_phase_ref import candidates
+    sc, sysm, (faces, edges, surf) = twobox8
+    print("case: broad phase sizes", nf, ne, nsv, scale, flush=True)
+    rng = np.random.default_rng(11)
+    f = faces[rng.permutation(len(faces))[:nf]]
+    e = edges[np.sort(rng.permutation(len(edges))[:ne])]
+    v = surf[np.sort(rng.permutation(len(surf))[:nsv])]
+    dhat = scale * sc.dhat
+    pt, ee = _broad(torch_cuda, sysm, f, e, v, dhat, cap=(1 << 20, 1 << 21))
+    rpt, ree = candidates(sc.x, f, e, v, dhat)
+    if len(e) < 2:
+        ree = ree[:0]
+    assert sorted(map(tuple, pt)) == sorted(map(tuple, rpt)) and sorted(map(tuple, ee)) == sorted(map(tuple, ree))
+    assert (np.diff(pt[:, 0]) >= 0).all() if len(pt) else True
+    if len(ee):
+        first = {tuple(q): i for i, q in reversed(list(enumerate(map(tuple, e))))}
+        assert (np.diff([first[tuple(q[:2])] for q in ee]) >= 0).all()
+    if scale == 1e5:
+        assert np.bincount(pt[:, 0]).max() > 32 and len(ee) > 32 * len(e)

@@ -5,8 +5,8 @@
 // a single read of the keys, one exclusive scan of those histograms (the
 // first output position of every digit), then per pass one "onesweep"
 // kernel (Adinets and Merrill, "Onesweep: A Faster Least Significant Digit
-// Radix Sort for GPUs", 2022): each workgroup takes the next tile of 4096
-// keys from a counter, ranks its keys by digit (stable: wave-striped rounds
+// Radix Sort for GPUs", 2022): each workgroup takes the next tile of 1024
+// to 4096 keys from a counter, ranks its keys by digit (stable: wave-striped rounds
 // of 64 consecutive keys, equal digits matched with eight ballots), publishes
 // the tile's digit counts and looks back over the earlier tiles' published
 // counts for its global offsets (decoupled look-back), then stages the tile
@@ -27,12 +27,18 @@ namespace {
 
 constexpr int kRT = 256;               // threads per workgroup (one per digit)
 constexpr int kRW = kRT / 64;          // wavefronts
-constexpr int kRI = 16;                // keys per thread
-constexpr int kRTile = kRT * kRI;      // 4096 keys per tile
+// Keys per thread (16, 8 or 4: tiles of 4096, 2048 or 1024): a pass over few
+// tiles is one tile's latency (its ranking rounds are serial), so inputs that
+// would give fewer than kTilesWanted tiles take shorter ones.  Per pass, tiles
+// of 4096 against 1024: 77 k 32-bit keys 13.8 against 10.2 us, 30 k 64-bit
+// keys 14.3 against 7.9 us, but 727 k 64-bit keys 18 against 27 us (more
+// tiles to look back over and shorter output runs).
+constexpr int kTilesWanted = 128;
 constexpr unsigned kAgg = 1u << 30;    // tile count published
 constexpr unsigned kPre = 2u << 30;    // inclusive prefix through this tile published
 constexpr unsigned kVal = (1u << 30) - 1u;
 constexpr long long kMaxSpin = 1LL << 24;
+constexpr int kLook = 16;              // earlier tiles read per look-back step
 
 // digit of pass p: 8 bits, fewer in the last pass (keys sort by bits [0, bits))
 __device__ __host__ inline unsigned digit_mask(int bits, int p) {
@@ -81,11 +87,12 @@ __global__ void __launch_bounds__(256) k_digit_starts(const int* __restrict__ hi
     dstart[p * 256 + d] = scan256(hist[p * 256 + d], sh);
 }
 
-template <typename K>
+template <typename K, int kRI>
 __global__ void __launch_bounds__(kRT) k_onesweep(const K* __restrict__ kin, const int* __restrict__ vin, int id_base,
                                                   K* __restrict__ kout, int* __restrict__ vout, long long n, int shift,
                                                   unsigned dmask, unsigned* __restrict__ status, const int* __restrict__ dstart,
                                                   int* __restrict__ tile_ctr, int* __restrict__ err) {
+    constexpr int kRTile = kRT * kRI;
     __shared__ int cnt[kRW][256];  // per wavefront and digit: keys so far, then the wavefront's offset
     __shared__ int toff[256];      // first tile position of each digit
     __shared__ long long gofs[256];
@@ -145,21 +152,35 @@ __global__ void __launch_bounds__(kRT) k_onesweep(const K* __restrict__ kin, con
             __hip_atomic_store(mine, kPre | (unsigned)run, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         } else {
             __hip_atomic_store(mine, kAgg | (unsigned)run, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            // kLook earlier tiles' words are read together: one round trip
+            // covers kLook tiles, not one (a word read unpublished is waited for)
             long long spins = 0;
-            for (int p = tile - 1; p >= 0;) {
-                const unsigned st =
-                    __hip_atomic_load(status + (size_t)p * 256 + d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                if ((st >> 30) == 0u) {
+            bool found = false;
+            for (int p = tile - 1; p >= 0 && !found;) {
+                unsigned st[kLook];
+#pragma unroll
+                for (int q = 0; q < kLook; ++q)
+                    st[q] = __hip_atomic_load(status + (size_t)max(p - q, 0) * 256 + d, __ATOMIC_RELAXED,
+                                              __HIP_MEMORY_SCOPE_AGENT);
+                int taken = 0;
+#pragma unroll
+                for (int q = 0; q < kLook; ++q) {
+                    // consume in order up to the first unpublished word or the first prefix
+                    const bool use = !found && taken == q && p - q >= 0 && (st[q] >> 30) != 0u;
+                    if (use) {
+                        excl += (long long)(st[q] & kVal);
+                        found = (st[q] & kPre) != 0u;
+                        ++taken;
+                    }
+                }
+                p -= taken;
+                if (taken == 0) {
                     if (++spins > kMaxSpin) {
                         atomicOr(err, 1);
                         break;
                     }
                     __builtin_amdgcn_s_sleep(1);
-                    continue;
                 }
-                excl += (long long)(st & kVal);
-                if (st & kPre) break;
-                --p;
             }
             __hip_atomic_store(mine, kPre | (unsigned)((excl + run) & kVal), __ATOMIC_RELAXED,
                                __HIP_MEMORY_SCOPE_AGENT);
@@ -202,7 +223,9 @@ void sort_t(Ctx& c, const K* kin, K* kout, const int* vin, int id_base, int* vou
     if (bits < 1 || bits > 8 * (int)sizeof(K)) throw arg_error("radix_sort: bad key bit count");
     if ((const void*)kin == (const void*)kout) throw arg_error("radix_sort: keys must not be sorted in place");
     const int P = (bits + 7) / 8;
-    const long long ntiles = (n + kRTile - 1) / kRTile;
+    int per = 16;
+    while (per > 4 && n < (long long)kTilesWanted * kRT * per) per /= 2;
+    const long long ntiles = div_up(n, kRT * per);
     // scratch: keys and values of the other ping-pong buffer, then the ints
     const size_t kb = ((size_t)n * sizeof(K) + 255) / 256 * 256;
     const size_t vb = ((size_t)n * sizeof(int) + 255) / 256 * 256;
@@ -228,9 +251,14 @@ void sort_t(Ctx& c, const K* kin, K* kout, const int* vin, int id_base, int* vou
         const bool to_out = ((P - 1 - p) % 2) == 0;
         K* kd = to_out ? kout : ktmp;
         int* vd = to_out ? vout : vtmp;
-        hipLaunchKernelGGL((k_onesweep<K>), dim3((unsigned)ntiles), dim3(kRT), 0, s, ks, vs, id_base, kd, vd, n, 8 * p,
-                           digit_mask(bits, p), status + (size_t)p * ntiles * 256, (const int*)(dst + p * 256),
-                           ctr + p, err);
+        auto launch = [&](auto kern) {
+            hipLaunchKernelGGL(kern, dim3((unsigned)ntiles), dim3(kRT), 0, s, ks, vs, id_base, kd, vd, n, 8 * p,
+                               digit_mask(bits, p), status + (size_t)p * ntiles * 256, (const int*)(dst + p * 256),
+                               ctr + p, err);
+        };
+        if (per == 16) launch(k_onesweep<K, 16>);
+        else if (per == 8) launch(k_onesweep<K, 8>);
+        else launch(k_onesweep<K, 4>);
         SGIPC_LAUNCH_CHECK();
         ks = kd;
         vs = vd;

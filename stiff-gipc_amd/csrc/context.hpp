@@ -25,11 +25,12 @@ struct SymBcoo {
     DBuf<int2> ent;     // lower references + K (<= 2K)
     DBuf<float> valf;   // 12 * K FP32 copy of the BCOO values, padded columns (mixed precision)
     bool valf_ok = false;
-    // row-contiguous FP32 copy of both triangles in entry order (mixed
-    // precision): entry e of ent as its block, transposed where it is a
-    // transposed reference, 10 words (9 column-major floats + its column)
-    DBuf<float> valfull;
-    bool full_ok = false;
+    // copies of both triangles in entry order, for the PCG SpMV: entry e of
+    // ent as its block, transposed where it is a transposed reference, and its
+    // column, in groups of 64 entries (FullCopy in spmv_sym.hpp)
+    DBuf<float> full32;
+    DBuf<double> full64;
+    bool full32_ok = false, full64_ok = false;
 };
 
 // Sort of the static (FEM + mass) triplet segment, built where it started at
@@ -216,9 +217,8 @@ struct Ctx {
     DBuf<int> dev_int;    // small device ints (totals)
     SymBcoo bsr;
     bool have_bsr = false;
-    int spmv_group = 8;  // lanes per block row in the PCG SpMV (env SGIPC_SPMV_G: 4, 8, 16)
-    int spmv_blocks = 0; // cap on the mixed PCG SpMV's workgroups: 2 per CU (env SGIPC_SPMV_BLOCKS; 0: one per chunk, at most 1024)
-    int spmv_full32 = 1; // mixed precision: row-contiguous FP32 copy of both triangles (env SGIPC_SPMV_FULL32=0: upper BCOO)
+    int spmv_group = 8;  // lanes per block row in the batched solvers' SpMV and the upper-BCOO one (env SGIPC_SPMV_G: 4, 8, 16)
+    int spmv_full32 = 1; // mixed precision: FP32 copy of both triangles (env SGIPC_SPMV_FULL32=0: upper BCOO)
     int deterministic = 0;  // 1: MAS projection and barrier gradient summed in a fixed order (bitwise repeatable)
     DBuf<double> grad_scr;               // ordered barrier gradient: per-pair rows (12 doubles per pair)
     DBuf<unsigned> grad_key, grad_rec;   // (vertex, record) pairs, double-buffered for the sort
@@ -297,7 +297,8 @@ double ground_step_bound(Ctx& c, int m, const unsigned* ids, const double* x, co
 int bcoo_convert(Ctx& c, long long nt, int nblockrows);
 void bsr_build(Ctx& c);
 const float* bsr_values_f32(Ctx& c);
-const float* bsr_full_f32(Ctx& c);
+const float* bsr_full(Ctx& c, float);    // both triangles in entry order, FP32
+const double* bsr_full(Ctx& c, double);  // the same in FP64
 void spmv64(Ctx& c, double a, const double* x, double b, double* y);
 
 double kinetic_energy(Ctx& c, int n, const double* x, const double* xt, const double* m);

@@ -225,83 +225,153 @@ __global__ void __launch_bounds__(kThreads) k_simple_precond_dot(long long N, co
     write_partial(v, part_rz, sh);
 }
 
-// The same with the row-contiguous FP32 copy of both triangles: the G lanes
-// of a row read consecutive entries (40 bytes each: two 16-byte loads at
-// 8-byte alignment and one 8-byte load that also brings the column), no
-// block index, no transposition in registers, no column stream (44 -> 40
-// bytes per entry: counted traffic 96.7 -> 80.4 MB per launch at 137 k
-// block rows, the launch time within box-to-box noise of 2-3 %); the
-// column's three z values come in one 12-byte load; same
-// entry order and the same products, so the same sums.  (Measured and kept
-// out: 9-float entries read at 4-byte alignment, 30 % slower; the row's own
-// z, p, Ap loaded ahead of the row sums, 35 % slower.)
-template <int G, typename V>
-__global__ void __launch_bounds__(kThreads) k_spmv_pap_full(int nb, const int* __restrict__ eptr,
-                                                            const float* __restrict__ vf, const V* __restrict__ z,
-                                                            V* __restrict__ p, V* __restrict__ Ap,
-                                                            const double* __restrict__ rz_last,
-                                                            const double* __restrict__ rz_prev, int np_rz,
-                                                            double* __restrict__ part, int* __restrict__ ctrl) {
+// The same over the copy of both triangles (FullCopy): a workgroup takes a
+// chunk of R consecutive block rows and reads their entries as one contiguous
+// run, one entry per thread and load, whatever the rows' lengths; the products
+// A_e z_e (three per entry) go to LDS, and every row component is then summed
+// from there by g lanes (g a power of two that fills the workgroup: 1 for the
+// largest chunks, whose lanes keep four running sums).
+// Rows of this matrix have 7 or 19 entries (and more at contacts), so lanes
+// per row leave half the lanes idle or take a third round; here every lane
+// has an entry, the loads are contiguous, and the row pointers, the previous
+// dots and the row's own z, p and Ap are in flight before them.
+// Measured per launch against 8 lanes per row: at 137 k block rows FP32
+// (70 MB) 20.3 -> 17.7 us, FP64 (134 MB; the upper BCOO has 68 MB, but a
+// scattered 72-byte gather per transposed block) 37.3 -> 28.6 us, where a plain
+// read of as many bytes takes about 12 and 21 us; at 525 block rows 8.9 ->
+// 4.9 us.  Several entries in flight per thread were slower (more registers,
+// fewer wavefronts): 21.3 and 22.6 us for two and four against 19.8 us.
+constexpr int kFT = 256;          // threads
+constexpr int kFRows = 72;        // block rows per chunk, at most (three components each, of 256 threads)
+constexpr int kFBatch = 1024;     // entries per LDS batch
+constexpr int kFChunks = 4096;    // workgroups (p.Ap partials), at most
+
+template <typename V>
+__global__ void __launch_bounds__(kFT) k_spmv_pap_full(int nb, int R, int nchunks, int g, const int* __restrict__ eptr,
+                                                       const V* __restrict__ vf, const V* __restrict__ z,
+                                                       V* __restrict__ p, V* __restrict__ Ap,
+                                                       const double* __restrict__ rz_last,
+                                                       const double* __restrict__ rz_prev, int np_rz,
+                                                       double* __restrict__ part, int* __restrict__ ctrl) {
+    __shared__ V prod[3 * kFBatch];
+    __shared__ int er[kFRows + 1];
+    __shared__ double sh[3 * kFT / 64];
+    const int t = threadIdx.x, wv = t >> 6;
+    const ChunkWalk w = xcd_chunks(nchunks);
+    const int task = t / g, sub = t & (g - 1);  // this thread's row component of the chunk
+    const int row = task / 3;
+    // loads that depend on nothing: the first chunk's row pointers, the dots
+    double rn = 0.0, ro = 0.0;
+    int ev = 0;
+    if (w.first < w.end && t <= R) ev = eptr[min(w.first * R + t, nb)];
+    for (int i = t; i < np_rz; i += kFT) {
+        rn += rz_last[i];
+        ro += rz_prev[i];
+    }
     if (ctrl[C_STOP]) return;
     const int iter = ctrl[C_ITER];
     if (iter >= ctrl[C_MAXIT]) {
-        if (blockIdx.x == 0 && threadIdx.x == 0) { ctrl[C_NOCONV] = 1; ctrl[C_STOP] = ctrl[C_MAXIT]; }
+        if (blockIdx.x == 0 && t == 0) { ctrl[C_NOCONV] = 1; ctrl[C_STOP] = ctrl[C_MAXIT]; }
         return;
     }
-    __shared__ double sh[2 * (kThreads / 64)];
     const bool first = iter == 1;
-    // beta = rz_last / rz_prev is formed after the first chunk's row sums,
-    // so its partial-sum reduction overlaps the matrix loads (the chunk loop
-    // is uniform over the workgroup, so every thread reaches the barrier).
-    // The FP64 kernel keeps it first: holding its row state across the
-    // reduction cost it occupancy.
-    double be = 0.0;
-    bool have_be = first;
-    constexpr int RPB = kThreads / G;
-    const int nchunks = (nb + RPB - 1) / RPB;
-    ChunkWalk w = xcd_chunks(nchunks);
-    double contrib = 0.0;
+    // the waves' sums meet at the first chunk's barrier
+    rn = wave_sum(rn);
+    ro = wave_sum(ro);
+    if ((t & 63) == 0) {
+        sh[wv] = rn;
+        sh[kFT / 64 + wv] = ro;
+    }
+    double be = 0.0, contrib = 0.0;
     for (int ch = w.first; ch < w.end; ch += w.step) {
-        int row = ch * RPB + threadIdx.x / G, sub = threadIdx.x % G;
-        float s0 = 0, s1 = 0, s2 = 0;
-        if (row < nb) {
-            const int end = eptr[row + 1];
-            int e = eptr[row] + sub;
-            for (; e + G < end; e += 2 * G) {  // two entries in flight
-                const FullEntry fa = load_full_entry(vf, e), fb = load_full_entry(vf, e + G);
-                const f3_a4 xa = load_z3(z, fa.col), xb = load_z3(z, fb.col);
-                full_madd(fa, xa, s0, s1, s2);
-                full_madd(fb, xb, s0, s1, s2);
-            }
-            if (e < end) {
-                const FullEntry f = load_full_entry(vf, e);
-                full_madd(f, load_z3(z, f.col), s0, s1, s2);
+        const int r0 = ch * R, nr = min(R, nb - r0);
+        if (ch != w.first) {
+            if (t <= R) ev = eptr[min(r0 + t, nb)];
+            __syncthreads();  // every read of the previous chunk's er is done
+        }
+        if (t <= R) er[t] = ev;
+        const bool mine = row < nr;
+        const size_t o = 3 * (size_t)r0 + task;
+        V zo = 0, po = 0, ao = 0;
+        if (mine && sub == 0) {
+            zo = z[o];
+            if (!first) {
+                po = p[o];
+                ao = Ap[o];
             }
         }
-        group_sum3<G, float>(s0, s1, s2);
-        if (!have_be) {
-            double rn, ro;
-            sum_partials2(rz_last, np_rz, rz_prev, np_rz, sh, rn, ro);
+        __syncthreads();
+        if (!first && ch == w.first) {
+            rn = ro = 0.0;
+#pragma unroll
+            for (int i = 0; i < kFT / 64; ++i) {
+                rn += sh[i];
+                ro += sh[kFT / 64 + i];
+            }
             be = rn / ro;
-            have_be = true;
         }
-        if (sub < 3 && row < nb) {
-            const size_t o = 3 * (size_t)row + sub;
-            const V aw = (V)(sub == 0 ? s0 : (sub == 1 ? s1 : s2));
+        const int e0 = er[0], e1 = er[nr];
+        const int lo = mine ? er[row] : 0, hi = mine ? er[row + 1] : 0;
+        V s0 = 0, s1 = 0, s2 = 0, s3 = 0;
+        // batches start at a whole group of 64 entries
+        for (int b0 = e0 & ~63; b0 < e1; b0 += kFBatch) {
+            // (an index outside the chunk's run is clamped to it; a wavefront
+            // past the run does nothing)
+#pragma unroll
+            for (int j = 0; j < kFBatch / kFT; ++j) {
+                if (b0 + j * kFT + 64 * wv >= e1) continue;
+                V a[9], x[3];
+                int c;
+                FullCopy<V>::load(vf, max(e0, min(b0 + j * kFT + t, e1 - 1)), a, c);
+                load_x3(z, c, x);
+                V* pr = prod + 3 * (j * kFT + t);
+                pr[0] = a[0] * x[0] + a[3] * x[1] + a[6] * x[2];
+                pr[1] = a[1] * x[0] + a[4] * x[1] + a[7] * x[2];
+                pr[2] = a[2] * x[0] + a[5] * x[1] + a[8] * x[2];
+            }
+            __syncthreads();
+            if (mine) {
+                const int last = min(hi, b0 + kFBatch), st = 3 * g;
+                int e = lo + sub;
+                if (e < b0) e += (b0 - e + g - 1) / g * g;
+                const V* q = prod + 3 * (e - b0) + (task - 3 * row);
+                for (; e + 3 * g < last; e += 4 * g, q += 4 * st) {  // four running sums
+                    s0 += q[0];
+                    s1 += q[st];
+                    s2 += q[2 * st];
+                    s3 += q[3 * st];
+                }
+                if (e < last) s0 += q[0];
+                if (e + g < last) s1 += q[st];
+                if (e + 2 * g < last) s2 += q[2 * st];
+            }
+            __syncthreads();
+        }
+        V aw = (s0 + s1) + (s2 + s3);
+        for (int off = g >> 1; off > 0; off >>= 1) aw += __shfl_xor(aw, off, 64);
+        if (mine && sub == 0) {
             V pq, aq;
             if (first) {
-                pq = z[o];
+                pq = zo;
                 aq = aw;
             } else {
-                pq = (V)((double)z[o] + be * (double)p[o]);
-                aq = (V)((double)aw + be * (double)Ap[o]);
+                pq = (V)((double)zo + be * (double)po);
+                aq = (V)((double)aw + be * (double)ao);
             }
             p[o] = pq;
             Ap[o] = aq;
             contrib += (double)pq * (double)aq;
         }
     }
-    write_partial(contrib, part, sh);
+    contrib = wave_sum(contrib);
+    if ((t & 63) == 0) sh[2 * kFT / 64 + wv] = contrib;
+    __syncthreads();
+    if (t == 0) {
+        double v = 0.0;
+#pragma unroll
+        for (int i = 0; i < kFT / 64; ++i) v += sh[2 * kFT / 64 + i];
+        part[blockIdx.x] = v;
+    }
 }
 
 template <typename TD, typename TS>
@@ -397,8 +467,23 @@ struct Engine {
 
     int G = 8;  // lanes per block row in the SpMV (4, 8 or 16)
     double rz0_h = 0.0;  // rz0 of the last run, read with its final words
-    // mixed precision: the row-contiguous FP32 copy (null: the upper BCOO)
-    const float* vfull = nullptr;
+    // copy of both triangles in entry order (null: the upper BCOO) and its
+    // SpMV's chunks of rF block rows, nF of them, g lanes per row component
+    const V* vfull = nullptr;
+    int rF = 1, nF = 1, gF = 1;
+    // Rows per chunk: at least 8, so that small systems spread over many
+    // workgroups (one entry per thread), and more once there are 1920 chunks,
+    // seven or eight resident workgroups per CU, up to 72 (at 137 k rows, 42,
+    // 54, 64, 72 and 85 rows: 20.8, 20.0, 21.1, 18.8 and 19.8 us in FP32, the
+    // same order in FP64).
+    void use_full(const V* vf) {
+        vfull = vf;
+        rF = std::max(8, std::min(kFRows, (int)div_up(c.nb, 1920)));
+        nF = (int)div_up(c.nb, rF);
+        gF = 1;
+        while (gF < 64 && 2 * gF * 3 * rF <= kFT) gF *= 2;
+        gS = std::min(kFChunks, std::max(8, (int)div_up(nF, 8) * 8));
+    }
     // pinned progress words published by the MAS collect kernel (set while
     // the last iteration of a captured group is enqueued)
     volatile int* pub_h = nullptr;
@@ -434,16 +519,13 @@ struct Engine {
                                (const double*)rz_last, (const double*)rz_this, nRZ, part_pap, ctrl);
         };
         if (vfull) {
-            auto launchf = [&](auto kern) {
-                hipLaunchKernelGGL(kern, dim3(gS), dim3(kThreads), 0, s, S.nb, S.eptr.p, vfull, (const V*)z, p,
-                                   Ap, (const double*)rz_last, (const double*)rz_this, nRZ, part_pap, ctrl);
-            };
-            if (G == 4) launchf(k_spmv_pap_full<4, V>);
-            else if (G == 16) launchf(k_spmv_pap_full<16, V>);
-            else launchf(k_spmv_pap_full<8, V>);
-        } else if (G == 4) launch(k_spmv_pap<4, MV, V>);
-        else if (G == 16) launch(k_spmv_pap<16, MV, V>);
-        else launch(k_spmv_pap<8, MV, V>);
+            hipLaunchKernelGGL((k_spmv_pap_full<V>), dim3(gS), dim3(kFT), 0, s, S.nb, rF, nF, gF, S.eptr.p, vfull,
+                               (const V*)z, p, Ap, (const double*)rz_last, (const double*)rz_this, nRZ, part_pap, ctrl);
+        } else if constexpr (sizeof(V) == 4) {
+            if (G == 4) launch(k_spmv_pap<4, MV, V>);
+            else if (G == 16) launch(k_spmv_pap<16, MV, V>);
+            else launch(k_spmv_pap<8, MV, V>);
+        }
         SGIPC_LAUNCH_CHECK();
         prof_end(c, PROF_SPMV);
         if (mas) {
@@ -494,7 +576,7 @@ struct Engine {
         size_t h = 1469598103934665603ull;
         auto mix = [&](size_t v) { h ^= v + 0x9e3779b97f4a7c15ull + (h << 6) + (h >> 2); };
         const SymBcoo& S = c.bsr;
-        mix((size_t)N); mix((size_t)gN); mix((size_t)gS); mix((size_t)G); mix((size_t)gU); mix((size_t)S.nb); mix((size_t)S.K);
+        mix((size_t)N); mix((size_t)gN); mix((size_t)gS); mix((size_t)G); mix((size_t)rF); mix((size_t)nF); mix((size_t)gF); mix((size_t)gU); mix((size_t)S.nb); mix((size_t)S.K);
         mix((size_t)S.eptr.p); mix((size_t)S.ent.p); mix((size_t)val); mix((size_t)r); mix((size_t)z); mix((size_t)p);
         mix((size_t)Ap); mix((size_t)x); mix((size_t)part_rz[0]); mix((size_t)sc);
         mix((size_t)ctrl); mix((size_t)mas); mix((size_t)R); mix((size_t)Z); mix((size_t)Dinv); mix((size_t)rule);
@@ -772,18 +854,15 @@ void pcg_solve(Ctx& c, const double* b, double* x, const SolveOpts& o, SolveStat
     const bool mas = (c.precond_kind == 2 || c.precond_kind == 3);
     if (mas && !c.mas.ready) throw state_error("solve: MAS preconditioner not built");
     if (c.precond_kind == 1 && !w.Dinv.p) throw state_error("solve: block-Jacobi preconditioner not built");
-    double* parts = w.partials.reserve(6 * kPart);
+    double* parts = w.partials.reserve(5 * kPart + kFChunks);
     double* sc = w.scal.reserve(S_NUM + 8);
     int* ctrl = w.ctrl.reserve(C_NUM + 8);
     const int max_iter = o.max_iter > 0 ? o.max_iter : (int)(o.max_iter_ratio * (double)N);
     const int gN = grid_for(N);
-    // SpMV: chunks of kThreads / G block rows, a multiple of 8 workgroups (one range per XCD)
+    // SpMV on the upper BCOO: chunks of kThreads / G block rows, a multiple of 8 workgroups (one range per XCD)
     const int G = c.spmv_group;
     const int nchunks = (int)div_up((long long)c.nb, kThreads / G);
-    int gS = std::min(kPart, std::max(8, (int)div_up(nchunks, 8) * 8));
-    // the FP32 full-copy SpMV of mixed solves runs best as one resident round
-    // of workgroups walking the chunks (the FP64 kernel as one per chunk)
-    if (o.precision != 0 && c.spmv_blocks > 0) gS = std::min(gS, std::max(8, c.spmv_blocks / 8 * 8));
+    const int gS = std::min(kPart, std::max(8, (int)div_up(nchunks, 8) * 8));
     st.refinements = 0;
     if (o.precision == 0) {
         auto run64 = [&](auto tag) {
@@ -792,12 +871,12 @@ void pcg_solve(Ctx& c, const double* b, double* x, const SolveOpts& o, SolveStat
             Engine<double, double, T> E{c, N, gN, gS,
                                         w.r.reserve(N + 1), w.z.reserve(N + 1), w.p.reserve(N + 1),
                                         w.Ap.reserve(N + 1),
-                                        x, {parts, parts + kPart}, parts + 2 * kPart, parts + 3 * kPart,
-                                        parts + 4 * kPart, sc, ctrl, (const double*)c.t_vals, mas,
+                                        x, {parts, parts + kPart}, parts + 5 * kPart, parts + 2 * kPart,
+                                        parts + 3 * kPart, sc, ctrl, (const double*)c.t_vals, mas,
                                         mas ? (T*)(fp32mas ? (void*)c.mas.R32.p : (void*)c.mas.R64.p) : nullptr,
                                         mas ? (T*)(fp32mas ? (void*)c.mas.Z32.p : (void*)c.mas.Z64.p) : nullptr,
                                         c.precond_kind == 1 ? w.Dinv.p : nullptr, o.stop_rule};
-            E.G = G;
+            E.use_full(bsr_full(c, double{}));
             hipLaunchKernelGGL((k_copy_cast<double, double>), dim3(gN), dim3(kThreads), 0, s, N, E.r, b);
             SGIPC_LAUNCH_CHECK();
             E.init(o.tol, max_iter);
@@ -826,18 +905,18 @@ void pcg_solve(Ctx& c, const double* b, double* x, const SolveOpts& o, SolveStat
         Engine<float, float, float> E{c, N, gN, gS,
                                       rf, w.zf.reserve(N + 1), w.pf.reserve(N + 1),
                                       w.Apf.reserve(N + 1),
-                                      d64, {parts, parts + kPart}, parts + 2 * kPart, parts + 3 * kPart,
-                                      parts + 4 * kPart, sc, ctrl,
+                                      d64, {parts, parts + kPart}, parts + 5 * kPart, parts + 2 * kPart,
+                                      parts + 3 * kPart, sc, ctrl,
                                       c.spmv_full32 ? nullptr : bsr_values_f32(c),  // the full copy replaces it
                                       mas,
                                       mas ? c.mas.R32.p : nullptr, mas ? c.mas.Z32.p : nullptr,
                                       c.precond_kind == 1 ? w.Dinv.p : nullptr, 1};
         E.G = G;
-        if (c.spmv_full32) E.vfull = bsr_full_f32(c);
+        if (c.spmv_full32) E.use_full(bsr_full(c, float{}));
         fill<double>(x, 0.0, N, s);
         hipLaunchKernelGGL((k_copy_cast<double, double>), dim3(gN), dim3(kThreads), 0, s, N, r64, b);
         SGIPC_LAUNCH_CHECK();
-        double* part_o = parts + 5 * kPart;
+        double* part_o = parts + 4 * kPart;
         // ||b||^2 stays on the device until the first true residual is read
         // with it (the first inner tolerance needs only ||r|| = ||b||)
         constexpr int S_B2 = S_NUM + 1;
@@ -888,7 +967,7 @@ void pcg_solve(Ctx& c, const double* b, double* x, const SolveOpts& o, SolveStat
     SGIPC_LAUNCH_CHECK();
     spmv64(c, -1.0, x, 1.0, tmp);
     // ||b||^2 is the init's S_BB (r held b); one read for both
-    device_norm2_to(c, tmp, N, parts + 5 * kPart, sc, S_NUM);
+    device_norm2_to(c, tmp, N, parts + 4 * kPart, sc, S_NUM);
     double rr = 0.0, bb = 0.0;
     read_scalars(c, sc, S_NUM, S_BB, rr, bb);
     st.rel_residual = bb > 0.0 ? std::sqrt(rr / bb) : std::sqrt(rr);

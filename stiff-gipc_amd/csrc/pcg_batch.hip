@@ -93,15 +93,25 @@ __global__ void __launch_bounds__(1024) k_bspmv_full(const int* __restrict__ chu
     if (row < r1) {
         const int end = eptr[row + 1];
         int e = eptr[row] + sub;
+        auto madd = [&](const float a[9], const float x[3]) {
+            s0 += a[0] * x[0] + a[3] * x[1] + a[6] * x[2];
+            s1 += a[1] * x[0] + a[4] * x[1] + a[7] * x[2];
+            s2 += a[2] * x[0] + a[5] * x[1] + a[8] * x[2];
+        };
+        float a[9], b[9], xa[3], xb[3];
+        int ca, cb;
         for (; e + G < end; e += 2 * G) {  // two entries in flight
-            const FullEntry fa = load_full_entry(vf, e), fb = load_full_entry(vf, e + G);
-            const f3_a4 xa = load_z3(p, fa.col), xb = load_z3(p, fb.col);
-            full_madd(fa, xa, s0, s1, s2);
-            full_madd(fb, xb, s0, s1, s2);
+            FullCopy<float>::load(vf, e, a, ca);
+            FullCopy<float>::load(vf, e + G, b, cb);
+            load_x3(p, ca, xa);
+            load_x3(p, cb, xb);
+            madd(a, xa);
+            madd(b, xb);
         }
         if (e < end) {
-            const FullEntry f = load_full_entry(vf, e);
-            full_madd(f, load_z3(p, f.col), s0, s1, s2);
+            FullCopy<float>::load(vf, e, a, ca);
+            load_x3(p, ca, xa);
+            madd(a, xa);
         }
     }
     group_sum3<G, float>(s0, s1, s2);
@@ -621,7 +631,7 @@ void pcg_solve_batched(Ctx& c, int S, const int* h_row_start, const double* b, d
         double* d64 = pw.d64.reserve(N + 1);
         // the SpMV reads the row-contiguous FP32 copy of both triangles, or
         // (SGIPC_SPMV_FULL32=0) the FP32 copy of the upper BCOO; only one is built
-        const float* vfull = c.spmv_full32 ? bsr_full_f32(c) : nullptr;
+        const float* vfull = c.spmv_full32 ? bsr_full(c, float{}) : nullptr;
         BEngine<float, float, float> E{c, w, N, S, w.nch, G, rf, pw.zf.reserve(N + 1), pw.pf.reserve(N + 1),
                                       pw.Apf.reserve(N + 1), d64, vfull ? nullptr : bsr_values_f32(c), true, 1};
         E.vfull = vfull;

@@ -89,37 +89,27 @@ __global__ void k_to_f32(long long K, const double* __restrict__ s, float* __res
     }
 }
 
-// entry-ordered FP32 copy: eight lanes per block row, lane j taking entries
-// j, j + 8, ... of the row, so a row's lanes write adjacent 40-byte entries
-// (nine floats and the column: five aligned 8-byte stores each); rows are
-// walked in per-XCD ranges, as in the SpMV, so the transposed blocks a row
-// gathers are shared in L2.
-constexpr int kFullG = 8;
-__global__ void __launch_bounds__(256) k_full_f32(int nb, const int* __restrict__ eptr, const int2* __restrict__ ent,
-                                                  const double* __restrict__ vals, float* __restrict__ vf) {
-    constexpr int RPB = 256 / kFullG;
-    const ChunkWalk w = xcd_chunks((nb + RPB - 1) / RPB);
+// copy of both triangles in entry order (FullCopy): one thread per entry, so
+// the stores are contiguous.  Entry (k, c) is block k transposed where c is
+// the block's row and not its column.  Workgroups take entries in per-XCD
+// ranges: the blocks that nearby rows share, once upright and once
+// transposed, meet in one L2.
+template <typename T>
+__global__ void __launch_bounds__(256) k_full_copy(int nb, const int* __restrict__ eptr, const int2* __restrict__ ent,
+                                                   const int* __restrict__ cols, const double* __restrict__ vals,
+                                                   T* __restrict__ vf) {
+    const int n = eptr[nb];
+    const ChunkWalk w = xcd_chunks((n + 255) / 256);
     for (int ch = w.first; ch < w.end; ch += w.step) {
-        const int r = ch * RPB + threadIdx.x / kFullG, sub = threadIdx.x % kFullG;
-        if (r >= nb) continue;
-        const int end = eptr[r + 1];
-        for (int e = eptr[r] + sub; e < end; e += kFullG) {
-            const int2 q = ent[e];
-            const double* A = vals + 9 * (size_t)q.x;
-            double a[9];
+        const int e = ch * 256 + (int)threadIdx.x;
+        if (e >= n) continue;
+        const int2 q = ent[e];
+        double a[9];
+        load_block<double>(vals, q.x, cols[q.x] != q.y, a);
+        T t[9];
 #pragma unroll
-            for (int k = 0; k < 9; ++k) a[k] = A[k];
-            float d[10];
-            const bool tr = q.y < r;
-#pragma unroll
-            for (int pp = 0; pp < 3; ++pp)
-#pragma unroll
-                for (int qq = 0; qq < 3; ++qq) d[pp + 3 * qq] = (float)(tr ? a[qq + 3 * pp] : a[pp + 3 * qq]);
-            d[9] = __int_as_float(q.y);
-            float2* o = reinterpret_cast<float2*>(vf + kF32FullStride * (size_t)e);
-#pragma unroll
-            for (int k = 0; k < 5; ++k) o[k] = make_float2(d[2 * k], d[2 * k + 1]);
-        }
+        for (int k = 0; k < 9; ++k) t[k] = (T)a[k];
+        FullCopy<T>::store(vf, e, t, q.y);
     }
 }
 
@@ -175,24 +165,31 @@ void bsr_build(Ctx& c) {
                        (const int2*)lref, (const int*)c.uniq_start.p, (const int*)c.t_cols, eptr, ent);
     SGIPC_LAUNCH_CHECK();
     S.valf_ok = false;
-    S.full_ok = false;
+    S.full32_ok = S.full64_ok = false;
     c.have_bsr = true;
 }
 
-// Row-contiguous FP32 copy of both triangles (mixed-precision SpMV)
-const float* bsr_full_f32(Ctx& c) {
-    if (!c.have_bsr) bsr_build(c);
+template <typename T>
+static const T* full_copy(Ctx& c, DBuf<T>& buf, bool& ok) {
     SymBcoo& S = c.bsr;
-    const size_t ne = 2 * (size_t)S.K;  // bound on the entries (lower references + upper blocks)
-    float* vf = S.valfull.reserve(kF32FullStride * ne + 4);
-    if (!S.full_ok && S.nb > 0) {
-        const int blocks = 8 * std::min(div_up(div_up(S.nb, 256 / kFullG), 8), 2048);
-        hipLaunchKernelGGL(k_full_f32, dim3(blocks), dim3(256), 0, c.stream, S.nb, (const int*)S.eptr.p,
-                           (const int2*)S.ent.p, (const double*)c.t_vals, vf);
+    // 2K bounds the entries (lower references + upper blocks); whole groups of 64
+    T* vf = buf.reserve(((2 * (size_t)S.K + 63) / 64 + 1) * FullCopy<T>::kGroup);
+    if (!ok && S.nb > 0 && S.K > 0) {
+        const int blocks = 8 * std::max(1, std::min((int)div_up(2LL * S.K, 8 * 256), 1024));
+        hipLaunchKernelGGL(k_full_copy<T>, dim3(blocks), dim3(256), 0, c.stream, S.nb, (const int*)S.eptr.p,
+                           (const int2*)S.ent.p, (const int*)c.t_cols, (const double*)c.t_vals, vf);
         SGIPC_LAUNCH_CHECK();
     }
-    S.full_ok = true;
+    ok = true;
     return vf;
+}
+const float* bsr_full(Ctx& c, float) {
+    if (!c.have_bsr) bsr_build(c);
+    return full_copy<float>(c, c.bsr.full32, c.bsr.full32_ok);
+}
+const double* bsr_full(Ctx& c, double) {
+    if (!c.have_bsr) bsr_build(c);
+    return full_copy<double>(c, c.bsr.full64, c.bsr.full64_ok);
 }
 
 // FP32 copy of the BCOO values for the mixed-precision solve

@@ -40,7 +40,6 @@ __device__ inline ChunkWalk xcd_chunks(int nchunks) {
 // (48 B per block, columns in float4 lanes 0-2), three aligned 16-byte loads.
 typedef double double2_a8 __attribute__((ext_vector_type(2), aligned(8)));
 constexpr int kF32BlockStride = 12;  // floats per block in the FP32 copy
-constexpr int kF32FullStride = 10;   // words per entry in the row-contiguous FP32 copy: 9 floats + the column (five aligned 8-byte pairs)
 
 template <typename TV>
 __device__ inline void load_block(const TV* __restrict__ vals, int k, bool tr, TV a[9]);
@@ -119,43 +118,69 @@ __device__ inline void sym_row_lane(int row, int sub, const int* __restrict__ ep
     }
 }
 
-// Row-contiguous FP32 copy of both triangles (mixed precision): entry e is
-// its block (transposed where it is a transposed reference), 10 floats, read
-// as two 16-byte loads at 8-byte alignment and one 8-byte load.
-typedef float f4_a8 __attribute__((ext_vector_type(4), aligned(8)));
+// Copy of both triangles in entry order: entry e of ent as its 3x3 block,
+// transposed where it is a transposed reference, with its column.  Entries lie
+// in groups of 64, the pieces of a group one after the other (64 pieces of 16
+// bytes each, ..., the last element and the column), so that 64 lanes reading
+// 64 consecutive entries read contiguous memory with every load: 40 bytes an
+// entry in FP32, 76 in FP64.
 typedef float f3_a4 __attribute__((ext_vector_type(3), aligned(4)));
+typedef double d2_a8 __attribute__((ext_vector_type(2), aligned(8)));
 
-struct FullEntry {
-    f4_a8 lo, hi;  // column-major elements 0-3, 4-7
-    float a8;
-    int col;       // block column (the entry's tenth word)
-};
-__device__ inline FullEntry load_full_entry(const float* __restrict__ vf, int e) {
-    const float* A = vf + kF32FullStride * (size_t)e;
-    FullEntry f;
-    f.lo = *reinterpret_cast<const f4_a8*>(A);
-    f.hi = *reinterpret_cast<const f4_a8*>(A + 4);
-    const int2 t = *reinterpret_cast<const int2*>(A + 8);
-    f.a8 = __int_as_float(t.x);
-    f.col = t.y;
-    return f;
-}
-template <typename V>
-__device__ inline f3_a4 load_z3(const V* __restrict__ z, int c) {
-    if constexpr (sizeof(V) == 4) {
-        return *reinterpret_cast<const f3_a4*>(z + 3 * (size_t)c);
-    } else {
-        f3_a4 r;
-        r.x = (float)z[3 * (size_t)c];
-        r.y = (float)z[3 * (size_t)c + 1];
-        r.z = (float)z[3 * (size_t)c + 2];
-        return r;
+template <typename T>
+struct FullCopy;
+template <>
+struct FullCopy<float> {
+    static constexpr int kGroup = 640;  // floats per group of 64 entries
+    __device__ static inline void load(const float* __restrict__ vf, int e, float a[9], int& col) {
+        const float* g = vf + (size_t)(e >> 6) * kGroup;
+        const int l = e & 63;
+        const float4 u = reinterpret_cast<const float4*>(g)[l], v = reinterpret_cast<const float4*>(g + 256)[l];
+        const int2 w = reinterpret_cast<const int2*>(g + 512)[l];
+        a[0] = u.x; a[1] = u.y; a[2] = u.z; a[3] = u.w; a[4] = v.x; a[5] = v.y; a[6] = v.z; a[7] = v.w;
+        a[8] = __int_as_float(w.x);
+        col = w.y;
     }
+    __device__ static inline void store(float* __restrict__ vf, int e, const float a[9], int col) {
+        float* g = vf + (size_t)(e >> 6) * kGroup;
+        const int l = e & 63;
+        reinterpret_cast<float4*>(g)[l] = make_float4(a[0], a[1], a[2], a[3]);
+        reinterpret_cast<float4*>(g + 256)[l] = make_float4(a[4], a[5], a[6], a[7]);
+        reinterpret_cast<int2*>(g + 512)[l] = make_int2(__float_as_int(a[8]), col);
+    }
+};
+template <>
+struct FullCopy<double> {
+    static constexpr int kGroup = 608;  // doubles per group of 64 entries
+    __device__ static inline void load(const double* __restrict__ vf, int e, double a[9], int& col) {
+        const double* g = vf + (size_t)(e >> 6) * kGroup;
+        const int l = e & 63;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const double2 u = reinterpret_cast<const double2*>(g + 128 * k)[l];
+            a[2 * k] = u.x;
+            a[2 * k + 1] = u.y;
+        }
+        a[8] = g[512 + l];
+        col = reinterpret_cast<const int*>(g + 576)[l];
+    }
+    __device__ static inline void store(double* __restrict__ vf, int e, const double a[9], int col) {
+        double* g = vf + (size_t)(e >> 6) * kGroup;
+        const int l = e & 63;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) reinterpret_cast<double2*>(g + 128 * k)[l] = make_double2(a[2 * k], a[2 * k + 1]);
+        g[512 + l] = a[8];
+        reinterpret_cast<int*>(g + 576)[l] = col;
+    }
+};
+// the three components of block row c of a vector
+__device__ inline void load_x3(const float* __restrict__ z, int c, float x[3]) {
+    const f3_a4 v = *reinterpret_cast<const f3_a4*>(z + 3 * (size_t)c);
+    x[0] = v.x; x[1] = v.y; x[2] = v.z;
 }
-__device__ inline void full_madd(const FullEntry& f, const f3_a4& x, float& s0, float& s1, float& s2) {
-    s0 += f.lo.x * x.x + f.lo.w * x.y + f.hi.z * x.z;
-    s1 += f.lo.y * x.x + f.hi.x * x.y + f.hi.w * x.z;
-    s2 += f.lo.z * x.x + f.hi.y * x.y + f.a8 * x.z;
+__device__ inline void load_x3(const double* __restrict__ z, int c, double x[3]) {
+    const d2_a8 v = *reinterpret_cast<const d2_a8*>(z + 3 * (size_t)c);
+    x[0] = v.x; x[1] = v.y; x[2] = z[3 * (size_t)c + 2];
 }
 
 template <int G, typename TV>

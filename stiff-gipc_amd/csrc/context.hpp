@@ -47,6 +47,13 @@ struct ConvertPlan {
     DBuf<int> ucol, urun;       // per unique block: column, run start in sorted
 };
 
+// MAS level-0 slot: its vertex (-1: empty), the vertex's level-1 node
+// (level-local id) and the bank lanes of its level-0 component
+struct alignas(16) SlotNode {
+    int v, node;
+    unsigned mask, pad;
+};
+
 struct MasState {
     bool ready = false;
     int bank = 16;
@@ -60,6 +67,7 @@ struct MasState {
     DBuf<int> part_map, real_map;
     DBuf<unsigned> nstart, nnum, nlist;
     DBuf<unsigned> fine_mask, next_mask;
+    DBuf<SlotNode> slot_node;  // M
     DBuf<int> prefix0, psum0, next_prefix, next_psum;
     DBuf<int> level_size;  // 2*(L+2)
     DBuf<int> coarse_space;  // L*n

@@ -168,7 +168,7 @@ __global__ void __launch_bounds__(kTB) k_l0_closure(int M, int B, const int* __r
 __global__ void __launch_bounds__(kTB) k_level1(int M, int Mpad, int n, int B, const int* __restrict__ part_map,
                                                  const unsigned* __restrict__ fine_mask,
                                                  const int* __restrict__ psum0, int* __restrict__ coarse_space,
-                                                 int* __restrict__ going_next) {
+                                                 int* __restrict__ going_next, SlotNode* __restrict__ slot_node) {
     __shared__ unsigned sel[kTB];
     int s = blockIdx.x * blockDim.x + threadIdx.x;
     int lane = threadIdx.x % B, bbase = threadIdx.x - lane;
@@ -176,13 +176,17 @@ __global__ void __launch_bounds__(kTB) k_level1(int M, int Mpad, int n, int B, c
     unsigned fm = (v >= 0) ? fine_mask[v] : 0u;
     sel[threadIdx.x] = (v >= 0 && (fm & ltmask(lane)) == 0u) ? (1u << lane) : 0u;
     __syncthreads();
-    if (v < 0) return;
+    if (v < 0) {
+        if (s < M) slot_node[s] = SlotNode{-1, -1, 0u, 0u};
+        return;
+    }
     unsigned elected = 0u;
     for (int l = 0; l < B; ++l) elected |= sel[bbase + l];
     int el = lowbit(fm);
     int pre = __popc(elected & ltmask(el)) + psum0[s / B];
     coarse_space[v] = pre;
     going_next[v] = pre + Mpad;
+    slot_node[s] = SlotNode{v, pre, fm, 0u};
 }
 
 __global__ void k_set_level_size(int* __restrict__ ls, int level, const int* __restrict__ total, int B,
@@ -864,45 +868,57 @@ __global__ void k_collect(int n, int L, const int* __restrict__ node_of, const T
 // Component sum of one bank-aligned group of nodes held in LDS (one node
 // per thread).  `mask` holds the bank lanes of this node's component (its
 // closure, self included); only the lowest lane of the component sums, in
-// ascending lane order.  Returns true for that lane, with the sums.
+// ascending lane order (16 lanes' values are read at once; a lane outside the
+// component adds nothing).  Returns true for that lane, with the sums.
 template <typename T>
 __device__ inline bool component_sum(unsigned mask, const T* a0, const T* a1, const T* a2, int B, T& s0, T& s1,
                                      T& s2) {
-    int t = threadIdx.x, lane = t % B, bbase = t - lane;
+    const int t = threadIdx.x, lane = t & (B - 1), bbase = t - lane;
     if (mask & ltmask(lane)) return false;
     s0 = 0; s1 = 0; s2 = 0;
-    for (unsigned m = mask; m; m &= m - 1u) {
-        int l = lowbit(m);
-        s0 += a0[bbase + l]; s1 += a1[bbase + l]; s2 += a2[bbase + l];
+    for (int h = 0; h < B; h += 16) {
+        T q[16][3];
+#pragma unroll
+        for (int l = 0; l < 16; ++l) {
+            q[l][0] = a0[bbase + h + l];
+            q[l][1] = a1[bbase + h + l];
+            q[l][2] = a2[bbase + h + l];
+        }
+#pragma unroll
+        for (int l = 0; l < 16; ++l)
+            if ((mask >> (h + l)) & 1u) { s0 += q[l][0]; s1 += q[l][1]; s2 += q[l][2]; }
     }
     return true;
 }
 
 // level-0 slots -> level-1 sums of the nodes of level-1 bank b, then
-// level 1 -> 2 inside that bank.  `value(v, sl, own, ...)` gives the
-// level-0 value of vertex v at slot sl.  A vertex is owned by exactly one
-// workgroup: the one whose level-1 bank holds the vertex's level-1 node.
-// Only the owner reads or writes the vertex's data (value() is called with
-// own = false for the others and their values are never summed: a
-// component's lanes all share one level-1 node), so a level-0 bank whose
-// coarse nodes straddle two level-1 banks is split between their
-// workgroups with no slot touched twice.  fine_mask / comp_mask: component
-// lanes of each level-0 vertex / coarse node.
-// The index loads of level-1 bank b that do not depend on the residual:
-// its level-0 slot range, the first slot chunk's vertices and the level
-// 1 -> 2 mapping of its nodes.  Issued before a kernel's partial-sum
-// reduction, their latency overlaps it.
+// level 1 -> 2 inside that bank.  `load(v)` reads what a vertex's level-0
+// value needs and `value(v, ...)` gives it (and does what else the owner of v
+// does).  A vertex is owned by exactly one workgroup: the one whose level-1
+// bank holds the vertex's level-1 node.  Only the owner reads or writes the
+// vertex's data, so a level-0 bank whose coarse nodes straddle two level-1
+// banks is split between their workgroups with no slot touched twice (a
+// component's lanes all share one level-1 node).  slot_node: vertex, level-1
+// node and component lanes of every level-0 slot; comp_mask: component lanes
+// of each coarse node.
+// The loads of level-1 bank b that do not depend on the residual: its level-0
+// slot range, the first slot chunk's entries and the level 1 -> 2 mapping of
+// its nodes.  Issued before a kernel's partial-sum reduction, their latency
+// overlaps it.
 struct BankIdx {
-    int lo, hi, v0, q;
+    int lo, hi, q;
+    SlotNode sn;
     unsigned mask2;
     bool valid;
 };
-__device__ inline BankIdx bank_index(int b, int B, int L, int cnt1, int beg1, const int* __restrict__ part_map,
+__device__ inline BankIdx bank_index(int b, int B, int L, int cnt1, int beg1, const SlotNode* __restrict__ slot_node,
                                      const int* __restrict__ going_next, const unsigned* __restrict__ comp_mask,
                                      const int* __restrict__ l1lo, const int* __restrict__ l1hi) {
     const int t = threadIdx.x;
     BankIdx x;
     const int loc2 = b * B + t;
+    x.lo = l1lo[b] * B;
+    x.hi = l1hi[b] * B;
     x.valid = L >= 3 && t < B && loc2 < cnt1;
     x.q = -1;
     x.mask2 = 0u;
@@ -910,61 +926,48 @@ __device__ inline BankIdx bank_index(int b, int B, int L, int cnt1, int beg1, co
         x.q = going_next[(size_t)beg1 + loc2];
         x.mask2 = comp_mask[(size_t)beg1 + loc2];
     }
-    x.lo = l1lo[b] * B;
-    x.hi = l1hi[b] * B;
     const int sl = x.lo + t;
-    x.v0 = (sl < x.hi) ? part_map[sl] : -1;
+    x.sn = (sl < x.hi) ? slot_node[sl] : SlotNode{-1, -1, 0u, 0u};
     return x;
 }
 
-template <typename T, typename F>
-__device__ inline void restrict_bank(int b, int B, int L, int cnt1, int beg1, const int* __restrict__ part_map,
-                                     const int* __restrict__ going_next, const unsigned* __restrict__ fine_mask,
-                                     const unsigned* __restrict__ comp_mask, const BankIdx& pre, T* __restrict__ R,
-                                     T (*sv)[kTB], T (*l1v)[32], F value) {
+// this workgroup's (bank b's) own slot among those read
+__device__ inline bool owned(const SlotNode& s, int b, int B) { return s.v >= 0 && (s.node & ~(B - 1)) == b * B; }
+
+template <typename T, typename FL, typename FV>
+__device__ inline void restrict_bank(int b, int B, int L, int beg1, const SlotNode* __restrict__ slot_node,
+                                     const BankIdx& pre, T* __restrict__ R, T (*sv)[kTB], T (*l1v)[32], bool loaded,
+                                     FL load, FV value) {
     const int t = threadIdx.x;
     const bool valid = pre.valid;
-    const int q = pre.q;
-    const unsigned mask2 = pre.mask2;
     const int lo = pre.lo, hi = pre.hi;
     for (int c0 = lo; c0 < hi; c0 += kTB) {
-        int sl = c0 + t;
-        int v = c0 == lo ? pre.v0 : ((sl < hi) ? part_map[sl] : -1);
-        int p = -1;
-        unsigned mask = 0u;
+        const int sl = c0 + t;
+        SlotNode sn = pre.sn;
+        if (c0 != lo) sn = (sl < hi) ? slot_node[sl] : SlotNode{-1, -1, 0u, 0u};
+        const bool own = owned(sn, b, B);
         T v0 = 0, v1 = 0, v2 = 0;
-        if (v >= 0) {
-            const int loc = going_next[v] - beg1;
-            const bool own = loc / B == b;
-            value(v, sl, own, v0, v1, v2);
-            if (own) {
-                R[3 * (size_t)sl] = v0; R[3 * (size_t)sl + 1] = v1; R[3 * (size_t)sl + 2] = v2;
-                p = loc;
-                mask = fine_mask[v];
-            }
+        if (own) {
+            if (c0 != lo || !loaded) load(sn.v);
+            value(sn.v, v0, v1, v2);
+            R[3 * (size_t)sl] = v0; R[3 * (size_t)sl + 1] = v1; R[3 * (size_t)sl + 2] = v2;
         }
         sv[0][t] = v0; sv[1][t] = v1; sv[2][t] = v2;
         __syncthreads();
         T s0, s1, s2;
-        if (p >= 0 && component_sum<T>(mask, sv[0], sv[1], sv[2], B, s0, s1, s2)) {
-            size_t g = (size_t)beg1 + p;
+        if (own && component_sum<T>(sn.mask, sv[0], sv[1], sv[2], B, s0, s1, s2)) {
+            size_t g = (size_t)beg1 + sn.node;
             R[3 * g] = s0; R[3 * g + 1] = s1; R[3 * g + 2] = s2;
-            l1v[0][p - b * B] = s0; l1v[1][p - b * B] = s1; l1v[2][p - b * B] = s2;
+            l1v[0][sn.node - b * B] = s0; l1v[1][sn.node - b * B] = s1; l1v[2][sn.node - b * B] = s2;
         }
         __syncthreads();
     }
     if (L < 3) return;
-    if (t < B) {
-        sv[0][t] = valid ? l1v[0][t] : (T)0;
-        sv[1][t] = valid ? l1v[1][t] : (T)0;
-        sv[2][t] = valid ? l1v[2][t] : (T)0;
-    }
-    __syncthreads();
+    // level 1 -> 2: nodes past the bank's last are in no component's mask
     T s0, s1, s2;
-    if (valid && component_sum<T>(mask2, sv[0], sv[1], sv[2], B, s0, s1, s2)) {
-        R[3 * (size_t)q] = s0; R[3 * (size_t)q + 1] = s1; R[3 * (size_t)q + 2] = s2;
+    if (valid && component_sum<T>(pre.mask2, l1v[0], l1v[1], l1v[2], B, s0, s1, s2)) {
+        R[3 * (size_t)pre.q] = s0; R[3 * (size_t)pre.q + 1] = s1; R[3 * (size_t)pre.q + 2] = s2;
     }
-    __syncthreads();
 }
 
 // Multilevel restriction R_l = sum of children, levels 0 to 2 in one launch.
@@ -976,25 +979,25 @@ __device__ inline void restrict_bank(int b, int B, int L, int cnt1, int beg1, co
 // component sums, so results do not depend on the schedule.
 template <typename V, typename T>
 __global__ void __launch_bounds__(kTB) k_restrict_all(const V* __restrict__ r, long long sub3, int B, int L,
-                                                       const int* __restrict__ ls, const int* __restrict__ part_map,
+                                                       const int* __restrict__ ls,
+                                                       const SlotNode* __restrict__ slot_node,
                                                        const int* __restrict__ going_next,
-                                                       const unsigned* __restrict__ fine_mask,
                                                        const unsigned* __restrict__ comp_mask,
                                                        const int* __restrict__ l1lo, const int* __restrict__ l1hi,
                                                        T* __restrict__ R,
                                                        const int* __restrict__ ctrl, SceneSkip skip) {
+    const BankIdx pre = bank_index(blockIdx.x, B, L, ls[2], ls[3], slot_node, going_next, comp_mask, l1lo, l1hi);
     if (ctrl && ctrl[0]) return;
     if (skip.bank_scene && skip.stopped(ls[3] / B + (int)blockIdx.x)) return;
     __shared__ T sv[3][kTB];
     __shared__ T l1v[3][32];
-    auto value = [&](int v, int, bool own, T& v0, T& v1, T& v2) {
-        if (!own) return;
+    V q0 = 0, q1 = 0, q2 = 0;
+    auto load = [&](int v) {
         const V* rv = r + sub3 + 3 * (size_t)v;
-        v0 = (T)rv[0]; v1 = (T)rv[1]; v2 = (T)rv[2];
+        q0 = rv[0]; q1 = rv[1]; q2 = rv[2];
     };
-    const BankIdx pre = bank_index(blockIdx.x, B, L, ls[2], ls[3], part_map, going_next, comp_mask, l1lo, l1hi);
-    restrict_bank<T>(blockIdx.x, B, L, ls[2], ls[3], part_map, going_next, fine_mask, comp_mask, pre, R, sv, l1v,
-                     value);
+    auto value = [&](int, T& v0, T& v1, T& v2) { v0 = (T)q0; v1 = (T)q1; v2 = (T)q2; };
+    restrict_bank<T>(blockIdx.x, B, L, ls[3], slot_node, pre, R, sv, l1v, false, load, value);
 }
 
 // One PCG step fused with the restriction of its new residual:
@@ -1004,46 +1007,71 @@ __global__ void __launch_bounds__(kTB) k_restrict_all(const V* __restrict__ r, l
 // a level-0 bank straddles two level-1 banks) and stores x, r and R_0 only
 // for the banks it owns; workgroups [g1, grid) update the dofs outside the
 // preconditioned range.  The iteration counter advances at the end.
+// Bound by dependent round trips (606 workgroups at 137 k rows): the slot
+// entries, the vectors of the first slots and both sets of dot partials are in
+// flight before the stop word is looked at, one barrier joins both sums, and
+// a component's lanes are summed from reads issued together.  At 137 k block
+// rows 12.3 -> 8.4 us per launch in FP32, 14.4 -> 11.3 us in FP64; 7.5 -> 6.7 us
+// at 525.
 template <typename V, typename T>
 __global__ void __launch_bounds__(kTB) k_update_restrict(
     long long N, double* __restrict__ x, V* __restrict__ r, const V* __restrict__ p, const V* __restrict__ Ap,
     const double* __restrict__ part_pap, int np_pap, const double* __restrict__ part_rz, int np_rz,
     double* __restrict__ part_rr, int* __restrict__ ctrl, int sub_off, int n_mas, int B, int L,
-    const int* __restrict__ ls, const int* __restrict__ part_map, const int* __restrict__ going_next,
-    const unsigned* __restrict__ fine_mask, const unsigned* __restrict__ comp_mask, const int* __restrict__ l1lo,
+    const int* __restrict__ ls, const SlotNode* __restrict__ slot_node, const int* __restrict__ going_next,
+    const unsigned* __restrict__ comp_mask, const int* __restrict__ l1lo,
     const int* __restrict__ l1hi, int nb1, int g1, T* __restrict__ R) {
-    if (ctrl[C_STOP]) return;
-    __shared__ double sh[2 * (kTB / 64)];
+    constexpr int NW = kTB / 64;
+    __shared__ double sh[3 * NW];
     __shared__ T sv[3][kTB];
     __shared__ T l1v[3][32];
-    // this workgroup's first bank indices, loaded while the dots are reduced
-    BankIdx pre{0, 0, -1, -1, 0u, false};
-    if ((int)blockIdx.x < g1 && (int)blockIdx.x < nb1)
-        pre = bank_index(blockIdx.x, B, L, ls[2], ls[3], part_map, going_next, comp_mask, l1lo, l1hi);
-    double rz, pap;
-    sum_partials2(part_rz, np_rz, part_pap, np_pap, sh, rz, pap);
-    const double al = rz / pap;
+    const bool banked = (int)blockIdx.x < g1 && (int)blockIdx.x < nb1;
+    const int cnt1 = ls[2], beg1 = ls[3];
+    // this workgroup's first bank: its indices, then its vertices' vectors
+    BankIdx pre{0, 0, -1, SlotNode{-1, -1, 0u, 0u}, 0u, false};
+    if (banked) pre = bank_index(blockIdx.x, B, L, cnt1, beg1, slot_node, going_next, comp_mask, l1lo, l1hi);
+    const double rz_share = strided_share<4>(part_rz, np_rz), pap_share = strided_share<8>(part_pap, np_pap);
+    V rv[3], av[3], pv[3];
+    double xv[3];
+    // only the vertex's owner reads and updates r in place (see restrict_bank)
+    auto load = [&](int v) {
+        const size_t o = 3 * ((size_t)sub_off + v);
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            rv[k] = r[o + k];
+            av[k] = Ap[o + k];
+            pv[k] = p[o + k];
+            xv[k] = x[o + k];
+        }
+    };
+    if (owned(pre.sn, blockIdx.x, B)) load(pre.sn.v);
+    if (ctrl[C_STOP]) return;
+    wave_sums_put(rz_share, sh);
+    wave_sums_put(pap_share, sh + NW);
+    __syncthreads();
+    const double al = wave_sums_total<NW>(sh) / wave_sums_total<NW>(sh + NW);
     double acc = 0.0;
     if ((int)blockIdx.x < g1) {
-        const int cnt1 = ls[2], beg1 = ls[3];
-        // only the vertex's owner reads and updates r in place (see restrict_bank)
-        auto value = [&](int v, int, bool own, T& v0, T& v1, T& v2) {
-            if (!own) return;
+        auto value = [&](int v, T& v0, T& v1, T& v2) {
             const size_t o = 3 * ((size_t)sub_off + v);
-            V r0 = (V)((double)r[o] - al * (double)Ap[o]);
-            V r1 = (V)((double)r[o + 1] - al * (double)Ap[o + 1]);
-            V r2 = (V)((double)r[o + 2] - al * (double)Ap[o + 2]);
-            x[o] += al * (double)p[o]; x[o + 1] += al * (double)p[o + 1]; x[o + 2] += al * (double)p[o + 2];
-            r[o] = r0; r[o + 1] = r1; r[o + 2] = r2;
-            acc += (double)r0 * (double)r0 + (double)r1 * (double)r1 + (double)r2 * (double)r2;
-            v0 = (T)r0; v1 = (T)r1; v2 = (T)r2;
+            V rn[3];
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                rn[k] = (V)((double)rv[k] - al * (double)av[k]);
+                x[o + k] = xv[k] + al * (double)pv[k];
+                r[o + k] = rn[k];
+                acc += (double)rn[k] * (double)rn[k];
+            }
+            v0 = (T)rn[0]; v1 = (T)rn[1]; v2 = (T)rn[2];
         };
-        for (int b = blockIdx.x; b < nb1; b += g1)
-            restrict_bank<T>(b, B, L, cnt1, beg1, part_map, going_next, fine_mask, comp_mask,
-                             b == (int)blockIdx.x ? pre
-                                                  : bank_index(b, B, L, cnt1, beg1, part_map, going_next, comp_mask,
-                                                               l1lo, l1hi),
-                             R, sv, l1v, value);
+        for (int b = blockIdx.x; b < nb1; b += g1) {
+            const bool at_first = b == (int)blockIdx.x;
+            if (!at_first) {
+                __syncthreads();  // the previous bank's level-1 sums have been read
+                pre = bank_index(b, B, L, cnt1, beg1, slot_node, going_next, comp_mask, l1lo, l1hi);
+            }
+            restrict_bank<T>(b, B, L, beg1, slot_node, pre, R, sv, l1v, at_first, load, value);
+        }
     } else {
         const long long m0 = 3LL * sub_off, m1 = 3LL * ((long long)sub_off + n_mas), nout = N - (m1 - m0);
         for (long long q = (long long)(blockIdx.x - g1) * kTB + threadIdx.x; q < nout;
@@ -1055,8 +1083,12 @@ __global__ void __launch_bounds__(kTB) k_update_restrict(
             acc += (double)ri * (double)ri;
         }
     }
-    write_partial(acc, part_rr, sh);
-    if (blockIdx.x == 0 && threadIdx.x == 0) ctrl[C_ITER] += 1;
+    wave_sums_put(acc, sh + 2 * NW);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        part_rr[blockIdx.x] = wave_sums_total<NW>(sh + 2 * NW);
+        if (blockIdx.x == 0) ctrl[C_ITER] += 1;
+    }
 }
 
 // Levels 2 -> 3 -> ... -> L-1 (few nodes): one workgroup, level by level.
@@ -1288,9 +1320,8 @@ void mas_restrict_t(Ctx& c, const V* r, long long sub3, T* R, const int* ctrl, b
     MasState& m = c.mas;
     if (m.nb1 <= 0) return;
     hipLaunchKernelGGL((k_restrict_all<V, T>), dim3(m.nb1), dim3(kTB), 0, c.stream, r, sub3, m.bank, m.L,
-                       (const int*)m.level_size.p, (const int*)m.part_map.p, (const int*)m.going_next.p,
-                       (const unsigned*)m.fine_mask.p, (const unsigned*)m.comp_mask.p,
-                       (const int*)m.l1lo.p, (const int*)m.l1hi.p, R, ctrl, skip);
+                       (const int*)m.level_size.p, (const SlotNode*)m.slot_node.p, (const int*)m.going_next.p,
+                       (const unsigned*)m.comp_mask.p, (const int*)m.l1lo.p, (const int*)m.l1hi.p, R, ctrl, skip);
     SGIPC_LAUNCH_CHECK();
     if (top && m.L >= 4) {
         hipLaunchKernelGGL((k_restrict_top<T>), dim3(1), dim3(kTop), 0, c.stream, m.bank, m.L,
@@ -1365,6 +1396,7 @@ void mas_set_topology(Ctx& c, int n, int node_offset, const unsigned* nstart, co
     }
     if (nlist_len) SGIPC_HIP(hipMemcpy(m.nlist.p, nlist, sizeof(unsigned) * nlist_len, hipMemcpyHostToDevice));
     m.fine_mask.reserve((size_t)n + 1);
+    m.slot_node.reserve((size_t)M + 1);
     m.next_mask.reserve((size_t)n + bank + 1);
     size_t nbk = (size_t)std::max(M, n) / bank + 2;
     m.prefix0.reserve(nbk);
@@ -1409,7 +1441,7 @@ void mas_build(Ctx& c, int sub_offset, int sub_nb, const int* pairs, int npairs)
     hipLaunchKernelGGL(k_set_level_size, dim3(1), dim3(1), 0, s, ls, 0, tot + 6, B, Mpad);
     SGIPC_LAUNCH_CHECK();
     hipLaunchKernelGGL(k_level1, dim3(div_up(M, kTB)), dim3(kTB), 0, s, M, Mpad, n, B, m.part_map.p, m.fine_mask.p,
-                       m.psum0.p, m.coarse_space.p, m.going_next.p);
+                       m.psum0.p, m.coarse_space.p, m.going_next.p, m.slot_node.p);
     SGIPC_LAUNCH_CHECK();
     const int nmax = n;  // level-local node count never exceeds n
     for (int level = 1; level < L; ++level) {
@@ -1635,16 +1667,14 @@ static void update_restrict_t(Ctx& c, double* x, V* r, const V* p, const V* Ap, 
     if (fp32) {
         hipLaunchKernelGGL((k_update_restrict<V, float>), dim3(g1 + gx), dim3(kTB), 0, c.stream, N, x, r, p, Ap,
                            part_pap, np_pap, part_rz, np_rz, part_rr, ctrl, c.sub_offset, m.n, m.bank, m.L,
-                           (const int*)m.level_size.p, (const int*)m.part_map.p, (const int*)m.going_next.p,
-                           (const unsigned*)m.fine_mask.p, (const unsigned*)m.comp_mask.p,
-                           (const int*)m.l1lo.p, (const int*)m.l1hi.p, m.nb1, g1, m.R32.p);
+                           (const int*)m.level_size.p, (const SlotNode*)m.slot_node.p, (const int*)m.going_next.p,
+                           (const unsigned*)m.comp_mask.p, (const int*)m.l1lo.p, (const int*)m.l1hi.p, m.nb1, g1, m.R32.p);
     } else {
         if (sizeof(V) != 8) throw state_error("MAS: FP32 residual needs the FP32 preconditioner data");
         hipLaunchKernelGGL((k_update_restrict<V, double>), dim3(g1 + gx), dim3(kTB), 0, c.stream, N, x, r, p, Ap,
                            part_pap, np_pap, part_rz, np_rz, part_rr, ctrl, c.sub_offset, m.n, m.bank, m.L,
-                           (const int*)m.level_size.p, (const int*)m.part_map.p, (const int*)m.going_next.p,
-                           (const unsigned*)m.fine_mask.p, (const unsigned*)m.comp_mask.p,
-                           (const int*)m.l1lo.p, (const int*)m.l1hi.p, m.nb1, g1, m.R64.p);
+                           (const int*)m.level_size.p, (const SlotNode*)m.slot_node.p, (const int*)m.going_next.p,
+                           (const unsigned*)m.comp_mask.p, (const int*)m.l1lo.p, (const int*)m.l1hi.p, m.nb1, g1, m.R64.p);
     }
     SGIPC_LAUNCH_CHECK();
     if (m.L >= 4 && top) {

@@ -43,6 +43,40 @@ __device__ inline void block_sum_all2(double& a, double& b, double* sh) {
     b = sb;
 }
 
+// This thread's strided share of np partials, U of them in flight together (a
+// loop of dependent load and add takes one round trip each).  Loads past the
+// end are clamped to the last partial: U should not be far above np / threads.
+template <int U>
+__device__ inline double strided_share(const double* __restrict__ part, int np) {
+    double v = 0.0;
+    for (int i = threadIdx.x; i < np; i += U * blockDim.x) {
+        double q[U];
+#pragma unroll
+        for (int k = 0; k < U; ++k) {
+            const int j = i + k * (int)blockDim.x;
+            q[k] = part[min(j, np - 1)];
+        }
+#pragma unroll
+        for (int k = 0; k < U; ++k)
+            if (i + k * (int)blockDim.x < np) v += q[k];
+    }
+    return v;
+}
+
+// The wavefronts' sums of v meet in sh[0 .. waves) (written here; read them
+// after a barrier with wave_sums_total, in wavefront order)
+__device__ inline void wave_sums_put(double v, double* sh) {
+    v = wave_sum(v);
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
+}
+template <int NW>
+__device__ inline double wave_sums_total(const double* sh) {
+    double s = 0.0;
+#pragma unroll
+    for (int i = 0; i < NW; ++i) s += sh[i];
+    return s;
+}
+
 // sums of two partial sets, as two sum_partials calls would give them
 __device__ inline void sum_partials2(const double* __restrict__ pa, int na, const double* __restrict__ pb, int nb,
                                      double* sh, double& a, double& b) {
@@ -77,21 +111,13 @@ constexpr int kLevelBatch = 8;    // MAS levels whose loads are in flight togeth
 // sum_partials), so a kernel can issue its loads early and reduce late.
 __device__ inline double stop_share(int rule, const double* __restrict__ part_rz_prev, int np_rz,
                                     const double* __restrict__ part_rr, int np_rr) {
-    double v = 0.0;
-    if (rule == 0) {
-        for (int i = threadIdx.x; i < np_rz; i += blockDim.x) v += part_rz_prev[i];
-    } else if (rule > 0) {
-        for (int i = threadIdx.x; i < np_rr; i += blockDim.x) v += part_rr[i];
-    }
-    return v;
+    return rule == 0 ? strided_share<4>(part_rz_prev, np_rz) : rule > 0 ? strided_share<4>(part_rr, np_rr) : 0.0;
 }
 
-// Stop test from the shares: rule 0 |r.z| <= tol * r0.z0 (previous r.z),
+// Stop test from the sum of the shares: rule 0 |r.z| <= tol * r0.z0 (previous r.z),
 // rule 1 ||r|| <= tol * ||b||; block 0 records the progress and the stop.
-__device__ inline bool stop_test_share(int rule, double share, double* __restrict__ sc, int* __restrict__ ctrl,
-                                       double* sh) {
+__device__ inline bool stop_test_sum(int rule, double sum, double* __restrict__ sc, int* __restrict__ ctrl) {
     if (rule < 0) return false;
-    const double sum = block_sum_all(share, sh);
     bool stop;
     double q;  // progress: the ratio compared with the tolerance
     if (rule == 0) {
@@ -111,7 +137,9 @@ __device__ inline bool stop_test_share(int rule, double share, double* __restric
 __device__ inline bool stop_test(int rule, const double* __restrict__ part_rz_prev, int np_rz,
                                  const double* __restrict__ part_rr, int np_rr, double* __restrict__ sc,
                                  int* __restrict__ ctrl, double* sh) {
-    return stop_test_share(rule, stop_share(rule, part_rz_prev, np_rz, part_rr, np_rr), sc, ctrl, sh);
+    if (rule < 0) return false;
+    const double sum = block_sum_all(stop_share(rule, part_rz_prev, np_rz, part_rr, np_rr), sh);
+    return stop_test_sum(rule, sum, sc, ctrl);
 }
 
 // Progress words for the host's pinned-memory polling: the stop and

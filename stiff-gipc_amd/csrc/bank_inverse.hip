@@ -22,6 +22,7 @@
 //    refinement step X1 = X0 + X0 (I - A X0) with the residual I - A X0
 //    accumulated in FP64 MFMA from the FP64 bank matrix; X1 is stored FP32.
 #include "context.hpp"
+#include "bank_solve.hpp"
 #include <utility>
 
 namespace sgipc {
@@ -202,13 +203,13 @@ __global__ void __launch_bounds__(64) k_bank_inverse_mfma(int nbanks, const doub
     }
     __syncthreads();
     block_gauss_jordan<T, NT>(S, W, l);
-    // upper triangle (r <= c) packed by rows
+    // upper triangle (r <= c)
     for (int e = l; e < NP; e += 64) {
         const int r = packed_row<D>(e);
         const int c = r + (e - r * (2 * D - r + 1) / 2);
         const T v = S.at(r, c);
-        if constexpr (sizeof(T) == 8) inv64[(size_t)b * NP + e] = v;
-        inv32[(size_t)b * NP + e] = (float)v;
+        if constexpr (sizeof(T) == 8) inv64[(size_t)b * NP + inv_index<D, double>(r, c)] = v;
+        inv32[(size_t)b * NP + inv_index<D, float>(r, c)] = (float)v;
     }
 }
 
@@ -336,7 +337,7 @@ __global__ void __launch_bounds__(64) k_bank_inverse_mfma48(int nbanks, const do
         A[k][k] = P;
         __syncthreads();
     }
-    // upper triangle (row <= column) packed by rows
+    // upper triangle (row <= column)
     double* o64 = inv64 + (size_t)b * NP;
     float* o32 = inv32 + (size_t)b * NP;
 #pragma unroll
@@ -347,9 +348,8 @@ __global__ void __launch_bounds__(64) k_bank_inverse_mfma48(int nbanks, const do
             for (int r = 0; r < 4; ++r) {
                 const int row = 16 * ti + Mf<T>::row(q, r), c = 16 * tj + j;
                 if (row <= c) {
-                    const int e = row * (2 * D - row + 1) / 2 + (c - row);
-                    if constexpr (sizeof(T) == 8) o64[e] = A[ti][tj][r];
-                    o32[e] = (float)A[ti][tj][r];
+                    if constexpr (sizeof(T) == 8) o64[inv_index<D, double>(row, c)] = A[ti][tj][r];
+                    o32[inv_index<D, float>(row, c)] = (float)A[ti][tj][r];
                 }
             }
     if (inv16 == nullptr) return;
@@ -378,10 +378,9 @@ __global__ void __launch_bounds__(64) k_bank_inverse_mfma48(int nbanks, const do
             for (int r = 0; r < 4; ++r) {
                 const int row = 16 * ti + Mf<T>::row(q, r), c = 16 * tj + j;
                 if (row <= c) {
-                    const int e = row * (2 * D - row + 1) / 2 + (c - row);
                     const float v = (float)((double)A[ti][tj][r] / (dg[row] * dg[c]));
                     const _Float16 hv = (_Float16)fminf(fmaxf(v, -65504.f), 65504.f);
-                    o16[e] = __builtin_bit_cast(unsigned short, hv);
+                    o16[inv_index<D, _Float16>(row, c)] = __builtin_bit_cast(unsigned short, hv);
                 }
             }
 }
@@ -408,7 +407,7 @@ __global__ void __launch_bounds__(64) k_bank_refine(int nbanks, const double* __
     for (int e = l; e < NP; e += 64) {
         const int r = packed_row<D>(e);
         const int c = r + (e - r * (2 * D - r + 1) / 2);
-        const double v = (double)out[e];
+        const double v = (double)out[inv_index<D, float>(r, c)];
         X.at(r, c) = v;
         X.at(c, r) = v;
     }
@@ -451,7 +450,7 @@ __global__ void __launch_bounds__(64) k_bank_refine(int nbanks, const double* __
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int row = 16 * i + Mf<double>::row(q, r);
-                if (row <= c) out[row * (2 * D - row + 1) / 2 + (c - row)] = (float)a[r];
+                if (row <= c) out[inv_index<D, float>(row, c)] = (float)a[r];
             }
         }
     }

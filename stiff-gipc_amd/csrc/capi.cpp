@@ -4,6 +4,7 @@
 #include <vector>
 #include "../../include/sgipc.h"
 #include "context.hpp"
+#include "bank_solve.hpp"
 
 #include <new>
 
@@ -750,6 +751,14 @@ int sgipc_mas_tables(sgipc_ctx* c, int* cs, int* gn, int* ct, uint32_t* fm, int*
     });
 }
 
+}  // extern "C"
+// place of element (r, c), r <= c, in the device storage of a bank's inverse
+template <typename S>
+static int bank_place(int bank, int r, int c) {
+    return bank == 16 ? sgipc::inv_index<48, S>(r, c) : sgipc::inv_index<96, S>(r, c);
+}
+extern "C" {
+
 int sgipc_mas_bank_inverse(sgipc_ctx* c, int b, double* inv) {
     CHECK_CTX(c);
     return guard(c, [&] {
@@ -759,13 +768,12 @@ int sgipc_mas_bank_inverse(sgipc_ctx* c, int b, double* inv) {
         if (b < 0 || b >= m.nbanks || !inv) throw sgipc::arg_error("mas_bank_inverse: bad bank");
         set_device(c);
         SGIPC_HIP(hipStreamSynchronize(c->stream));
-        // device copy: upper triangle packed by rows; expand to dense row-major
+        // expand the device storage (upper triangle) to dense row-major
         const size_t D = 3 * (size_t)m.bank, NP = D * (D + 1) / 2;
         std::vector<double> up(NP);
         SGIPC_HIP(hipMemcpy(up.data(), m.inv64.p + (size_t)b * NP, sizeof(double) * NP, hipMemcpyDeviceToHost));
-        size_t e = 0;
-        for (size_t r = 0; r < D; ++r)
-            for (size_t q = r; q < D; ++q, ++e) inv[r * D + q] = inv[q * D + r] = up[e];
+        for (int r = 0; r < (int)D; ++r)
+            for (int q = r; q < (int)D; ++q) inv[r * D + q] = inv[q * D + r] = up[bank_place<double>(m.bank, r, q)];
     });
 }
 
@@ -780,9 +788,8 @@ int sgipc_mas_bank_inverse_f32(sgipc_ctx* c, int b, float* inv) {
         const size_t D = 3 * (size_t)m.bank, NP = D * (D + 1) / 2;
         std::vector<float> up(NP);
         SGIPC_HIP(hipMemcpy(up.data(), m.inv32.p + (size_t)b * NP, sizeof(float) * NP, hipMemcpyDeviceToHost));
-        size_t e = 0;
-        for (size_t r = 0; r < D; ++r)
-            for (size_t q = r; q < D; ++q, ++e) inv[r * D + q] = inv[q * D + r] = up[e];
+        for (int r = 0; r < (int)D; ++r)
+            for (int q = r; q < (int)D; ++q) inv[r * D + q] = inv[q * D + r] = up[bank_place<float>(m.bank, r, q)];
     });
 }
 
@@ -800,11 +807,10 @@ int sgipc_mas_bank_inverse_f16(sgipc_ctx* c, int b, float* inv) {
         std::vector<float> d(D);
         SGIPC_HIP(hipMemcpy(up.data(), m.inv16.p + (size_t)b * NP, sizeof(unsigned short) * NP, hipMemcpyDeviceToHost));
         SGIPC_HIP(hipMemcpy(d.data(), m.inv16_d.p + (size_t)b * D, sizeof(float) * D, hipMemcpyDeviceToHost));
-        size_t e = 0;
-        for (size_t r = 0; r < D; ++r)
-            for (size_t q = r; q < D; ++q, ++e) {
+        for (int r = 0; r < (int)D; ++r)
+            for (int q = r; q < (int)D; ++q) {
                 _Float16 h;
-                std::memcpy(&h, &up[e], sizeof h);
+                std::memcpy(&h, &up[bank_place<unsigned short>(m.bank, r, q)], sizeof h);
                 inv[r * D + q] = inv[q * D + r] = d[r] * (float)h * d[q];
             }
     });

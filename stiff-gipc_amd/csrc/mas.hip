@@ -18,6 +18,7 @@
 #include <rocprim/device/device_radix_sort.hpp>
 #include <utility>
 #include "pcg_dev.hpp"
+#include "bank_solve.hpp"
 #include <algorithm>
 
 namespace sgipc {
@@ -584,11 +585,6 @@ __global__ void k_owned_vertices(int nb0, int B, const int* __restrict__ prefix0
     atomicMax(vhi + f, mx + 1);
 }
 
-// element (r, c), r <= c, of a symmetric D x D matrix stored as its upper
-// triangle packed by rows
-template <int D>
-__device__ inline int sym_index(int r, int c) { return r * (2 * D - r + 1) / 2 + (c - r); }
-
 // ---- bank inverse: unpivoted in-place Gauss-Jordan in LDS -------------------
 template <int B>
 __global__ void __launch_bounds__(B == 16 ? 64 : 128) k_bank_inverse(int nbanks, const double* __restrict__ bank_upper,
@@ -635,9 +631,8 @@ __global__ void __launch_bounds__(B == 16 ? 64 : 128) k_bank_inverse(int nbanks,
         double* o64 = inv64 + (size_t)b * NP;
         float* o32 = inv32 + (size_t)b * NP;
         for (int r = 0; r <= i; ++r) {
-            int e = sym_index<D>(r, i);
-            o64[e] = S[r][i];
-            o32[e] = (float)S[r][i];
+            o64[inv_index<D, double>(r, i)] = S[r][i];
+            o32[inv_index<D, float>(r, i)] = (float)S[r][i];
         }
     }
 }
@@ -743,9 +738,8 @@ __global__ void __launch_bounds__(64) k_bank_inverse_reg48(int nbanks, const dou
 #pragma unroll
         for (int r = 0; r < D; ++r)
             if (r <= i) {
-                const int e = sym_index<D>(r, i);
-                o64[e] = S[r];
-                o32[e] = (float)S[r];
+                o64[inv_index<D, double>(r, i)] = S[r];
+                o32[inv_index<D, float>(r, i)] = (float)S[r];
             }
     }
 }
@@ -764,7 +758,7 @@ __global__ void __launch_bounds__(64) k_pack_inv_half(int nbanks, const S* __res
     if (b >= nbanks) return;
     const S* src = inv + (size_t)b * NP;
     if (i < D) {
-        const double a = (double)src[pack_index(D, i, i)];
+        const double a = (double)src[inv_index<D, S>(i, i)];
         const double di = a > 0.0 ? sqrt(a) : 1.0;
         d[i] = di;
         dsc[(size_t)b * D + i] = (float)di;
@@ -774,48 +768,35 @@ __global__ void __launch_bounds__(64) k_pack_inv_half(int nbanks, const S* __res
     for (int r = 0; r < D; ++r) {
         const int c = r + i;
         if (c < D) {
-            const int q = pack_index(D, r, c);
-            const float v = (float)((double)src[q] / (d[r] * d[c]));
+            const float v = (float)((double)src[inv_index<D, S>(r, c)] / (d[r] * d[c]));
             const _Float16 hv = (_Float16)fminf(fmaxf(v, -65504.f), 65504.f);
-            dst[q] = __builtin_bit_cast(unsigned short, hv);
+            dst[inv_index<D, _Float16>(r, c)] = __builtin_bit_cast(unsigned short, hv);
         }
     }
 }
 
 // ---- apply -----------------------------------------------------------------
-// value of v in lane j of the wavefront (j uniform)
-__device__ inline float lane_bcast(float v, int j) {
-    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), j));
-}
-__device__ inline double lane_bcast(double v, int j) {
-    const long long b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_readlane((int)(b & 0xffffffffll), j);
-    const int hi = __builtin_amdgcn_readlane((int)(b >> 32), j);
-    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
-}
-
 // address-space-qualified pointers for the direct global -> LDS load builtin
 typedef __attribute__((address_space(1))) const void* gptr_t;
 typedef __attribute__((address_space(3))) void* lptr_t;
 
-// z_bank = A^-1 r_bank for every bank of every level: the packed inverse is
-// staged through LDS (the bytes of this kernel are almost all inverse
-// bytes), then lane i forms row i, summing over columns in order.
-template <int B, typename T>
-__global__ void __launch_bounds__(B == 16 ? 64 : 128) k_bank_solve(const T* __restrict__ inv, const T* __restrict__ R,
-                                                                    T* __restrict__ Z, const int* __restrict__ ctrl,
-                                                                    SceneSkip skip) {
+// z_bank = A^-1 r_bank for every bank of every level, 32-vertex banks: the
+// packed inverse is staged through LDS (the bytes of this kernel are almost
+// all inverse bytes), then lane i forms row i, summing over columns in order.
+template <typename T>
+__global__ void __launch_bounds__(128) k_bank_solve32(const T* __restrict__ inv, const T* __restrict__ R,
+                                                      T* __restrict__ Z, const int* __restrict__ ctrl,
+                                                      SceneSkip skip) {
     if (ctrl && ctrl[0]) return;
     if (skip.stopped(blockIdx.x)) return;
-    constexpr int D = 3 * B;
+    constexpr int D = 96, NT = 128;
     constexpr int NP = D * (D + 1) / 2;
-    constexpr int NT = (B == 16) ? 64 : 128;
-    constexpr int NV = NP * (int)sizeof(T) / 16;  // exact: NP * sizeof(T) is a multiple of 16 for B = 16, 32
+    constexpr int NV = NP * (int)sizeof(T) / 16;
     static_assert(NP * sizeof(T) % 16 == 0, "packed bank must be a whole number of 16-byte vectors");
     using V4 = typename std::conditional<sizeof(T) == 8, double2, float4>::type;
     constexpr int PER = (NV + NT - 1) / NT;
     __shared__ V4 As[PER * NT];  // padded to whole 1 KB wave chunks
-    __shared__ T rs[B == 16 ? 1 : D];
+    __shared__ T rs[D];
     const int b = blockIdx.x, i = threadIdx.x;
     const V4* src = reinterpret_cast<const V4*>(inv + (size_t)b * NP);
     // Direct global -> LDS loads (16 B per lane, one 1 KB chunk per wave and
@@ -829,27 +810,38 @@ __global__ void __launch_bounds__(B == 16 ? 64 : 128) k_bank_solve(const T* __re
         __builtin_amdgcn_global_load_lds((gptr_t)(src + min(q0 + lane, NV - 1)), (lptr_t)(As + q0), 16, 0, 0);
     }
     __builtin_amdgcn_s_waitcnt(0);
-    if constexpr (B != 16) {
-        if (i < D) rs[i] = rv;
-    }
+    if (i < D) rs[i] = rv;
     __syncthreads();
     if (i >= D) return;
     const T* A = reinterpret_cast<const T*>(As);
     // Row i of the symmetric bank from the packed upper triangle: element
     // (j, i) for j <= i, then (i, j); the packed index advances by D - 1 - j
-    // while j < i and by 1 after.  r_j comes from lane j's register when the
-    // bank fits one wavefront (B = 16), from LDS otherwise.
+    // while j < i and by 1 after.
     T acc = 0;
     int idx = i;  // (0, i)
 #pragma unroll 8
     for (int j = 0; j < D; ++j) {
-        T rj;
-        if constexpr (B == 16) rj = lane_bcast(rv, j);
-        else rj = rs[j];
-        acc += A[idx] * rj;
+        acc += A[idx] * rs[j];
         idx += (j < i) ? (D - 1 - j) : 1;
     }
     Z[(size_t)b * D + i] = acc;
+}
+
+// 16-vertex banks: one wavefront per bank
+constexpr int kBankWaves = 4;
+template <typename T>
+__global__ void __launch_bounds__(64 * kBankWaves) k_bank_solve16(int nbanks, const T* __restrict__ inv,
+                                                                  const T* __restrict__ R, T* __restrict__ Z,
+                                                                  const int* __restrict__ ctrl, SceneSkip skip) {
+    if (ctrl && ctrl[0]) return;
+    __shared__ T lds[kBankWaves][kBankLds];
+    const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63, b = blockIdx.x * kBankWaves + wv;
+    if (b >= nbanks || skip.stopped(b)) return;
+    BankSolve<T, T> B;
+    B.load_r(R, b, lane);
+    B.load(inv, nullptr, b, lane);
+    const T z = B.solve(lds[wv], lane);
+    if (lane < 48) Z[(size_t)b * 48 + lane] = z;
 }
 
 template <typename T>
@@ -868,24 +860,24 @@ __global__ void k_collect(int n, int L, const int* __restrict__ node_of, const T
 // Component sum of one bank-aligned group of nodes held in LDS (one node
 // per thread).  `mask` holds the bank lanes of this node's component (its
 // closure, self included); only the lowest lane of the component sums, in
-// ascending lane order (16 lanes' values are read at once; a lane outside the
+// ascending lane order (U lanes' values are read at once; a lane outside the
 // component adds nothing).  Returns true for that lane, with the sums.
-template <typename T>
+template <typename T, int U = 16>
 __device__ inline bool component_sum(unsigned mask, const T* a0, const T* a1, const T* a2, int B, T& s0, T& s1,
                                      T& s2) {
     const int t = threadIdx.x, lane = t & (B - 1), bbase = t - lane;
     if (mask & ltmask(lane)) return false;
     s0 = 0; s1 = 0; s2 = 0;
-    for (int h = 0; h < B; h += 16) {
-        T q[16][3];
+    for (int h = 0; h < B; h += U) {
+        T q[U][3];
 #pragma unroll
-        for (int l = 0; l < 16; ++l) {
+        for (int l = 0; l < U; ++l) {
             q[l][0] = a0[bbase + h + l];
             q[l][1] = a1[bbase + h + l];
             q[l][2] = a2[bbase + h + l];
         }
 #pragma unroll
-        for (int l = 0; l < 16; ++l)
+        for (int l = 0; l < U; ++l)
             if ((mask >> (h + l)) & 1u) { s0 += q[l][0]; s1 += q[l][1]; s2 += q[l][2]; }
     }
     return true;
@@ -1026,11 +1018,14 @@ __global__ void __launch_bounds__(kTB) k_update_restrict(
     __shared__ T sv[3][kTB];
     __shared__ T l1v[3][32];
     const bool banked = (int)blockIdx.x < g1 && (int)blockIdx.x < nb1;
-    const int cnt1 = ls[2], beg1 = ls[3];
+    const int stopped = ctrl[C_STOP], cnt1 = ls[2], beg1 = ls[3];
+    Share<4, kTB> rz_share;
+    Share<8, kTB> pap_share;
+    rz_share.take(part_rz, np_rz);
+    pap_share.take(part_pap, np_pap);
     // this workgroup's first bank: its indices, then its vertices' vectors
     BankIdx pre{0, 0, -1, SlotNode{-1, -1, 0u, 0u}, 0u, false};
     if (banked) pre = bank_index(blockIdx.x, B, L, cnt1, beg1, slot_node, going_next, comp_mask, l1lo, l1hi);
-    const double rz_share = strided_share<4>(part_rz, np_rz), pap_share = strided_share<8>(part_pap, np_pap);
     V rv[3], av[3], pv[3];
     double xv[3];
     // only the vertex's owner reads and updates r in place (see restrict_bank)
@@ -1045,9 +1040,9 @@ __global__ void __launch_bounds__(kTB) k_update_restrict(
         }
     };
     if (owned(pre.sn, blockIdx.x, B)) load(pre.sn.v);
-    if (ctrl[C_STOP]) return;
-    wave_sums_put(rz_share, sh);
-    wave_sums_put(pap_share, sh + NW);
+    if (stopped) return;
+    wave_sums_put(rz_share.sum(), sh);
+    wave_sums_put(pap_share.sum(), sh + NW);
     __syncthreads();
     const double al = wave_sums_total<NW>(sh) / wave_sums_total<NW>(sh + NW);
     double acc = 0.0;
@@ -1142,89 +1137,14 @@ __global__ void __launch_bounds__(kTop) k_restrict_top(int B, int L, const int* 
 // then solves the banks of levels >= 3 on its own results; the other
 // workgroups solve every bank of levels 0..2, whose restriction is complete
 // at launch, at the same time.  No workgroup waits for another.
-constexpr int kCW = 8;               // wavefronts per workgroup of k_mas_coarse
+constexpr int kCW = 8;               // wavefronts per workgroup
 constexpr int kCT = 64 * kCW;
 
-// One 48 x 48 bank solve by one wavefront: the packed FP32/FP64 inverse is
-// staged into this wavefront's LDS area by direct global -> LDS loads, lane
-// i < 48 forms row i (the arithmetic of k_bank_solve<16>).
-template <typename T>
-__device__ inline T wave_bank_solve(const T* __restrict__ inv, const T* __restrict__ R, int b, void* lds) {
-    constexpr int D = 48, NP = D * (D + 1) / 2;
-    using V4 = typename std::conditional<sizeof(T) == 8, double2, float4>::type;
-    constexpr int NV = NP * (int)sizeof(T) / 16;
-    constexpr int PER = (NV + 63) / 64;
-    V4* As = static_cast<V4*>(lds);
-    const int i = threadIdx.x & 63;
-    const V4* src = reinterpret_cast<const V4*>(inv + (size_t)b * NP);
-    const T rv = R[(size_t)b * D + min(i, D - 1)];
-#pragma unroll
-    for (int k = 0; k < PER; ++k) {
-        const int q0 = k * 64;
-        __builtin_amdgcn_global_load_lds((gptr_t)(src + min(q0 + i, NV - 1)), (lptr_t)(As + q0), 16, 0, 0);
-    }
-    __builtin_amdgcn_s_waitcnt(0);
-    __builtin_amdgcn_wave_barrier();
-    const T* A = reinterpret_cast<const T*>(As);
-    T acc = 0;
-    if (i < D) {
-        int idx = i;
-#pragma unroll 8
-        for (int j = 0; j < D; ++j) {
-            acc += A[idx] * lane_bcast(rv, j);
-            idx += (j < i) ? (D - 1 - j) : 1;
-        }
-    }
-    __builtin_amdgcn_wave_barrier();  // every lane's reads of this bank done before the area is reused
-    return acc;
-}
-
-// The same solve from the half-storage form of an inverse: inv = D S D with
-// D = diag(sqrt(inv_ii)) (FP32, one per bank row) and S (unit diagonal,
-// |S_ij| <= 1 for an SPD inverse) packed like inv as FP16, so the bank reads
-// 2352 + 192 bytes instead of 4704.  z_i = d_i sum_j S_ij (d_j r_j), FP32
-// arithmetic.
-__device__ inline float wave_bank_solve_h(const unsigned short* __restrict__ inv, const float* __restrict__ dsc,
-                                          const float* __restrict__ R, int b, void* lds) {
-    constexpr int D = 48, NP = D * (D + 1) / 2;
-    constexpr int NV = NP * 2 / 16;  // 147 16-byte pieces per bank (2352 bytes)
-    constexpr int PER = (NV + 63) / 64;
-    float4* As = static_cast<float4*>(lds);
-    const int i = threadIdx.x & 63;
-    const float4* src = reinterpret_cast<const float4*>(inv + (size_t)b * NP);
-    const float di = dsc[(size_t)b * D + min(i, D - 1)];
-    const float rv = R[(size_t)b * D + min(i, D - 1)] * di;
-#pragma unroll
-    for (int k = 0; k < PER; ++k) {
-        const int q0 = k * 64;
-        __builtin_amdgcn_global_load_lds((gptr_t)(src + min(q0 + i, NV - 1)), (lptr_t)(As + q0), 16, 0, 0);
-    }
-    __builtin_amdgcn_s_waitcnt(0);
-    __builtin_amdgcn_wave_barrier();
-    const _Float16* A = reinterpret_cast<const _Float16*>(As);
-    float acc = 0.f;
-    if (i < D) {
-        int idx = i;
-#pragma unroll 8
-        for (int j = 0; j < D; ++j) {
-            acc += (float)A[idx] * lane_bcast(rv, j);
-            idx += (j < i) ? (D - 1 - j) : 1;
-        }
-    }
-    __builtin_amdgcn_wave_barrier();
-    return acc * di;
-}
-
-// one bank solve from either storage (H: the half form; inv is then the FP16
-// S and dsc its row scales)
-template <typename T, bool H>
-__device__ inline T bank_solve_any(const void* __restrict__ inv, const float* __restrict__ dsc,
-                                   const T* __restrict__ R, int b, void* lds) {
-    if constexpr (H) return wave_bank_solve_h(static_cast<const unsigned short*>(inv), dsc, R, b, lds);
-    else return wave_bank_solve<T>(static_cast<const T*>(inv), R, b, lds);
-}
-
-template <typename T, bool H>
+// NB banks per wavefront of the other workgroups (levels 0 .. 2).  Bound by the
+// inverses' bytes: 10,359 banks, 49 MB FP32 / 97 MB FP64, 13.2 -> 9.7 us and
+// 20.0 -> 17.2 us per launch against staging packed triangles in LDS (a plain
+// read of as many bytes takes about 8 and 15 us).
+template <typename T, bool H, int NB>
 __global__ void __launch_bounds__(kCT) k_mas_solve_top(int L, const int* __restrict__ ls,
                                                      const int* __restrict__ going_next,
                                                      const unsigned* __restrict__ comp_mask, int top_bank0,
@@ -1232,17 +1152,22 @@ __global__ void __launch_bounds__(kCT) k_mas_solve_top(int L, const int* __restr
                                                      const float* __restrict__ dsc, T* __restrict__ R,
                                                      T* __restrict__ Z, const int* __restrict__ ctrl, SceneSkip skip) {
     static_assert(!H || sizeof(T) == 4, "half-storage inverses serve FP32 applies");
-    if (ctrl[C_STOP]) return;
+    using Solve = BankSolve<T, typename std::conditional<H, _Float16, T>::type>;
     constexpr int D = 48;
-    using V4 = typename std::conditional<sizeof(T) == 8, double2, float4>::type;
-    constexpr int PER = ((D * (D + 1) / 2) * (int)sizeof(T) / 16 + 63) / 64;
-    static_assert(kCW * PER * 64 * sizeof(V4) >= 6 * kCT * sizeof(T), "LDS union too small");
-    __shared__ V4 lds[kCW][PER * 64];
+    static_assert(6 * kCT >= kCW * kBankLds, "one area for the restriction and the bank solves");
+    __shared__ T lds[6 * kCT];
     const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    T* mine = lds + kBankLds * wv;
+    const int stopped = ctrl[C_STOP];
     if (blockIdx.x == 0) {
+        // this wavefront's first top bank, loaded while the levels are restricted
+        Solve B;
+        const int b0 = top_bank0 + wv;
+        B.load(inv, dsc, min(b0, nbanks - 1), lane);
+        if (stopped) return;
         // levels 2 -> L-1, one level at a time (the sums of k_restrict_top)
-        T(*sv)[kCT] = reinterpret_cast<T(*)[kCT]>(&lds[0][0]);
-        T(*nx)[kCT] = reinterpret_cast<T(*)[kCT]>(reinterpret_cast<char*>(&lds[0][0]) + 3 * kCT * sizeof(T));
+        T(*sv)[kCT] = reinterpret_cast<T(*)[kCT]>(lds);
+        T(*nx)[kCT] = reinterpret_cast<T(*)[kCT]>(lds + 3 * kCT);
         const int t = threadIdx.x;
         bool in_lds = false;
         for (int l = 2; l + 1 < L; ++l) {
@@ -1263,7 +1188,7 @@ __global__ void __launch_bounds__(kCT) k_mas_solve_top(int L, const int* __restr
                 sv[0][t] = v0; sv[1][t] = v1; sv[2][t] = v2;
                 __syncthreads();
                 T s0, s1, s2;
-                if (valid && component_sum<T>(mask, sv[0], sv[1], sv[2], 16, s0, s1, s2)) {
+                if (valid && component_sum<T, 4>(mask, sv[0], sv[1], sv[2], 16, s0, s1, s2)) {
                     const size_t q = (size_t)pp;
                     R[3 * q] = s0; R[3 * q + 1] = s1; R[3 * q + 2] = s2;
                     if (next_fits) { const int j = (int)(q - begn); nx[0][j] = s0; nx[1][j] = s1; nx[2][j] = s2; }
@@ -1276,16 +1201,38 @@ __global__ void __launch_bounds__(kCT) k_mas_solve_top(int L, const int* __restr
         // the barrier orders this workgroup's global writes and reads)
         __threadfence_block();
         __syncthreads();
-        for (int b = top_bank0 + wv; b < nbanks; b += kCW) {
+        if (b0 < nbanks && !skip.stopped(b0)) {
+            B.load_r(R, b0, lane);
+            const T zb = B.solve(mine, lane);
+            if (lane < D) Z[(size_t)b0 * D + lane] = zb;
+        }
+        for (int b = b0 + kCW; b < nbanks; b += kCW) {
             if (skip.stopped(b)) continue;
-            const T zb = bank_solve_any<T, H>(inv, dsc, R, b, &lds[wv][0]);
+            Solve C;
+            C.load(inv, dsc, b, lane);
+            C.load_r(R, b, lane);
+            const T zb = C.solve(mine, lane);
             if (lane < D) Z[(size_t)b * D + lane] = zb;
         }
         return;
     }
-    const int b = (blockIdx.x - 1) * kCW + wv;  // levels 0 .. 2
-    if (b < top_bank0 && !skip.stopped(b)) {
-        const T zb = bank_solve_any<T, H>(inv, dsc, R, b, &lds[wv][0]);
+    Solve B[NB];
+    bool on[NB];
+#pragma unroll
+    for (int k = 0; k < NB; ++k) {
+        const int b = ((blockIdx.x - 1) * NB + k) * kCW + wv;
+        on[k] = b < top_bank0 && !skip.stopped(b);
+        if (on[k]) {
+            B[k].load_r(R, b, lane);
+            B[k].load(inv, dsc, b, lane);
+        }
+    }
+    if (stopped) return;
+#pragma unroll
+    for (int k = 0; k < NB; ++k) {
+        if (!on[k]) continue;
+        const int b = ((blockIdx.x - 1) * NB + k) * kCW + wv;
+        const T zb = B[k].solve(mine, lane);
         if (lane < D) Z[(size_t)b * D + lane] = zb;
     }
 }
@@ -1335,9 +1282,10 @@ void mas_solve_t(Ctx& c, const T* inv, const T* R, T* Z, const int* ctrl, SceneS
     MasState& m = c.mas;
     prof_begin(c, PROF_MAS_SOLVE);
     if (m.bank == 16)
-        hipLaunchKernelGGL((k_bank_solve<16, T>), dim3(m.nbanks), dim3(64), 0, c.stream, inv, R, Z, ctrl, skip);
+        hipLaunchKernelGGL(k_bank_solve16<T>, dim3(div_up(m.nbanks, kBankWaves)), dim3(64 * kBankWaves), 0, c.stream,
+                           m.nbanks, inv, R, Z, ctrl, skip);
     else
-        hipLaunchKernelGGL((k_bank_solve<32, T>), dim3(m.nbanks), dim3(128), 0, c.stream, inv, R, Z, ctrl, skip);
+        hipLaunchKernelGGL(k_bank_solve32<T>, dim3(m.nbanks), dim3(128), 0, c.stream, inv, R, Z, ctrl, skip);
     SGIPC_LAUNCH_CHECK();
     prof_end(c, PROF_MAS_SOLVE);
 }
@@ -1706,9 +1654,17 @@ static void solve_top_t(Ctx& c, const void* inv, const float* dsc, T* R, T* Z, c
     MasState& m = c.mas;
     const int top_bank0 = m.L >= 4 ? m.level_size_h[7] / m.bank : m.nbanks;
     prof_begin(c, PROF_MAS_SOLVE);
-    hipLaunchKernelGGL((k_mas_solve_top<T, H>), dim3(1 + div_up(top_bank0, kCW)), dim3(kCT), 0, c.stream, m.L,
-                       (const int*)m.level_size.p, (const int*)m.going_next.p, (const unsigned*)m.comp_mask.p,
-                       top_bank0, m.nbanks, inv, dsc, R, Z, ctrl, skip);
+    auto launch = [&](auto kern, int nb) {
+        hipLaunchKernelGGL(kern, dim3(1 + div_up(top_bank0, kCW * nb)), dim3(kCT), 0, c.stream, m.L,
+                           (const int*)m.level_size.p, (const int*)m.going_next.p, (const unsigned*)m.comp_mask.p,
+                           top_bank0, m.nbanks, inv, dsc, R, Z, ctrl, skip);
+    };
+    // Two banks per wavefront once one each would not be resident at once
+    // (256 CUs x 32 wavefronts): 10,359 FP32 banks 10.2 -> 9.7 us.  FP64 banks
+    // hold 24 more registers and gain nothing (17.2, 17.4 us); few banks lose
+    // the second one's latency.
+    if (sizeof(T) == 4 && top_bank0 > 8192) launch(k_mas_solve_top<T, H, sizeof(T) == 4 ? 2 : 1>, 2);
+    else launch(k_mas_solve_top<T, H, 1>, 1);
     SGIPC_LAUNCH_CHECK();
     prof_end(c, PROF_MAS_SOLVE);
 }

@@ -158,9 +158,11 @@ __global__ void __launch_bounds__(kCollectThreads) k_collect_dot(int nb, const V
         if (row < nb) load_x3(r, row, rv);
     };
     int row = blockIdx.x * kCollectThreads + threadIdx.x;
+    const int stopped = ctrl[C_STOP];
+    Share<4, kCollectThreads> test;  // the stop test's partials (rule < 0: none)
+    test.take(rule == 0 ? part_rz_prev : part_rr, rule == 0 ? np_rz : rule > 0 ? np_rr : 0);
     fetch(row);
-    const double share = stop_share(rule, part_rz_prev, np_rz, part_rr, np_rr);
-    if (ctrl[C_STOP]) {
+    if (stopped) {
         if (hp && blockIdx.x == 0 && threadIdx.x == 0) publish_progress(ctrl, sc, hp, hq);
         return;
     }
@@ -207,7 +209,7 @@ __global__ void __launch_bounds__(kCollectThreads) k_collect_dot(int nb, const V
         fetch(row + gridDim.x * kCollectThreads);
     }
     constexpr int NW = kCollectThreads / 64;
-    wave_sums_put(share, sh);
+    wave_sums_put(test.sum(), sh);
     wave_sums_put(v, sh + NW);
     __syncthreads();
     const bool stop = stop_test_sum(rule, wave_sums_total<NW>(sh), sc, ctrl);
@@ -281,21 +283,21 @@ __global__ void __launch_bounds__(kFT) k_spmv_pap_full(int nb, int R, int nchunk
     const int task = t / g, sub = t & (g - 1);  // this thread's row component of the chunk
     const int row = task / 3;
     // loads that depend on nothing: the first chunk's row pointers, the dots
-    double rn, ro;
+    const int stopped = ctrl[C_STOP], iter = ctrl[C_ITER], maxit = ctrl[C_MAXIT];
+    Share<4, kFT> rn, ro;
+    rn.take(rz_last, np_rz);
+    ro.take(rz_prev, np_rz);
     int ev = 0;
     if (w.first < w.end && t <= R) ev = eptr[min(w.first * R + t, nb)];
-    rn = strided_share<4>(rz_last, np_rz);
-    ro = strided_share<4>(rz_prev, np_rz);
-    if (ctrl[C_STOP]) return;
-    const int iter = ctrl[C_ITER];
-    if (iter >= ctrl[C_MAXIT]) {
-        if (blockIdx.x == 0 && t == 0) { ctrl[C_NOCONV] = 1; ctrl[C_STOP] = ctrl[C_MAXIT]; }
+    if (stopped) return;
+    if (iter >= maxit) {
+        if (blockIdx.x == 0 && t == 0) { ctrl[C_NOCONV] = 1; ctrl[C_STOP] = maxit; }
         return;
     }
     const bool first = iter == 1;
     // the waves' sums meet at the first chunk's barrier
-    wave_sums_put(rn, sh);
-    wave_sums_put(ro, sh + kFT / 64);
+    wave_sums_put(rn.sum(), sh);
+    wave_sums_put(ro.sum(), sh + kFT / 64);
     double be = 0.0, contrib = 0.0;
     for (int ch = w.first; ch < w.end; ch += w.step) {
         const int r0 = ch * R, nr = min(R, nb - r0);

@@ -43,25 +43,31 @@ __device__ inline void block_sum_all2(double& a, double& b, double* sh) {
     b = sb;
 }
 
-// This thread's strided share of np partials, U of them in flight together (a
-// loop of dependent load and add takes one round trip each).  Loads past the
-// end are clamped to the last partial: U should not be far above np / threads.
-template <int U>
-__device__ inline double strided_share(const double* __restrict__ part, int np) {
-    double v = 0.0;
-    for (int i = threadIdx.x; i < np; i += U * blockDim.x) {
-        double q[U];
+// A thread's strided share of np partials (workgroup of NT threads): take()
+// issues the loads of its first U partials, sum() adds them up -- and any
+// further ones -- in order.  Between the two, other loads can be issued (a loop
+// of dependent load and add takes one round trip each).  Loads past the end
+// are clamped to the last partial: U should not be far above np / NT.
+template <int U, int NT>
+struct Share {
+    const double* p;
+    int np;
+    double q[U];
+    __device__ inline void take(const double* __restrict__ part, int n) {
+        p = part;
+        np = n;
 #pragma unroll
-        for (int k = 0; k < U; ++k) {
-            const int j = i + k * (int)blockDim.x;
-            q[k] = part[min(j, np - 1)];
-        }
+        for (int k = 0; k < U; ++k) q[k] = part[max(0, min((int)threadIdx.x + k * NT, n - 1))];
+    }
+    __device__ inline double sum() const {
+        double v = 0.0;
 #pragma unroll
         for (int k = 0; k < U; ++k)
-            if (i + k * (int)blockDim.x < np) v += q[k];
+            if ((int)threadIdx.x + k * NT < np) v += q[k];
+        for (int i = (int)threadIdx.x + U * NT; i < np; i += NT) v += p[i];
+        return v;
     }
-    return v;
-}
+};
 
 // The wavefronts' sums of v meet in sh[0 .. waves) (written here; read them
 // after a barrier with wave_sums_total, in wavefront order)
@@ -107,13 +113,6 @@ constexpr int kLevelBatch = 8;    // MAS levels whose loads are in flight togeth
 // follows the x/r update (so no block depends on another's flag write):
 // rule 0 (reference): |rz_prev| <= tol * rz0 on the pre-update rz;
 // rule 1: ||r|| <= tol * ||b|| on the updated residual.  rule < 0: none.
-// This thread's share of the stop test's partial sum (the strided part of
-// sum_partials), so a kernel can issue its loads early and reduce late.
-__device__ inline double stop_share(int rule, const double* __restrict__ part_rz_prev, int np_rz,
-                                    const double* __restrict__ part_rr, int np_rr) {
-    return rule == 0 ? strided_share<4>(part_rz_prev, np_rz) : rule > 0 ? strided_share<4>(part_rr, np_rr) : 0.0;
-}
-
 // Stop test from the sum of the shares: rule 0 |r.z| <= tol * r0.z0 (previous r.z),
 // rule 1 ||r|| <= tol * ||b||; block 0 records the progress and the stop.
 __device__ inline bool stop_test_sum(int rule, double sum, double* __restrict__ sc, int* __restrict__ ctrl) {
@@ -138,8 +137,8 @@ __device__ inline bool stop_test(int rule, const double* __restrict__ part_rz_pr
                                  const double* __restrict__ part_rr, int np_rr, double* __restrict__ sc,
                                  int* __restrict__ ctrl, double* sh) {
     if (rule < 0) return false;
-    const double sum = block_sum_all(stop_share(rule, part_rz_prev, np_rz, part_rr, np_rr), sh);
-    return stop_test_sum(rule, sum, sc, ctrl);
+    const double* part = rule == 0 ? part_rz_prev : part_rr;
+    return stop_test_sum(rule, sum_partials(part, rule == 0 ? np_rz : np_rr, sh), sc, ctrl);
 }
 
 // Progress words for the host's pinned-memory polling: the stop and

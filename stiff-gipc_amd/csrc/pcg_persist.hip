@@ -24,6 +24,7 @@
 // level order), so results repeat bitwise.
 #include "spmv_sym.hpp"
 #include "pcg_dev.hpp"
+#include "bank_solve.hpp"
 #include <algorithm>
 #include <numeric>
 #include <type_traits>
@@ -31,20 +32,6 @@
 namespace sgipc {
 namespace {
 
-typedef __attribute__((address_space(1))) const void* pg_gptr_t;
-typedef __attribute__((address_space(3))) void* pg_lptr_t;
-
-constexpr int kSolveWaves = 8;  // wavefronts that solve banks (one LDS staging area each)
-
-__device__ inline float bcast_lane(float v, int j) {
-    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), j));
-}
-__device__ inline double bcast_lane(double v, int j) {
-    const long long b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_readlane((int)(b & 0xffffffffll), j);
-    const int hi = __builtin_amdgcn_readlane((int)(b >> 32), j);
-    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
-}
 __device__ inline unsigned pg_ltmask(int lane) { return lane >= 32 ? 0xffffffffu : ((1u << lane) - 1u); }
 
 // component sum of the bank-aligned group in LDS (the restriction's sum):
@@ -110,7 +97,7 @@ struct SceneSolver {
     int s, r0, r1;
     double* sh;   // NTH / 64 doubles
     T (*sv)[NTH];
-    void* stage;  // kSolveWaves staging areas
+    T* stage;     // kBankLds values per wavefront
 
     __device__ double block_sum(double v) { return block_sum_all(v, sh); }
 
@@ -159,36 +146,16 @@ struct SceneSolver {
     }
 
     // one bank of 48 rows by one wavefront, R of the scene's own nodes only
-    __device__ void bank_solve(int bank, void* area) {
-        constexpr int D = 48, NP = D * (D + 1) / 2;
-        using V4 = typename std::conditional<sizeof(T) == 8, double2, float4>::type;
-        constexpr int NV = NP * (int)sizeof(T) / 16;
-        constexpr int PER = (NV + 63) / 64;
-        V4* As = static_cast<V4*>(area);
+    __device__ void bank_solve(int bank, T* area) {
+        constexpr int D = 48;
         const int i = threadIdx.x & 63;
         const int node = bank * 16 + min(i, D - 1) / 3;
         const bool own = i < D && a.node_scene[node] == s;
-        const T rv = own ? a.R[(size_t)bank * D + i] : (T)0;
-        const V4* src = reinterpret_cast<const V4*>(a.inv + (size_t)bank * NP);
-#pragma unroll
-        for (int k = 0; k < PER; ++k) {
-            const int q0 = k * 64;
-            __builtin_amdgcn_global_load_lds((pg_gptr_t)(src + min(q0 + i, NV - 1)), (pg_lptr_t)(As + q0), 16, 0, 0);
-        }
-        __builtin_amdgcn_s_waitcnt(0);
-        __builtin_amdgcn_wave_barrier();
-        const T* A = reinterpret_cast<const T*>(As);
-        T acc = 0;
-        if (i < D) {
-            int idx = i;
-#pragma unroll 8
-            for (int j = 0; j < D; ++j) {
-                acc += A[idx] * bcast_lane(rv, j);
-                idx += (j < i) ? (D - 1 - j) : 1;
-            }
-        }
-        if (own) a.Z[(size_t)bank * D + i] = acc;
-        __builtin_amdgcn_wave_barrier();
+        BankSolve<T, T> B;
+        B.load(a.inv, nullptr, bank, i);
+        B.rv = own ? a.R[(size_t)bank * D + i] : (T)0;
+        const T z = B.solve(area, i);
+        if (own) a.Z[(size_t)bank * D + i] = z;
     }
 
     // z = M^-1 r on the scene (r holds the residual), returns r.z
@@ -245,10 +212,9 @@ struct SceneSolver {
         }
         // bank solves of every level (the banks holding the scene's nodes)
         const int wv = t >> 6;
-        if (wv < kSolveWaves) {
-            using V4 = typename std::conditional<sizeof(T) == 8, double2, float4>::type;
-            constexpr int PER = ((48 * 49 / 2) * (int)sizeof(T) / 16 + 63) / 64;
-            void* area = static_cast<V4*>(stage) + (size_t)wv * PER * 64;
+        {
+            constexpr int kSolveWaves = NTH / 64;
+            T* area = stage + kBankLds * wv;
             int k = wv;
             for (int l = 0; l < L; ++l) {
                 const int b0 = lo[l] / 16, b1 = (hi[l] + 15) / 16;  // banks [b0, b1)
@@ -378,11 +344,9 @@ struct SceneSolver {
 
 template <int NTH, int G, typename V, typename MV, typename T>
 __global__ void __launch_bounds__(NTH) k_pcg_persist(PArgs<V, MV, T> a) {
-    using V4 = typename std::conditional<sizeof(T) == 8, double2, float4>::type;
-    constexpr int PER = ((48 * 49 / 2) * (int)sizeof(T) / 16 + 63) / 64;
     __shared__ double sh[NTH / 64];
     __shared__ T sv[3][NTH];
-    __shared__ V4 stage[kSolveWaves * PER * 64];
+    __shared__ T stage[NTH / 64 * kBankLds];
     __shared__ int take;
     for (;;) {
         __syncthreads();

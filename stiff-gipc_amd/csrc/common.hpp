@@ -84,4 +84,43 @@ inline void fill(T* p, T v, long long n, hipStream_t s) {
     SGIPC_LAUNCH_CHECK();
 }
 
+// Several fills of 4-byte words in one launch (a launch costs about 2 us)
+struct FillRanges {
+    static constexpr int kMax = 6;
+    unsigned* p[kMax];
+    unsigned v[kMax];
+    long long end[kMax];  // running total of words
+    int n = 0;
+    template <typename T>
+    FillRanges& add(T* q, unsigned word, long long count) {
+        static_assert(sizeof(T) % 4 == 0, "whole words");
+        p[n] = reinterpret_cast<unsigned*>(q);
+        v[n] = word;
+        end[n] = (n ? end[n - 1] : 0) + count * (long long)(sizeof(T) / 4);
+        ++n;
+        return *this;
+    }
+};
+static __global__ void k_fill_ranges(FillRanges f) {
+    const long long stride = (long long)gridDim.x * blockDim.x;
+    for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < f.end[f.n - 1]; i += stride) {
+        long long base = 0;
+#pragma unroll
+        for (int k = 0; k < FillRanges::kMax; ++k) {
+            if (k >= f.n) break;
+            if (i < f.end[k]) {
+                f.p[k][i - base] = f.v[k];
+                break;
+            }
+            base = f.end[k];
+        }
+    }
+}
+inline void fill_ranges(const FillRanges& f, hipStream_t s) {
+    if (f.n == 0 || f.end[f.n - 1] <= 0) return;
+    const long long blocks = (f.end[f.n - 1] + 1023) / 1024;
+    hipLaunchKernelGGL(k_fill_ranges, dim3((unsigned)(blocks > 16384 ? 16384 : blocks)), dim3(256), 0, s, f);
+    SGIPC_LAUNCH_CHECK();
+}
+
 }  // namespace sgipc

@@ -1249,6 +1249,243 @@ __global__ void k_l1_ranges(int nb0, int B, const int* __restrict__ prefix0, con
     }
 }
 
+// ---- the whole numbering in one workgroup -----------------------------------
+// Systems of up to kSmallN vertices, kSmallM slots, kSmallList neighbours and
+// kSmallPairs contact pairs: every table of the hierarchy in one launch, with
+// the integers of the level-by-level kernels above.  Those take seven or eight
+// launches a level, 2 to 5 us each however small the level; here the neighbour
+// lists (16-bit), the masks and the vertices' nodes of the current level live
+// in LDS, a phase ends with a barrier, and only the tables go to memory.
+// Latency-bound: 20 us at 125 vertices and 59 us at 1331, where the launches
+// it replaces (about 40) took 90 and 150 us of a step.  Above 2048 vertices
+// (two per thread) one CU is too few: 369 us against 170 at 5488 vertices, with
+// the lists read from memory because they no longer fit LDS.
+constexpr int kSmallT = 1024;
+constexpr int kSmallN = 2048;
+constexpr int kSmallM = 4096;
+constexpr int kSmallPairs = 4096;
+constexpr int kSmallList = 40960;       // 80 KB of the 112 KB of LDS in use
+constexpr int kSmallV = kSmallN / kSmallT;
+static_assert(kSmallM / 16 <= kSmallT, "one scan step holds the banks of a level");
+
+struct SmallTables {
+    int M, Mpad, n, B, L, node_offset, npairs, nb1_cap, nlist_len;
+    const int *part_map, *real_map;
+    const unsigned *nstart, *nnum, *nlist;
+    const int4* pairs;
+    int *ls, *going_next, *coarse_space, *coarse_table, *node_of, *prefix0, *psum0, *l1lo, *l1hi, *own_lo, *own_hi;
+    unsigned *fine_mask, *comp_mask;
+    SlotNode* slot_node;
+    size_t going_cap;
+};
+
+// exclusive scan of cnt entries (at most kSmallT) of v in LDS, in place; returns the total
+__device__ inline int small_scan(int* v, int cnt, int* sh) {
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+    const int mine = t < cnt ? v[t] : 0;
+    int incl = mine;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const int u = __shfl_up(incl, off, 64);
+        if (lane >= off) incl += u;
+    }
+    if (lane == 63) sh[w] = incl;
+    __syncthreads();
+    int before = 0, total = 0;
+    for (int q = 0; q < kSmallT / 64; ++q) {
+        if (q < w) before += sh[q];
+        total += sh[q];
+    }
+    if (t < cnt) v[t] = before + incl - mine;
+    __syncthreads();
+    return total;
+}
+
+__global__ void __launch_bounds__(kSmallT) k_small_tables(SmallTables A) {
+    __shared__ unsigned fm[kSmallN];    // level-0 masks by vertex
+    __shared__ unsigned nm[kSmallN];    // this level's masks, then next ids, by node
+    __shared__ int cs[kSmallN];         // the vertices' slots, then their nodes at this level
+    __shared__ unsigned short nl[kSmallList];
+    __shared__ unsigned sm[kSmallT];
+    __shared__ int pre[kSmallT];        // components per bank, then their scan
+    __shared__ int sh[kSmallT / 64];
+    const int t = threadIdx.x, n = A.n, M = A.M, B = A.B, L = A.L;
+    const int lb = __ffs(B) - 1;  // ids are divided by shifts
+    const int lane = t & (B - 1), bbase = t - lane;
+    for (size_t i = t; i < A.going_cap; i += kSmallT) A.going_next[i] = 0;
+    for (int i = t; i < 2 * (L + 2); i += kSmallT) A.ls[i] = 0;
+    for (int i = t; i <= A.nb1_cap; i += kSmallT) {
+        A.l1lo[i] = M >> lb;
+        A.l1hi[i] = 0;
+        A.own_lo[i] = 0x7fffffff;
+        A.own_hi[i] = 0;
+    }
+    unsigned nst[kSmallV], nnn[kSmallV];  // neighbour ranges of this thread's vertices
+#pragma unroll
+    for (int j = 0; j < kSmallV; ++j) {
+        const int v = t + j * kSmallT;
+        nst[j] = v < n ? A.nstart[v] : 0u;
+        nnn[j] = v < n ? A.nnum[v] : 0u;
+        if (v < n) cs[v] = A.real_map[v];
+    }
+    for (int i = t; i < A.nlist_len; i += kSmallT) nl[i] = (unsigned short)A.nlist[i];
+    __syncthreads();  // the lists are whole; none of the cleared tables is written before
+    // the vertex's own bit and its neighbours' in the same bank
+    auto bank_mask = [&](int v, unsigned st, unsigned nn) {
+        const int c = cs[v], bank = c >> lb;
+        unsigned msk = 1u << (c & (B - 1));
+        for (unsigned i = 0; i < nn; ++i) {
+            const int cu = cs[nl[st + i]];
+            if ((cu >> lb) == bank) msk |= 1u << (cu & (B - 1));
+        }
+        return msk;
+    };
+#pragma unroll
+    for (int j = 0; j < kSmallV; ++j) {
+        const int v = t + j * kSmallT;
+        if (v < n) fm[v] = bank_mask(v, nst[j], nnn[j]);
+    }
+    __syncthreads();
+    // contact pairs: every two nodes of a pair that share a bank are connected
+    auto collide = [&](bool level0, unsigned* dst) {
+        for (int p = t; p < A.npairs; p += kSmallT) {
+            int v[4], cp[4];
+            const int cnt = decode_pair(A.pairs[p], A.node_offset, v);
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                cp[i] = (i >= cnt || v[i] < 0 || v[i] >= n) ? -1 : cs[v[i]];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                unsigned msk = 0u;
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    if (j != i && cp[i] >= 0 && cp[j] >= 0 && cp[i] != cp[j] && (cp[i] >> lb) == (cp[j] >> lb))
+                        msk |= 1u << (cp[j] & (B - 1));
+                if (msk) atomicOr(dst + (level0 ? v[i] : cp[i]), msk);
+            }
+        }
+        __syncthreads();
+    };
+    collide(true, fm);
+    // closure in every bank and its component count; fm is read and written
+    // by the vertex's own thread only
+    const int nb0 = M >> lb;
+    for (int s0 = 0; s0 < M; s0 += kSmallT) {
+        const int s = s0 + t, v = s < M ? A.part_map[s] : -1;
+        sm[t] = v >= 0 ? fm[v] : 0u;
+        __syncthreads();
+        unsigned cl = 0u;
+        if (v >= 0) {
+            cl = closure(sm[t], lane, sm + bbase);
+            fm[v] = cl;
+            A.fine_mask[v] = cl;
+        }
+        const unsigned long long lead = __ballot(v >= 0 && (cl & ltmask(lane)) == 0u);
+        if (lane == 0 && s < M) {
+            const int c = __popcll((lead >> (t & 63)) & ((1ull << B) - 1ull));
+            pre[s >> lb] = c;
+            A.prefix0[s >> lb] = c;
+        }
+        __syncthreads();
+    }
+    int total = small_scan(pre, nb0, sh);
+    // level-1 nodes
+    int begin = A.Mpad, number = total;
+    for (int s0 = 0; s0 < M; s0 += kSmallT) {
+        const int s = s0 + t, v = s < M ? A.part_map[s] : -1;
+        const unsigned f = v >= 0 ? fm[v] : 0u;
+        const unsigned long long lead = __ballot(v >= 0 && (f & ltmask(lane)) == 0u);
+        if (v >= 0) {
+            const unsigned elected = (unsigned)((lead >> ((t & 63) - lane)) & ((1ull << B) - 1ull));
+            const int id = __popc(elected & ltmask(lowbit(f))) + pre[s >> lb];
+            cs[v] = id;
+            A.coarse_space[v] = id;
+            A.going_next[v] = id + A.Mpad;
+            A.slot_node[s] = SlotNode{v, id, f, 0u};
+            A.node_of[v] = A.real_map[v];
+            A.node_of[(size_t)n + v] = begin + id;  // (L >= 2 always)
+            A.coarse_table[6 * (size_t)v] = begin + id;
+            for (int l = L - 1; l < 6; ++l) A.coarse_table[6 * (size_t)v + l] = 0;
+            // vertices owned by the level-1 bank of the level-0 bank's first node
+            const int f1 = pre[s >> lb] >> lb;
+            atomicMin(A.own_lo + f1, v);
+            atomicMax(A.own_hi + f1, v + 1);
+        } else if (s < M) {
+            A.slot_node[s] = SlotNode{-1, -1, 0u, 0u};
+        }
+        if (lane == 0 && s < M) {
+            const int first = pre[s >> lb], last = ((s >> lb) + 1 < nb0 ? pre[(s >> lb) + 1] : total) - 1;
+            A.psum0[s >> lb] = first;
+            for (int b = first >> lb; first <= last && b <= last >> lb; ++b) {
+                atomicMin(A.l1lo + b, s >> lb);
+                atomicMax(A.l1hi + b, (s >> lb) + 1);
+            }
+        }
+    }
+    if (t == 0) {
+        A.psum0[nb0] = total;
+        A.ls[2] = total;
+        A.ls[3] = A.Mpad;
+    }
+    for (int level = 1; level < L; ++level) {
+        __syncthreads();
+        for (int c = t; c < number; c += kSmallT) nm[c] = 0u;
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < kSmallV; ++j) {
+            const int v = t + j * kSmallT;
+            if (v < n) atomicOr(nm + cs[v], bank_mask(v, nst[j], nnn[j]));
+        }
+        __syncthreads();
+        collide(false, nm);
+        const int nbk = (number + B - 1) >> lb, pad = nbk * B;
+        for (int c0 = 0; c0 < number; c0 += kSmallT) {
+            const int c = c0 + t;
+            const bool valid = c < number;
+            sm[t] = valid ? ((1u << lane) | nm[c]) : 0u;
+            __syncthreads();
+            unsigned cl = 0u;
+            if (valid) {
+                cl = closure(sm[t], lane, sm + bbase);
+                nm[c] = cl;
+                A.comp_mask[(size_t)begin + c] = cl;
+            }
+            const unsigned long long lead = __ballot(valid && (cl & ltmask(lane)) == 0u);
+            if (lane == 0 && valid) pre[c >> lb] = __popcll((lead >> (t & 63)) & ((1ull << B) - 1ull));
+            __syncthreads();
+        }
+        total = small_scan(pre, nbk, sh);
+        for (int c0 = 0; c0 < number; c0 += kSmallT) {
+            const int c = c0 + t;
+            const bool valid = c < number;
+            const unsigned cm = valid ? nm[c] : 0u;
+            const unsigned long long lead = __ballot(valid && (cm & ltmask(lane)) == 0u);
+            if (valid) {
+                const unsigned elected = (unsigned)((lead >> ((t & 63) - lane)) & ((1ull << B) - 1ull));
+                const int id = __popc(elected & ltmask(lowbit(cm))) + pre[c >> lb];
+                nm[c] = (unsigned)id;
+                if ((size_t)begin + c < A.going_cap) A.going_next[(size_t)begin + c] = id + begin + pad;
+            }
+        }
+        __syncthreads();
+        begin += pad;
+        for (int v = t; v < n; v += kSmallT) {
+            const int id = (int)nm[cs[v]];
+            cs[v] = id;
+            A.coarse_space[(size_t)level * n + v] = id;
+            if (level + 1 < L) {
+                A.node_of[(size_t)(level + 1) * n + v] = begin + id;
+                A.coarse_table[6 * (size_t)v + level] = begin + id;
+            }
+        }
+        number = total;
+        if (t == 0) {
+            A.ls[2 * (level + 1)] = total;
+            A.ls[2 * (level + 1) + 1] = begin;
+        }
+    }
+}
+
 int num_levels(int nn, int B) {
     int nLevel = 1;
     int levelSz = (nn + B - 1) / B * B;
@@ -1328,6 +1565,7 @@ void mas_set_topology(Ctx& c, int n, int node_offset, const unsigned* nstart, co
         if (real_map[v] <= real_map[v - 1]) { m.slot_ordered = false; break; }
     m.node_offset = node_offset;
     m.M = M;
+    m.nlist_len = nlist_len;
     m.L = num_levels(std::max(M, n), bank);
     int Mpad = (M + bank - 1) / bank * bank;
     m.going_cap = (size_t)Mpad + (size_t)m.L * ((size_t)n + bank) + bank;
@@ -1370,55 +1608,70 @@ void mas_build(Ctx& c, int sub_offset, int sub_nb, const int* pairs, int npairs)
     if (sub_nb != n) throw arg_error("MAS build: subsystem block count differs from the MAS topology");
     m.ready = false;
     int* ls = m.level_size.p;
-    fill<int>(ls, 0, 2LL * (L + 2), s);
-    fill<int>(m.going_next.p, 0, (long long)m.going_cap, s);
-    // level 0
-    hipLaunchKernelGGL(k_l0_masks, dim3(div_up(M, 256)), dim3(256), 0, s, M, B, m.part_map.p, m.real_map.p, m.nstart.p,
-                       m.nnum.p, m.nlist.p, m.fine_mask.p);
-    SGIPC_LAUNCH_CHECK();
-    if (npairs > 0) {
-        hipLaunchKernelGGL(k_collision, dim3(div_up(npairs, 256)), dim3(256), 0, s, npairs, (const int4*)pairs,
-                           m.node_offset, n, B, -1, m.real_map.p, m.coarse_space.p, m.fine_mask.p);
+    const int nb1_cap = div_up(n, B);
+    int* l1lo = m.l1lo.reserve((size_t)nb1_cap + 2);
+    int* l1hi = m.l1hi.reserve((size_t)nb1_cap + 2);
+    int* vlo = m.own_lo.reserve((size_t)nb1_cap + 2);
+    int* vhi = m.own_hi.reserve((size_t)nb1_cap + 2);
+    const bool small = n > 0 && n <= kSmallN && M <= kSmallM && m.nlist_len <= kSmallList && npairs <= kSmallPairs;
+    if (small) {
+        hipLaunchKernelGGL(k_small_tables, dim3(1), dim3(kSmallT), 0, s,
+                           (SmallTables{M, Mpad, n, B, L, m.node_offset, npairs, nb1_cap, m.nlist_len, m.part_map.p, m.real_map.p,
+                                        m.nstart.p, m.nnum.p, m.nlist.p, (const int4*)pairs, ls, m.going_next.p,
+                                        m.coarse_space.p, m.coarse_table.p, m.node_of.p, m.prefix0.p, m.psum0.p, l1lo,
+                                        l1hi, vlo, vhi, m.fine_mask.p, m.comp_mask.p, m.slot_node.p, m.going_cap}));
         SGIPC_LAUNCH_CHECK();
-    }
-    hipLaunchKernelGGL(k_l0_closure, dim3(div_up(M, kTB)), dim3(kTB), 0, s, M, B, m.part_map.p, m.fine_mask.p,
-                       m.prefix0.p);
-    SGIPC_LAUNCH_CHECK();
-    int* tot = c.dev_int.reserve(8);
-    exclusive_scan(c, m.prefix0.p, m.psum0.p, M / B, tot + 6, s);
-    hipLaunchKernelGGL(k_set_level_size, dim3(1), dim3(1), 0, s, ls, 0, tot + 6, B, Mpad);
-    SGIPC_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_level1, dim3(div_up(M, kTB)), dim3(kTB), 0, s, M, Mpad, n, B, m.part_map.p, m.fine_mask.p,
-                       m.psum0.p, m.coarse_space.p, m.going_next.p, m.slot_node.p);
-    SGIPC_LAUNCH_CHECK();
-    const int nmax = n;  // level-local node count never exceeds n
-    for (int level = 1; level < L; ++level) {
-        fill<unsigned>(m.next_mask.p, 0u, (long long)nmax + B, s);
-        hipLaunchKernelGGL(k_lx_masks, dim3(div_up(n, 256)), dim3(256), 0, s, n, B, level, m.nstart.p, m.nnum.p,
-                           m.nlist.p, m.coarse_space.p, m.next_mask.p);
+    } else {
+        fill<int>(ls, 0, 2LL * (L + 2), s);
+        fill<int>(m.going_next.p, 0, (long long)m.going_cap, s);
+        // level 0
+        hipLaunchKernelGGL(k_l0_masks, dim3(div_up(M, 256)), dim3(256), 0, s, M, B, m.part_map.p, m.real_map.p, m.nstart.p,
+                           m.nnum.p, m.nlist.p, m.fine_mask.p);
         SGIPC_LAUNCH_CHECK();
         if (npairs > 0) {
             hipLaunchKernelGGL(k_collision, dim3(div_up(npairs, 256)), dim3(256), 0, s, npairs, (const int4*)pairs,
-                               m.node_offset, n, B, level, m.real_map.p, m.coarse_space.p, m.next_mask.p);
+                               m.node_offset, n, B, -1, m.real_map.p, m.coarse_space.p, m.fine_mask.p);
             SGIPC_LAUNCH_CHECK();
         }
-        int nbk = div_up(nmax, B);
-        hipLaunchKernelGGL(k_lx_closure, dim3(div_up((long long)nbk * B, kTB)), dim3(kTB), 0, s, nbk * B, B, level, ls,
-                           m.next_mask.p, m.next_prefix.p, m.comp_mask.p);
+        hipLaunchKernelGGL(k_l0_closure, dim3(div_up(M, kTB)), dim3(kTB), 0, s, M, B, m.part_map.p, m.fine_mask.p,
+                           m.prefix0.p);
         SGIPC_LAUNCH_CHECK();
-        exclusive_scan(c, m.next_prefix.p, m.next_psum.p, nbk, tot + 6, s);
-        hipLaunchKernelGGL(k_set_level_size, dim3(1), dim3(1), 0, s, ls, level, tot + 6, B, 0);
+        int* tot = c.dev_int.reserve(8);
+        exclusive_scan(c, m.prefix0.p, m.psum0.p, M / B, tot + 6, s);
+        hipLaunchKernelGGL(k_set_level_size, dim3(1), dim3(1), 0, s, ls, 0, tot + 6, B, Mpad);
         SGIPC_LAUNCH_CHECK();
-        hipLaunchKernelGGL(k_lx_renumber, dim3(div_up((long long)nbk * B, kTB)), dim3(kTB), 0, s, B, level, ls,
-                           m.next_mask.p, m.next_psum.p, m.going_next.p, m.going_cap);
+        hipLaunchKernelGGL(k_level1, dim3(div_up(M, kTB)), dim3(kTB), 0, s, M, Mpad, n, B, m.part_map.p, m.fine_mask.p,
+                           m.psum0.p, m.coarse_space.p, m.going_next.p, m.slot_node.p);
         SGIPC_LAUNCH_CHECK();
-        hipLaunchKernelGGL(k_next_table, dim3(div_up(n, 256)), dim3(256), 0, s, n, level, m.coarse_space.p,
-                           m.next_mask.p);
+        const int nmax = n;  // level-local node count never exceeds n
+        for (int level = 1; level < L; ++level) {
+            fill<unsigned>(m.next_mask.p, 0u, (long long)nmax + B, s);
+            hipLaunchKernelGGL(k_lx_masks, dim3(div_up(n, 256)), dim3(256), 0, s, n, B, level, m.nstart.p, m.nnum.p,
+                               m.nlist.p, m.coarse_space.p, m.next_mask.p);
+            SGIPC_LAUNCH_CHECK();
+            if (npairs > 0) {
+                hipLaunchKernelGGL(k_collision, dim3(div_up(npairs, 256)), dim3(256), 0, s, npairs, (const int4*)pairs,
+                                   m.node_offset, n, B, level, m.real_map.p, m.coarse_space.p, m.next_mask.p);
+                SGIPC_LAUNCH_CHECK();
+            }
+            int nbk = div_up(nmax, B);
+            hipLaunchKernelGGL(k_lx_closure, dim3(div_up((long long)nbk * B, kTB)), dim3(kTB), 0, s, nbk * B, B, level, ls,
+                               m.next_mask.p, m.next_prefix.p, m.comp_mask.p);
+            SGIPC_LAUNCH_CHECK();
+            exclusive_scan(c, m.next_prefix.p, m.next_psum.p, nbk, tot + 6, s);
+            hipLaunchKernelGGL(k_set_level_size, dim3(1), dim3(1), 0, s, ls, level, tot + 6, B, 0);
+            SGIPC_LAUNCH_CHECK();
+            hipLaunchKernelGGL(k_lx_renumber, dim3(div_up((long long)nbk * B, kTB)), dim3(kTB), 0, s, B, level, ls,
+                               m.next_mask.p, m.next_psum.p, m.going_next.p, m.going_cap);
+            SGIPC_LAUNCH_CHECK();
+            hipLaunchKernelGGL(k_next_table, dim3(div_up(n, 256)), dim3(256), 0, s, n, level, m.coarse_space.p,
+                               m.next_mask.p);
+            SGIPC_LAUNCH_CHECK();
+        }
+        hipLaunchKernelGGL(k_aggregate, dim3(div_up(n, 256)), dim3(256), 0, s, n, L, m.real_map.p, m.going_next.p,
+                           m.coarse_table.p, m.node_of.p);
         SGIPC_LAUNCH_CHECK();
     }
-    hipLaunchKernelGGL(k_aggregate, dim3(div_up(n, 256)), dim3(256), 0, s, n, L, m.real_map.p, m.going_next.p,
-                       m.coarse_table.p, m.node_of.p);
-    SGIPC_LAUNCH_CHECK();
     SGIPC_HIP(hipMemcpyAsync(m.level_size_h.data(), ls, sizeof(int) * 2 * (L + 1), hipMemcpyDeviceToHost, s));
     SGIPC_HIP(hipStreamSynchronize(s));
     m.total = m.level_size_h[2 * L + 1];
@@ -1429,21 +1682,38 @@ void mas_build(Ctx& c, int sub_offset, int sub_nb, const int* pairs, int npairs)
     m.bank_upper.reserve((size_t)m.nbanks * npack * 9);
     m.inv64.reserve((size_t)m.nbanks * (D * (D + 1) / 2));
     m.inv32.reserve((size_t)m.nbanks * (D * (D + 1) / 2));
-    // level-0 bank ranges of the level-1 banks (fused restriction)
+    // apply work vectors: allocated here so their addresses are stable for
+    // captured PCG graphs; padding entries stay zero (never written)
+    m.R64.reserve(3 * (size_t)m.total + 3);
+    m.Z64.reserve(3 * (size_t)m.total + 3);
+    m.R32.reserve(3 * (size_t)m.total + 3);
+    m.Z32.reserve(3 * (size_t)m.total + 3);
+    m.nb1 = div_up(m.level_size_h[2], B);
     {
+        // bank matrices and residuals to zero; level-0 bank ranges and owned
+        // vertices of the level-1 banks
+        FillRanges f;
+        f.add(m.bank_upper.p, 0u, (long long)m.nbanks * npack * 9).add(m.R64.p, 0u, 3LL * m.total + 3);
+        f.add(m.R32.p, 0u, 3LL * m.total + 3);
         const int nb0 = M / B;
-        m.nb1 = div_up(m.level_size_h[2], B);
-        int* lo = m.l1lo.reserve((size_t)m.nb1 + 1);
-        int* hi = m.l1hi.reserve((size_t)m.nb1 + 1);
-        fill<int>(lo, nb0, m.nb1 + 1, s);
-        fill<int>(hi, 0, m.nb1 + 1, s);
-        if (nb0 > 0) {
-            hipLaunchKernelGGL(k_l1_ranges, dim3(div_up(nb0, 256)), dim3(256), 0, s, nb0, B, m.prefix0.p, m.psum0.p,
-                               lo, hi);
-            SGIPC_LAUNCH_CHECK();
+        if (small) {
+            fill_ranges(f, s);
+        } else {
+            FillRanges g;
+            g.add(l1lo, (unsigned)nb0, m.nb1 + 1).add(l1hi, 0u, m.nb1 + 1).add(vlo, 0x7fffffffu, m.nb1 + 1);
+            g.add(vhi, 0u, m.nb1 + 1);
+            fill_ranges(f, s);
+            fill_ranges(g, s);
+            if (nb0 > 0) {
+                hipLaunchKernelGGL(k_l1_ranges, dim3(div_up(nb0, 256)), dim3(256), 0, s, nb0, B, m.prefix0.p,
+                                   m.psum0.p, l1lo, l1hi);
+                SGIPC_LAUNCH_CHECK();
+                hipLaunchKernelGGL(k_owned_vertices, dim3(div_up(nb0, 256)), dim3(256), 0, s, nb0, B, m.prefix0.p,
+                                   m.psum0.p, m.part_map.p, vlo, vhi);
+                SGIPC_LAUNCH_CHECK();
+            }
         }
     }
-    fill<double>(m.bank_upper.p, 0.0, (long long)m.nbanks * npack * 9, s);
     // The banked projection (16-vertex banks, vertex ids in slot order) sums
     // coarse levels in LDS with few atomics; every other case -- and the
     // deterministic mode -- uses the ordered projection, which sorts
@@ -1506,14 +1776,6 @@ void mas_build(Ctx& c, int sub_offset, int sub_nb, const int* pairs, int npairs)
             top_lvl = l;
         }
         const int win_levels = std::min(kProjWinLevels, top_lvl - 1);
-        const int nb0 = M / B;
-        int* vlo = m.own_lo.reserve((size_t)m.nb1 + 1);
-        int* vhi = m.own_hi.reserve((size_t)m.nb1 + 1);
-        fill<int>(vlo, 0x7fffffff, m.nb1, s);
-        fill<int>(vhi, 0, m.nb1, s);
-        hipLaunchKernelGGL(k_owned_vertices, dim3(div_up(nb0, 256)), dim3(256), 0, s, nb0, B, m.prefix0.p, m.psum0.p,
-                           m.part_map.p, vlo, vhi);
-        SGIPC_LAUNCH_CHECK();
         const int top_len = top_nb * kProjBank16;
         double* scratch = m.proj_scratch.reserve((size_t)m.nb1 * (top_len > 0 ? top_len : 1));
         auto launch = [&](auto kern) {
@@ -1566,14 +1828,6 @@ void mas_build(Ctx& c, int sub_offset, int sub_nb, const int* pairs, int npairs)
         SGIPC_LAUNCH_CHECK();
     }
     m.inv16_ok = half;
-    // apply work vectors: allocated here so their addresses are stable for
-    // captured PCG graphs; padding entries stay zero (never written)
-    m.R64.reserve(3 * (size_t)m.total + 3);
-    m.Z64.reserve(3 * (size_t)m.total + 3);
-    m.R32.reserve(3 * (size_t)m.total + 3);
-    m.Z32.reserve(3 * (size_t)m.total + 3);
-    fill<double>(m.R64.p, 0.0, 3LL * m.total + 3, s);
-    fill<float>(m.R32.p, 0.0f, 3LL * m.total + 3, s);
     m.ready = true;
 }
 

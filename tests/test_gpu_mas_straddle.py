@@ -114,3 +114,34 @@ def test_solves_repeat_bitwise_on_straddling_banks(scrambled_system):
             sys_.solve(tol=1e-6, stop_rule=capi.STOP_TRUE_REL, precision=prec, max_iter=2000)
             xs.append(sys_.dx.cpu().numpy().copy())
         assert np.array_equal(xs[0], xs[1]) and np.array_equal(xs[0], xs[2])
+
+
+@pytest.mark.parametrize("cells,boxes,bank", [(1, 1, 16), (2, 1, 32), (11, 1, 16), (11, 1, 32), (12, 1, 16),
+                                              (9, 2, 16), (9, 2, 32), (10, 2, 16)])
+def test_tables_and_apply_on_both_sides_of_the_one_workgroup_limit(torch_cuda, oracle, cells, boxes, bank):
+    """Up to 2048 vertices one workgroup numbers the whole hierarchy, above it
+    a few launches per level do: the integer tables equal the oracle's bit for
+    bit and the FP64 apply agrees to rounding (a 96-term bank product and its
+    inverse; 1e-11 is what the other apply tests hold), with and without
+    contacts, for the smallest meshes and just below and above the limit."""
+    from sgipc import capi, scene
+    from sgipc.system import NewtonSystem
+    print("case: mas tables", cells, boxes, bank, flush=True)
+    sc = (scene.cube_scene if boxes == 1 else scene.two_box_scene)(cells, seed=3, bank=bank)
+    s = NewtonSystem(sc, "cuda:0", precond=capi.PRECOND_MAS)
+    pairs = None
+    if boxes == 2:
+        s.setup_contacts(*scene.facing_contact_candidates(sc))
+        pairs = s.pairs.cpu().numpy().reshape(-1, 4)
+        assert 0 < len(pairs) <= 4096
+    s.assemble(); s.convert(); s.build_precond()
+    mas = oracle.Mas(sc.n, s.part_map, s.real_map, s.ns, s.nn, s.nl, sc.bank)
+    mas.build(*s.bcoo(), pairs=pairs)
+    t, to = s.mas_tables(), mas.tables()
+    for key in ("level_size", "coarse_space", "fine_mask", "prefix0"):
+        assert np.array_equal(t[key], to[key]), key
+    k = mas.levelnum - 1
+    assert np.array_equal(t["coarse_table"][:, :k], to["coarse_table"][:, :k])
+    r = np.random.default_rng(4).normal(size=3 * sc.n)
+    z, zo = s.precond_apply(r), mas.apply(r, fp32=False)
+    assert np.abs(z - zo).max() <= 1e-11 * np.abs(zo).max()

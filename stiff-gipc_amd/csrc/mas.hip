@@ -497,61 +497,106 @@ __global__ void k_proj_records(int K, const int* __restrict__ rows, const int* _
     for (int e = 0; e < 9; ++e) dst[e] += blk[e];
 }
 
-// contribution (9 doubles) of every sorted record
-__global__ void k_proj_contrib(long long m, const unsigned* __restrict__ key, const unsigned* __restrict__ rec,
-                               const int* __restrict__ rows, const int* __restrict__ cols,
-                               const double* __restrict__ vals, int off, int n, int B, const int* __restrict__ node_of,
-                               unsigned sentinel, double* __restrict__ contrib) {
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= m || key[i] == sentinel) return;
-    const unsigned q = rec[i];
-    const int k = (int)(q >> 3), l = (int)(q & 7u);
-    const int r = rows[k] - off, c = cols[k] - off;
-    const int I = node_of[(size_t)l * n + r], J = node_of[(size_t)l * n + c];
-    double H[9], blk[9];
-#pragma unroll
-    for (int e = 0; e < 9; ++e) H[e] = vals[9 * (size_t)k + e];
-    (void)project_block(B, I % B, J % B, r == c, H, blk);
-#pragma unroll
-    for (int e = 0; e < 9; ++e) contrib[9 * (size_t)i + e] = blk[e];
-}
-
-// Fixed-order segmented sum: records are cut into tiles of kProjTile; the
-// first record of each (entry, tile) piece sums the piece in record order,
-// then the first record of each entry sums its pieces in tile order.
+// Fixed-order segmented sum of the sorted records: a workgroup takes a tile of
+// kProjTile of them, puts their 3x3 contributions in LDS and adds every (entry,
+// tile) piece in record order, nine lanes (one component each) a piece.  A
+// piece that is a whole entry goes to its bank; one that begins in this tile
+// and goes on, or continues one of the tile before, goes to `part` and is added
+// in tile order by k_proj_carry.  Bound by the gather of the blocks (72 bytes
+// a record).  Contributions through memory with one thread a piece took 97 +
+// 710 + 64 us for 48 scenes (710 serial in pieces of up to 256), now 50 + 12; 64 to
+// 10 us for the one of 20 x 4 x 4 cells.
 constexpr int kProjTile = 256;
-__global__ void k_proj_pieces(long long m, const unsigned* __restrict__ key, unsigned sentinel,
-                              double* __restrict__ contrib) {
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= m) return;
-    const unsigned kk = key[i];
-    if (kk == sentinel || (i % kProjTile != 0 && key[i - 1] == kk)) return;
-    const long long tend = min(m, (i / kProjTile + 1) * kProjTile);
-    double acc[9];
+__global__ void __launch_bounds__(kProjTile) k_proj_tiles(long long m, const unsigned* __restrict__ key,
+                                                          const unsigned* __restrict__ rec,
+                                                          const int* __restrict__ rows, const int* __restrict__ cols,
+                                                          const double* __restrict__ vals, int off, int n, int B,
+                                                          const int* __restrict__ node_of, unsigned sentinel,
+                                                          double* __restrict__ bank_upper, double* __restrict__ part) {
+    __shared__ double v[kProjTile][9];
+    __shared__ unsigned keys[kProjTile];
+    __shared__ int head[kProjTile + 1];
+    __shared__ int waves[kProjTile / 64];
+    __shared__ int carried;  // the first piece continues one of the tile before
+    const int t = threadIdx.x;
+    const long long base = (long long)blockIdx.x * kProjTile, i = base + t;
+    const unsigned kk = i < m ? key[i] : sentinel;
+    const unsigned before = (i > 0 && i < m) ? key[i - 1] : sentinel;
+    const unsigned after = base + kProjTile < m ? key[base + kProjTile] : sentinel;
+    const bool valid = kk != sentinel;
+    keys[t] = kk;
+    if (valid) {
+        const unsigned q = rec[i];
+        const int k = (int)(q >> 3), l = (int)(q & 7u);
+        const int r = rows[k] - off, c = cols[k] - off;
+        double H[9], blk[9];
 #pragma unroll
-    for (int e = 0; e < 9; ++e) acc[e] = contrib[9 * (size_t)i + e];
-    for (long long j = i + 1; j < tend && key[j] == kk; ++j)
+        for (int e = 0; e < 9; ++e) H[e] = vals[9 * (size_t)k + e];
+        const int I = node_of[(size_t)l * n + r], J = node_of[(size_t)l * n + c];
+        (void)project_block(B, I % B, J % B, r == c, H, blk);
 #pragma unroll
-        for (int e = 0; e < 9; ++e) acc[e] += contrib[9 * (size_t)j + e];
+        for (int e = 0; e < 9; ++e) v[t][e] = blk[e];
+    }
+    const bool first = valid && (t == 0 || before != kk);
+    const unsigned long long heads = __ballot(first);
+    if ((t & 63) == 0) waves[t >> 6] = __popcll(heads);
+    const int nvalid = __syncthreads_count(valid);
+    int at = __popcll(heads & ((1ull << (t & 63)) - 1ull)), np = 0;
 #pragma unroll
-    for (int e = 0; e < 9; ++e) contrib[9 * (size_t)i + e] = acc[e];  // the piece sum, at the piece head
+    for (int w = 0; w < kProjTile / 64; ++w) {
+        if (w < (t >> 6)) at += waves[w];
+        np += waves[w];
+    }
+    if (first) head[at] = t;
+    if (t == 0) {
+        head[np] = nvalid;  // the sentinels sort last
+        carried = valid && before == kk;
+    }
+    __syncthreads();
+    for (int w = t; w < 9 * np; w += kProjTile) {
+        const int p = w / 9, e = w - 9 * p, h = head[p], end = head[p + 1];
+        double acc = v[h][e];
+#pragma unroll 8
+        for (int j = h + 1; j < end; ++j) acc += v[j][e];
+        if (p == 0 && carried)
+            part[((size_t)blockIdx.x * 2) * 9 + e] = acc;
+        else if (end == kProjTile && after == keys[h])
+            part[((size_t)blockIdx.x * 2 + 1) * 9 + e] = acc;
+        else
+            bank_upper[(size_t)keys[h] * 9 + e] = acc;
+    }
 }
 
-__global__ void k_proj_entries(long long m, const unsigned* __restrict__ key, unsigned sentinel,
-                               const double* __restrict__ contrib, double* __restrict__ bank_upper) {
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= m) return;
-    const unsigned kk = key[i];
-    if (kk == sentinel || (i > 0 && key[i - 1] == kk)) return;
-    double acc[9];
+// entries that run over several tiles: the piece of their first tile, then the
+// following ones in tile order (16 lanes a tile, eight pieces in flight)
+__global__ void k_proj_carry(long long m, int ntiles, const unsigned* __restrict__ key, unsigned sentinel,
+                             const double* __restrict__ part, double* __restrict__ bank_upper) {
+    const int g = blockIdx.x * blockDim.x + threadIdx.x, tile = g >> 4, e = g & 15;
+    if (tile + 1 >= ntiles || e >= 9) return;
+    const long long base = (long long)tile * kProjTile;
+    const unsigned kk = key[base + kProjTile - 1];
+    if (kk == sentinel || key[base + kProjTile] != kk) return;
+    if (tile > 0 && key[base] == kk && key[base - 1] == kk) return;  // began in an earlier tile
+    double acc = part[((size_t)tile * 2 + 1) * 9 + e];
+    constexpr int U = 8;
+    for (int t0 = tile + 1; t0 < ntiles; t0 += U) {
+        unsigned k[U];
+        double p[U];
 #pragma unroll
-    for (int e = 0; e < 9; ++e) acc[e] = contrib[9 * (size_t)i + e];
-    for (long long j = (i / kProjTile + 1) * kProjTile; j < m && key[j] == kk; j += kProjTile)
+        for (int u = 0; u < U; ++u) {
+            const int q = min(t0 + u, ntiles - 1);
+            k[u] = key[(long long)q * kProjTile];
+            p[u] = part[((size_t)q * 2) * 9 + e];
+        }
+        bool on = true;
 #pragma unroll
-        for (int e = 0; e < 9; ++e) acc[e] += contrib[9 * (size_t)j + e];
-    double* dst = bank_upper + (size_t)kk * 9;
-#pragma unroll
-    for (int e = 0; e < 9; ++e) dst[e] = acc[e];
+        for (int u = 0; u < U; ++u) {
+            on = on && t0 + u < ntiles && k[u] == kk;
+            if (on) acc += p[u];
+        }
+        if (!on) break;
+    }
+    bank_upper[(size_t)kk * 9 + e] = acc;
 }
 
 // top-level bank entries = sum of the per-workgroup partials, fixed order
@@ -1744,16 +1789,16 @@ void mas_build(Ctx& c, int sub_offset, int sub_nb, const int* pairs, int npairs)
                 SGIPC_HIP(rocprim::radix_sort_pairs(tmp, bytes, key, key + mrec, rec, rec + mrec, (size_t)mrec, 0,
                                                     bits, s));
             }
-            double* contrib = m.proj_contrib.reserve(9 * (size_t)mrec);
+            const int ntiles = div_up(mrec, kProjTile);
+            double* part = m.proj_part.reserve(18 * (size_t)ntiles);
             const unsigned* skey = key + mrec;
-            hipLaunchKernelGGL(k_proj_contrib, dim3(div_up(mrec, 256)), dim3(256), 0, s, mrec, skey,
+            hipLaunchKernelGGL(k_proj_tiles, dim3(ntiles), dim3(kProjTile), 0, s, mrec, skey,
                                (const unsigned*)(rec + mrec), (const int*)c.t_rows, (const int*)c.t_cols,
-                               (const double*)c.t_vals, sub_offset, n, B, (const int*)m.node_of.p, sentinel, contrib);
+                               (const double*)c.t_vals, sub_offset, n, B, (const int*)m.node_of.p, sentinel,
+                               m.bank_upper.p, part);
             SGIPC_LAUNCH_CHECK();
-            hipLaunchKernelGGL(k_proj_pieces, dim3(div_up(mrec, 256)), dim3(256), 0, s, mrec, skey, sentinel, contrib);
-            SGIPC_LAUNCH_CHECK();
-            hipLaunchKernelGGL(k_proj_entries, dim3(div_up(mrec, 256)), dim3(256), 0, s, mrec, skey, sentinel,
-                               (const double*)contrib, m.bank_upper.p);
+            hipLaunchKernelGGL(k_proj_carry, dim3(div_up(16LL * ntiles, 256)), dim3(256), 0, s, mrec, ntiles, skey,
+                               sentinel, (const double*)part, m.bank_upper.p);
             SGIPC_LAUNCH_CHECK();
         } else {
             hipLaunchKernelGGL(k_proj_records, dim3(div_up(c.K, 256)), dim3(256), 0, s, c.K, (const int*)c.t_rows,

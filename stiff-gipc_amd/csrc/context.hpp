@@ -120,11 +120,16 @@ struct Lbvh {
 };
 
 // Batched PCG over scenes concatenated block-row-wise (pcg_batch.hip)
+// A chunk of block rows [r0, r1) of one scene, and that scene's chunks [c0, c1)
+struct alignas(32) BatchChunk {
+    int r0, r1, scene, c0, c1;
+};
 struct BatchWork {
     int nch = 0;                                    // row chunks (never straddling a scene)
-    DBuf<int> chunk_row, chunk_scene, scene_chunk;  // nch + 1, nch, S + 1
+    DBuf<BatchChunk> chunk;                         // nch
+    DBuf<int> scene_chunk;                          // S + 1
     DBuf<double> part_pap, part_rr, part_rz;        // one partial per chunk
-    DBuf<double> bb, rz, rz0, alpha, beta, tol, segout;  // per scene
+    DBuf<double> bb, rz, rz0, tol, segout;  // per scene
     DBuf<int> stop, iters, noconv;                  // per scene
     DBuf<int> ctrl, bad, rstart;                    // C_* words; coupling check counter; row starts
     PcgGraph graph64, graph32, graph_mixed;

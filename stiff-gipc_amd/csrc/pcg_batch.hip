@@ -8,12 +8,12 @@
 //
 // Layout: block rows are cut into chunks that never straddle a scene (1024/G
 // rows for the SpMV with G lanes per row); one workgroup per chunk writes one
-// partial per dot product, and a scalar kernel (one wave per scene) sums
-// each scene's partials in chunk order (deterministic, no FP atomics) into
-// per-scene alpha / beta / stop words.  A stopped scene's rows are left untouched by
-// every later kernel.  The iteration sequence
-//   SpMV (Ap, p.Ap) -> alpha -> x, r update (r.r) -> MAS restrict + bank solve
-//   -> collect (z, r.z) -> beta + stop tests -> p update
+// partial per dot product, and every wavefront that needs a scene's sum adds
+// its partials in chunk order (deterministic, no FP atomics; the same value
+// everywhere), so no launch only sums.  A stopped scene's rows are left
+// untouched by every later kernel.  The iteration sequence
+//   SpMV (Ap, p.Ap) -> alpha; x, r update (r.r) -> MAS restrict + bank solve
+//   -> collect (z, r.z) -> stop test, beta; p update
 // is captured once into a HIP graph (several iterations per graph) and
 // replayed until every scene has stopped.
 //
@@ -29,33 +29,29 @@ namespace sgipc {
 namespace {
 
 constexpr int kBT = 256;       // threads of the row-wise batched kernels
-constexpr int kScalT = 1024;   // the scalar kernel: one wave per scene, 16 scenes per workgroup
+constexpr int kScalT = 1024;   // the start-up scalars: one wave per scene, 16 scenes per workgroup
 
-enum BPhase { B_INIT_BB = 0, B_INIT_RZ, B_ALPHA, B_BETA, B_SEGSUM };
+enum BPhase { B_INIT_BB = 0, B_INIT_RZ, B_SEGSUM };
 
 __device__ inline double wave_sum_partials(const double* __restrict__ part, int lo, int hi) {
     const int lane = threadIdx.x & 63;
     double v = 0.0;
     for (int i = lo + lane; i < hi; i += 64) v += part[i];
-    return wave_sum(v);
+    return __shfl(wave_sum(v), 0, 64);  // (the tree ends in the first lane)
 }
 
 // Ap = A p on the chunk's rows, partial p.Ap per chunk
 template <int G, typename MV, typename V>
-__global__ void __launch_bounds__(1024) k_bspmv(const int* __restrict__ chunk_row, const int* __restrict__ chunk_scene,
+__global__ void __launch_bounds__(1024) k_bspmv(const BatchChunk* __restrict__ chunk,
                                                 const int* __restrict__ eptr, const int2* __restrict__ ent,
                                                 const MV* __restrict__ val, const V* __restrict__ p,
                                                 V* __restrict__ Ap, const int* __restrict__ sstop,
                                                 double* __restrict__ part, const int* __restrict__ ctrl) {
-    if (ctrl[C_STOP]) return;
     __shared__ double sh[1024 / 64];
-    const int ch = blockIdx.x;
-    if (sstop[chunk_scene[ch]]) {
-        if (threadIdx.x == 0) part[ch] = 0.0;
-        return;
-    }
-    const int r0 = chunk_row[ch], r1 = chunk_row[ch + 1];
-    const int row = r0 + threadIdx.x / G, sub = threadIdx.x % G;
+    const BatchChunk c = chunk[blockIdx.x];
+    if (ctrl[C_STOP] || sstop[c.scene]) return;
+    const int r1 = c.r1;
+    const int row = c.r0 + threadIdx.x / G, sub = threadIdx.x % G;
     auto pv = [p](size_t i) { return p[i]; };
     MV s0 = 0, s1 = 0, s2 = 0;
     if (row < r1) sym_row_lane<G, MV>(row, sub, eptr, ent, val, pv, s0, s1, s2);
@@ -74,21 +70,17 @@ __global__ void __launch_bounds__(1024) k_bspmv(const int* __restrict__ chunk_ro
 // solves): the G lanes of a row stream consecutive entries; same entry
 // order and products as k_bspmv, so the same sums.
 template <int G>
-__global__ void __launch_bounds__(1024) k_bspmv_full(const int* __restrict__ chunk_row,
-                                                     const int* __restrict__ chunk_scene, const int* __restrict__ eptr,
+__global__ void __launch_bounds__(1024) k_bspmv_full(const BatchChunk* __restrict__ chunk,
+                                                     const int* __restrict__ eptr,
                                                      const float* __restrict__ vf,
                                                      const float* __restrict__ p, float* __restrict__ Ap,
                                                      const int* __restrict__ sstop, double* __restrict__ part,
                                                      const int* __restrict__ ctrl) {
-    if (ctrl[C_STOP]) return;
     __shared__ double sh[1024 / 64];
-    const int ch = blockIdx.x;
-    if (sstop[chunk_scene[ch]]) {
-        if (threadIdx.x == 0) part[ch] = 0.0;
-        return;
-    }
-    const int r0 = chunk_row[ch], r1 = chunk_row[ch + 1];
-    const int row = r0 + threadIdx.x / G, sub = threadIdx.x % G;
+    const BatchChunk c = chunk[blockIdx.x];
+    if (ctrl[C_STOP] || sstop[c.scene]) return;
+    const int r1 = c.r1;
+    const int row = c.r0 + threadIdx.x / G, sub = threadIdx.x % G;
     float s0 = 0, s1 = 0, s2 = 0;
     if (row < r1) {
         const int end = eptr[row + 1];
@@ -125,124 +117,188 @@ __global__ void __launch_bounds__(1024) k_bspmv_full(const int* __restrict__ chu
     write_partial(contrib, part, sh);
 }
 
-// x += alpha_s p ; r -= alpha_s Ap ; partial r.r per chunk
+// x += alpha_s p ; r -= alpha_s Ap ; partial r.r per chunk.  Every wavefront
+// sums its scene's partials of r.z and p.Ap for alpha; the scene's first chunk
+// keeps the old r.z for k_bpupdate.  Bound by dependent round trips, like the
+// two kernels below: the vectors are in flight while the partials are summed.
+// With alpha here and the stop test and beta in k_bpupdate, an iteration of 48
+// scenes has six launches instead of eight: 49.4 -> 40.5 us.
 template <typename V>
-__global__ void __launch_bounds__(kBT) k_bupdate(const int* __restrict__ chunk_row, const int* __restrict__ chunk_scene,
-                                                 double* __restrict__ x, V* __restrict__ r, const V* __restrict__ p,
-                                                 const V* __restrict__ Ap, const double* __restrict__ alpha,
+__global__ void __launch_bounds__(kBT) k_bupdate(const BatchChunk* __restrict__ chunk, double* __restrict__ x,
+                                                 V* __restrict__ r, const V* __restrict__ p, const V* __restrict__ Ap,
+                                                 const double* __restrict__ part_rz,
+                                                 const double* __restrict__ part_pap, double* __restrict__ rz,
                                                  const int* __restrict__ sstop, double* __restrict__ part,
-                                                 const int* __restrict__ ctrl) {
-    if (ctrl[C_STOP]) return;
+                                                 int* __restrict__ ctrl) {
     __shared__ double sh[kBT / 64];
-    const int ch = blockIdx.x, s = chunk_scene[ch];
-    if (sstop[s]) {
-        if (threadIdx.x == 0) part[ch] = 0.0;
-        return;
-    }
-    const double al = alpha[s];
-    const long long i1 = 3LL * chunk_row[ch + 1];
+    const BatchChunk c = chunk[blockIdx.x];
+    const int stopped = ctrl[C_STOP], ended = sstop[c.scene];
+    const double rzv = wave_sum_partials(part_rz, c.c0, c.c1);
+    const double pap = wave_sum_partials(part_pap, c.c0, c.c1);
+    constexpr int U = 2;
+    const long long i1 = 3LL * c.r1;
+    long long i = 3LL * c.r0 + threadIdx.x;
+    double xv[U];
+    V rv[U], pv[U], av[U];
+    auto take = [&]() {
+#pragma unroll
+        for (int k = 0; k < U; ++k) {
+            const long long j = min(i + k * kBT, i1 - 1);
+            xv[k] = x[j];
+            rv[k] = r[j];
+            pv[k] = p[j];
+            av[k] = Ap[j];
+        }
+    };
+    take();
+    if (stopped) return;
+    if (blockIdx.x == 0 && threadIdx.x == 0) ctrl[C_ITER] += 1;
+    if (ended) return;
+    const double al = rzv / pap;
     double v = 0.0;
-    for (long long i = 3LL * chunk_row[ch] + threadIdx.x; i < i1; i += kBT) {
-        x[i] += al * (double)p[i];
-        V ri = (V)((double)r[i] - al * (double)Ap[i]);
-        r[i] = ri;
-        v += (double)ri * (double)ri;
+    for (;;) {
+#pragma unroll
+        for (int k = 0; k < U; ++k) {
+            const long long j = i + k * kBT;
+            if (j >= i1) break;
+            x[j] = xv[k] + al * (double)pv[k];
+            const V ri = (V)((double)rv[k] - al * (double)av[k]);
+            r[j] = ri;
+            v += (double)ri * (double)ri;
+        }
+        i += U * kBT;
+        if (i - threadIdx.x >= i1) break;
+        take();
     }
     write_partial(v, part, sh);
+    if ((int)blockIdx.x == c.c0 && threadIdx.x == 0) rz[c.scene] = rzv;
 }
 
-// z = sum_l Z_l[node_l(v)] (MAS over all rows), partial r.z per chunk
+// z = sum_l Z_l[node_l(v)] (MAS over all rows), partial r.z per chunk; every
+// level's node, then every level's values, are loaded before any is used
 template <typename V, typename T>
-__global__ void __launch_bounds__(kBT) k_bcollect(const int* __restrict__ chunk_row, const int* __restrict__ chunk_scene,
-                                                  const V* __restrict__ r, V* __restrict__ z, int n, int L,
-                                                  const int* __restrict__ node_of, const T* __restrict__ Z,
-                                                  const int* __restrict__ sstop, double* __restrict__ part,
-                                                  const int* __restrict__ ctrl) {
-    if (ctrl[C_STOP]) return;
+__global__ void __launch_bounds__(kBT) k_bcollect(const BatchChunk* __restrict__ chunk, const V* __restrict__ r,
+                                                  V* __restrict__ z, int n, int L, const int* __restrict__ node_of,
+                                                  const T* __restrict__ Z, const int* __restrict__ sstop,
+                                                  double* __restrict__ part, const int* __restrict__ ctrl) {
     __shared__ double sh[kBT / 64];
-    const int ch = blockIdx.x;
-    if (sstop[chunk_scene[ch]]) {
-        if (threadIdx.x == 0) part[ch] = 0.0;
-        return;
-    }
+    constexpr int kL = 6;  // levels, at most
+    const BatchChunk c = chunk[blockIdx.x];
+    if (ctrl[C_STOP] || sstop[c.scene]) return;
     double v = 0.0;
-    for (int row = chunk_row[ch] + threadIdx.x; row < chunk_row[ch + 1]; row += kBT) {
-        T s0 = 0, s1 = 0, s2 = 0;
-        for (int l = 0; l < L; ++l) {
-            size_t g = 3 * (size_t)node_of[(size_t)l * n + row];
-            s0 += Z[g]; s1 += Z[g + 1]; s2 += Z[g + 2];
-        }
+    for (int row = c.r0 + threadIdx.x; row < c.r1; row += kBT) {
+        int g[kL];
+#pragma unroll
+        for (int l = 0; l < kL; ++l) g[l] = node_of[(size_t)min(l, L - 1) * n + row];
         const size_t o = 3 * (size_t)row;
+        const V r0 = r[o], r1 = r[o + 1], r2 = r[o + 2];
+        T q[kL][3];
+#pragma unroll
+        for (int l = 0; l < kL; ++l)
+#pragma unroll
+            for (int e = 0; e < 3; ++e) q[l][e] = Z[3 * (size_t)g[l] + e];
+        T s0 = 0, s1 = 0, s2 = 0;
+#pragma unroll
+        for (int l = 0; l < kL; ++l)
+            if (l < L) {
+                s0 += q[l][0];
+                s1 += q[l][1];
+                s2 += q[l][2];
+            }
         const V z0 = (V)s0, z1 = (V)s1, z2 = (V)s2;
         z[o] = z0; z[o + 1] = z1; z[o + 2] = z2;
-        v += (double)r[o] * (double)z0 + (double)r[o + 1] * (double)z1 + (double)r[o + 2] * (double)z2;
+        v += (double)r0 * (double)z0 + (double)r1 * (double)z1 + (double)r2 * (double)z2;
     }
-    write_partial(v, part, sh);
-}
-
-// p = z + beta_s p (beta_s = 0 on the first iteration)
-template <typename V>
-__global__ void __launch_bounds__(kBT) k_bpupdate(const int* __restrict__ chunk_row, const int* __restrict__ chunk_scene,
-                                                  const V* __restrict__ z, V* __restrict__ p,
-                                                  const double* __restrict__ beta, const int* __restrict__ sstop,
-                                                  const int* __restrict__ ctrl, int first) {
-    if (!first && ctrl[C_STOP]) return;
-    const int ch = blockIdx.x, s = chunk_scene[ch];
-    if (sstop[s]) return;
-    const double be = first ? 0.0 : beta[s];
-    const long long i1 = 3LL * chunk_row[ch + 1];
-    for (long long i = 3LL * chunk_row[ch] + threadIdx.x; i < i1; i += kBT)
-        p[i] = first ? z[i] : (V)((double)z[i] + be * (double)p[i]);
-}
-
-// partials of a.b per chunk (all scenes)
-template <typename VA, typename VB>
-__global__ void __launch_bounds__(kBT) k_bdot(const int* __restrict__ chunk_row, const VA* __restrict__ a,
-                                              const VB* __restrict__ b, double* __restrict__ part) {
-    __shared__ double sh[kBT / 64];
-    const int ch = blockIdx.x;
-    const long long i1 = 3LL * chunk_row[ch + 1];
-    double v = 0.0;
-    for (long long i = 3LL * chunk_row[ch] + threadIdx.x; i < i1; i += kBT) v += (double)a[i] * (double)b[i];
     write_partial(v, part, sh);
 }
 
 struct BScal {
-    double *bb, *rz, *rz0, *alpha, *beta, *tol, *out;
+    double *bb, *rz, *rz0, *tol, *out;
     int *stop, *iters, *noconv;
 };
 
-// extra control words of the batched solver (after the shared C_* words)
-constexpr int kCActive = C_NUM;      // active scenes counted by the workgroups of a scalar kernel
-constexpr int kCTicket = C_NUM + 1;  // workgroups of that kernel done
+constexpr int kCActive = C_NUM;      // scenes that have not stopped (after the shared C_* words)
+constexpr int kCTicket = C_NUM + 1;  // workgroups of the start-up scalars done
 
-// Per-scene scalars: one wave per scene, 16 scenes per workgroup.  The
-// phases that decide the stop (INIT_RZ, BETA) count active scenes per
-// workgroup; the last workgroup to finish sets the stop word and advances
-// the iteration counter (every workgroup has read both before it finishes).
+// Stop test of the scene, then p = z + beta_s p.  Every wavefront takes the
+// same decision from the same sums; the scene's first chunk writes it, and the
+// last scene to stop sets the stop word.  (A chunk that starts later and sees
+// its scene stopped would have left p alone as well.)
+template <typename V>
+__global__ void __launch_bounds__(kBT) k_bpupdate(const BatchChunk* __restrict__ chunk, const V* __restrict__ z,
+                                                  V* __restrict__ p, const double* __restrict__ part_rr,
+                                                  const double* __restrict__ part_rz, BScal q, int rule,
+                                                  int* __restrict__ ctrl) {
+    const BatchChunk c = chunk[blockIdx.x];
+    const int s = c.scene;
+    const int stopped = ctrl[C_STOP], ended = q.stop[s], k = ctrl[C_ITER] - 1, maxit = ctrl[C_MAXIT];
+    const double rr = wave_sum_partials(part_rr, c.c0, c.c1);
+    const double rzn = wave_sum_partials(part_rz, c.c0, c.c1);
+    const double rz = q.rz[s], tol = q.tol[s], ref = rule == 0 ? q.rz0[s] : q.bb[s];
+    constexpr int U = 2;
+    const long long i1 = 3LL * c.r1;
+    long long i = 3LL * c.r0 + threadIdx.x;
+    V zv[U], pv[U];
+    auto take = [&]() {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const long long j = min(i + u * kBT, i1 - 1);
+            zv[u] = z[j];
+            pv[u] = p[j];
+        }
+    };
+    take();
+    if (stopped || ended) return;
+    const bool met = rule == 0 ? fabs(rz) <= tol * ref : sqrt(rr) <= tol * sqrt(ref);
+    if (met || k + 1 >= maxit) {
+        if ((int)blockIdx.x == c.c0 && threadIdx.x == 0) {
+            q.iters[s] = met ? k : maxit;
+            if (!met) q.noconv[s] = 1;
+            q.stop[s] = 1;
+            if (atomicSub(ctrl + kCActive, 1) == 1) ctrl[C_STOP] = 1;
+        }
+        return;
+    }
+    const double be = rzn / rz;
+    for (;;) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const long long j = i + u * kBT;
+            if (j < i1) p[j] = (V)((double)zv[u] + be * (double)pv[u]);
+        }
+        i += U * kBT;
+        if (i - threadIdx.x >= i1) break;
+        take();
+    }
+}
+
+// partials of a.b per chunk (all scenes)
+template <typename VA, typename VB>
+__global__ void __launch_bounds__(kBT) k_bdot(const BatchChunk* __restrict__ chunk, const VA* __restrict__ a,
+                                              const VB* __restrict__ b, double* __restrict__ part) {
+    __shared__ double sh[kBT / 64];
+    const BatchChunk c = chunk[blockIdx.x];
+    const long long i1 = 3LL * c.r1;
+    double v = 0.0;
+    for (long long i = 3LL * c.r0 + threadIdx.x; i < i1; i += kBT) v += (double)a[i] * (double)b[i];
+    write_partial(v, part, sh);
+}
+
+// Per-scene sums outside the iterations: one wave per scene, 16 scenes per
+// workgroup.  INIT_RZ counts the scenes that have work; the last workgroup to
+// finish sets the stop word.
 __global__ void __launch_bounds__(kScalT) k_bscalars(int phase, int S, const int* __restrict__ scene_chunk,
-                                                     const double* __restrict__ pa, const double* __restrict__ pb,
-                                                     BScal q, int rule, int* __restrict__ ctrl) {
-    if ((phase == B_ALPHA || phase == B_BETA) && ctrl[C_STOP]) return;
+                                                     const double* __restrict__ pa, BScal q, int* __restrict__ ctrl) {
     __shared__ int act[kScalT / 64];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int k = ctrl[C_ITER];
+    const int s = blockIdx.x * (kScalT / 64) + w;
     int active = 0;
-    for (int s = blockIdx.x * (kScalT / 64) + w; s < S && s < (blockIdx.x + 1) * (kScalT / 64); s += kScalT / 64) {
-        const int lo = scene_chunk[s], hi = scene_chunk[s + 1];
-        if (phase == B_SEGSUM) {
-            double v = wave_sum_partials(pa, lo, hi);
-            if (lane == 0) q.out[s] = v;
-            continue;
-        }
-        if (phase == B_INIT_BB) {
-            double v = wave_sum_partials(pa, lo, hi);
-            if (lane == 0) q.bb[s] = v;
-            continue;
-        }
-        if (phase == B_INIT_RZ) {
-            double v = wave_sum_partials(pa, lo, hi);
-            if (lane == 0) {
+    if (s < S) {
+        const double v = wave_sum_partials(pa, scene_chunk[s], scene_chunk[s + 1]);
+        if (lane == 0) {
+            if (phase == B_SEGSUM) q.out[s] = v;
+            if (phase == B_INIT_BB) q.bb[s] = v;
+            if (phase == B_INIT_RZ) {
                 q.rz[s] = v;
                 q.rz0[s] = v;
                 q.iters[s] = 0;
@@ -253,37 +309,11 @@ __global__ void __launch_bounds__(kScalT) k_bscalars(int phase, int S, const int
                     q.iters[s] = ctrl[C_MAXIT];
                     q.noconv[s] = 1;
                 }
-                if (!q.stop[s]) active += 1;
-            }
-            continue;
-        }
-        if (q.stop[s]) continue;
-        if (phase == B_ALPHA) {
-            double pap = wave_sum_partials(pa, lo, hi);
-            if (lane == 0) q.alpha[s] = q.rz[s] / pap;
-            continue;
-        }
-        // B_BETA: pa = r.r partials (updated r), pb = r.z partials (new z)
-        double rr = wave_sum_partials(pa, lo, hi);
-        double rzn = wave_sum_partials(pb, lo, hi);
-        if (lane == 0) {
-            bool stop = rule == 0 ? fabs(q.rz[s]) <= q.tol[s] * q.rz0[s] : sqrt(rr) <= q.tol[s] * sqrt(q.bb[s]);
-            if (stop) {
-                q.stop[s] = 1;
-                q.iters[s] = k;
-            } else if (k + 1 >= ctrl[C_MAXIT]) {
-                q.stop[s] = 1;
-                q.iters[s] = ctrl[C_MAXIT];
-                q.noconv[s] = 1;
-            } else {
-                q.beta[s] = rzn / q.rz[s];
-                q.rz[s] = rzn;
-                active += 1;
+                if (!q.stop[s]) active = 1;
             }
         }
     }
-    if (phase == B_SEGSUM || phase == B_INIT_BB || phase == B_ALPHA) return;
-    active = (int)wave_sum((double)active);
+    if (phase != B_INIT_RZ) return;
     if (lane == 0) act[w] = active;
     __syncthreads();
     if (threadIdx.x == 0) {
@@ -293,17 +323,10 @@ __global__ void __launch_bounds__(kScalT) k_bscalars(int phase, int S, const int
         __threadfence();
         if (atomicAdd(ctrl + kCTicket, 1) == (int)gridDim.x - 1) {  // last workgroup
             __threadfence();
-            const int all = atomicAdd(ctrl + kCActive, 0);
-            ctrl[kCActive] = 0;
             ctrl[kCTicket] = 0;
-            if (phase == B_INIT_RZ) {
-                ctrl[C_ITER] = 1;
-                ctrl[C_STOP] = all == 0 ? 1 : 0;
-                ctrl[C_NOCONV] = 0;
-            } else {
-                ctrl[C_ITER] = k + 1;
-                if (all == 0) ctrl[C_STOP] = 1;
-            }
+            ctrl[C_ITER] = 1;
+            ctrl[C_STOP] = atomicAdd(ctrl + kCActive, 0) == 0 ? 1 : 0;
+            ctrl[C_NOCONV] = 0;
         }
     }
 }
@@ -363,15 +386,14 @@ struct BEngine {
     const float* vfull = nullptr;  // mixed: row-contiguous FP32 copy of both triangles (else the upper BCOO)
 
     BScal scal() {
-        return BScal{w.bb.p, w.rz.p, w.rz0.p, w.alpha.p, w.beta.p, w.tol.p, w.segout.p, w.stop.p, w.iters.p,
-                     w.noconv.p};
+        return BScal{w.bb.p, w.rz.p, w.rz0.p, w.tol.p, w.segout.p, w.stop.p, w.iters.p, w.noconv.p};
     }
     T* Rm() { return fp32mas ? (T*)(void*)c.mas.R32.p : (T*)(void*)c.mas.R64.p; }
     T* Zm() { return fp32mas ? (T*)(void*)c.mas.Z32.p : (T*)(void*)c.mas.Z64.p; }
 
-    void scalars(int phase, const double* pa, const double* pb) {
+    void scalars(int phase, const double* pa) {
         hipLaunchKernelGGL(k_bscalars, dim3(div_up(S, kScalT / 64)), dim3(kScalT), 0, c.stream, phase, S,
-                           (const int*)w.scene_chunk.p, pa, pb, scal(), rule, w.ctrl.p);
+                           (const int*)w.scene_chunk.p, pa, scal(), w.ctrl.p);
         SGIPC_LAUNCH_CHECK();
     }
 
@@ -382,8 +404,8 @@ struct BEngine {
         mas_restrict(c, r, 0, fp32mas, w.ctrl.p, !fused, skip);
         if (fused) mas_solve_with_top(c, fp32mas, w.ctrl.p, skip);
         else mas_bank_solve(c, fp32mas, w.ctrl.p, skip);
-        hipLaunchKernelGGL((k_bcollect<V, T>), dim3(nch), dim3(kBT), 0, c.stream, (const int*)w.chunk_row.p,
-                           (const int*)w.chunk_scene.p, (const V*)r, z, c.mas.n, c.mas.L, (const int*)c.mas.node_of.p,
+        hipLaunchKernelGGL((k_bcollect<V, T>), dim3(nch), dim3(kBT), 0, c.stream,
+                           (const BatchChunk*)w.chunk.p, (const V*)r, z, c.mas.n, c.mas.L, (const int*)c.mas.node_of.p,
                            (const T*)Zm(), (const int*)w.stop.p, w.part_rz.p, (const int*)w.ctrl.p);
         SGIPC_LAUNCH_CHECK();
     }
@@ -392,15 +414,15 @@ struct BEngine {
         hipStream_t s = c.stream;
         const SymBcoo& B = c.bsr;
         auto launch = [&](auto kern) {
-            hipLaunchKernelGGL(kern, dim3(nch), dim3(1024), 0, s, (const int*)w.chunk_row.p,
-                               (const int*)w.chunk_scene.p, (const int*)B.eptr.p, (const int2*)B.ent.p, val,
+            hipLaunchKernelGGL(kern, dim3(nch), dim3(1024), 0, s, (const BatchChunk*)w.chunk.p,
+                               (const int*)B.eptr.p, (const int2*)B.ent.p, val,
                                (const V*)p, Ap, (const int*)w.stop.p, w.part_pap.p, (const int*)w.ctrl.p);
         };
         if constexpr (sizeof(MV) == 4 && sizeof(V) == 4) {
             if (vfull) {
                 auto launchf = [&](auto kern) {
-                    hipLaunchKernelGGL(kern, dim3(nch), dim3(1024), 0, s, (const int*)w.chunk_row.p,
-                                       (const int*)w.chunk_scene.p, (const int*)B.eptr.p, vfull,
+                    hipLaunchKernelGGL(kern, dim3(nch), dim3(1024), 0, s,
+                                       (const BatchChunk*)w.chunk.p, (const int*)B.eptr.p, vfull,
                                        (const float*)p, (float*)Ap, (const int*)w.stop.p, w.part_pap.p,
                                        (const int*)w.ctrl.p);
                 };
@@ -415,16 +437,13 @@ struct BEngine {
             else launch(k_bspmv<8, MV, V>);
         }
         SGIPC_LAUNCH_CHECK();
-        scalars(B_ALPHA, w.part_pap.p, nullptr);
-        hipLaunchKernelGGL((k_bupdate<V>), dim3(nch), dim3(kBT), 0, s, (const int*)w.chunk_row.p,
-                           (const int*)w.chunk_scene.p, x, r, (const V*)p, (const V*)Ap, (const double*)w.alpha.p,
-                           (const int*)w.stop.p, w.part_rr.p, (const int*)w.ctrl.p);
+        hipLaunchKernelGGL((k_bupdate<V>), dim3(nch), dim3(kBT), 0, s, (const BatchChunk*)w.chunk.p, x, r,
+                           (const V*)p, (const V*)Ap, (const double*)w.part_rz.p, (const double*)w.part_pap.p, w.rz.p,
+                           (const int*)w.stop.p, w.part_rr.p, w.ctrl.p);
         SGIPC_LAUNCH_CHECK();
         precond();
-        scalars(B_BETA, w.part_rr.p, w.part_rz.p);
-        hipLaunchKernelGGL((k_bpupdate<V>), dim3(nch), dim3(kBT), 0, s, (const int*)w.chunk_row.p,
-                           (const int*)w.chunk_scene.p, (const V*)z, p, (const double*)w.beta.p,
-                           (const int*)w.stop.p, (const int*)w.ctrl.p, 0);
+        hipLaunchKernelGGL((k_bpupdate<V>), dim3(nch), dim3(kBT), 0, s, (const BatchChunk*)w.chunk.p, (const V*)z, p,
+                           (const double*)w.part_rr.p, (const double*)w.part_rz.p, scal(), rule, w.ctrl.p);
         SGIPC_LAUNCH_CHECK();
     }
 
@@ -435,15 +454,13 @@ struct BEngine {
         hipLaunchKernelGGL(k_bctrl_init, dim3(1), dim3(1), 0, s, w.ctrl.p, maxit);
         SGIPC_LAUNCH_CHECK();
         fill<double>(x, 0.0, N, s);
-        hipLaunchKernelGGL((k_bdot<V, V>), dim3(nch), dim3(kBT), 0, s, (const int*)w.chunk_row.p, (const V*)r,
-                           (const V*)r, w.part_rr.p);
+        hipLaunchKernelGGL((k_bdot<V, V>), dim3(nch), dim3(kBT), 0, s, (const BatchChunk*)w.chunk.p,
+                           (const V*)r, (const V*)r, w.part_rr.p);
         SGIPC_LAUNCH_CHECK();
-        scalars(B_INIT_BB, w.part_rr.p, nullptr);
+        scalars(B_INIT_BB, w.part_rr.p);
         precond();
-        scalars(B_INIT_RZ, w.part_rz.p, nullptr);
-        hipLaunchKernelGGL((k_bpupdate<V>), dim3(nch), dim3(kBT), 0, s, (const int*)w.chunk_row.p,
-                           (const int*)w.chunk_scene.p, (const V*)z, p, (const double*)w.beta.p,
-                           (const int*)w.stop.p, (const int*)w.ctrl.p, 1);
+        scalars(B_INIT_RZ, w.part_rz.p);
+        hipLaunchKernelGGL((k_bcast<V, V>), dim3(flat_grid(N)), dim3(256), 0, s, N, p, (const V*)z);
         SGIPC_LAUNCH_CHECK();
     }
 
@@ -455,10 +472,9 @@ struct BEngine {
         mix((size_t)rule); mix((size_t)r); mix((size_t)z); mix((size_t)p); mix((size_t)Ap); mix((size_t)x);
         mix((size_t)val); mix((size_t)fp32mas); mix((size_t)B.eptr.p); mix((size_t)B.ent.p); mix((size_t)B.nb);
         mix((size_t)vfull); mix((size_t)mas_fused(c));
-        for (const void* q : {(const void*)w.chunk_row.p, (const void*)w.chunk_scene.p, (const void*)w.scene_chunk.p,
+        for (const void* q : {(const void*)w.chunk.p, (const void*)w.scene_chunk.p,
                               (const void*)w.part_pap.p, (const void*)w.part_rr.p, (const void*)w.part_rz.p,
-                              (const void*)w.bb.p, (const void*)w.rz.p, (const void*)w.rz0.p, (const void*)w.alpha.p,
-                              (const void*)w.beta.p, (const void*)w.tol.p, (const void*)w.segout.p,
+                              (const void*)w.bb.p, (const void*)w.rz.p, (const void*)w.rz0.p, (const void*)w.tol.p, (const void*)w.segout.p,
                               (const void*)w.stop.p, (const void*)w.iters.p, (const void*)w.noconv.p,
                               (const void*)w.ctrl.p, (const void*)w.bank_scene.p})
             mix((size_t)q);
@@ -509,11 +525,9 @@ struct BEngine {
 // per-scene sums of a chunk-partial array, to the host
 void seg_to_host(Ctx& c, BatchWork& w, int S, const double* part, std::vector<double>& out) {
     hipLaunchKernelGGL(k_bscalars, dim3(div_up(S, kScalT / 64)), dim3(kScalT), 0, c.stream, (int)B_SEGSUM, S,
-                       (const int*)w.scene_chunk.p,
-                       part, (const double*)nullptr,
-                       BScal{w.bb.p, w.rz.p, w.rz0.p, w.alpha.p, w.beta.p, w.tol.p, w.segout.p, w.stop.p, w.iters.p,
-                             w.noconv.p},
-                       0, w.ctrl.p);
+                       (const int*)w.scene_chunk.p, part,
+                       BScal{w.bb.p, w.rz.p, w.rz0.p, w.tol.p, w.segout.p, w.stop.p, w.iters.p, w.noconv.p},
+                       w.ctrl.p);
     SGIPC_LAUNCH_CHECK();
     out.resize(S);
     SGIPC_HIP(hipMemcpyAsync(out.data(), w.segout.p, sizeof(double) * S, hipMemcpyDeviceToHost, c.stream));
@@ -523,23 +537,20 @@ void seg_to_host(Ctx& c, BatchWork& w, int S, const double* part, std::vector<do
 // chunk table: scenes cut into chunks of at most `rows` block rows
 void build_chunks(Ctx& c, BatchWork& w, const std::vector<int>& rs, int rows) {
     const int S = (int)rs.size() - 1;
-    std::vector<int> crow, cscene, schunk(S + 1, 0);
+    std::vector<BatchChunk> chunk;
+    std::vector<int> schunk(S + 1, 0);
     for (int s = 0; s < S; ++s) {
-        schunk[s] = (int)cscene.size();
-        for (int r0 = rs[s]; r0 < rs[s + 1]; r0 += rows) {
-            crow.push_back(r0);
-            cscene.push_back(s);
-        }
+        const int c0 = (int)chunk.size(), c1 = c0 + (rs[s + 1] - rs[s] + rows - 1) / rows;
+        schunk[s] = c0;
+        for (int r0 = rs[s]; r0 < rs[s + 1]; r0 += rows)
+            chunk.push_back(BatchChunk{r0, std::min(r0 + rows, rs[s + 1]), s, c0, c1});
     }
-    schunk[S] = (int)cscene.size();
-    crow.push_back(rs[S]);
-    const int nch = (int)cscene.size();
+    const int nch = (int)chunk.size();
+    schunk[S] = nch;
     w.nch = nch;
-    w.chunk_row.reserve(nch + 1);
-    w.chunk_scene.reserve(nch + 1);
+    w.chunk.reserve(nch + 1);
     w.scene_chunk.reserve(S + 1);
-    SGIPC_HIP(hipMemcpy(w.chunk_row.p, crow.data(), sizeof(int) * (nch + 1), hipMemcpyHostToDevice));
-    if (nch) SGIPC_HIP(hipMemcpy(w.chunk_scene.p, cscene.data(), sizeof(int) * nch, hipMemcpyHostToDevice));
+    if (nch) SGIPC_HIP(hipMemcpy(w.chunk.p, chunk.data(), sizeof(BatchChunk) * nch, hipMemcpyHostToDevice));
     SGIPC_HIP(hipMemcpy(w.scene_chunk.p, schunk.data(), sizeof(int) * (S + 1), hipMemcpyHostToDevice));
     for (DBuf<double>* b : {&w.part_pap, &w.part_rr, &w.part_rz}) b->reserve(nch + 1);
 }
@@ -589,7 +600,7 @@ void pcg_solve_batched(Ctx& c, int S, const int* h_row_start, const double* b, d
     build_chunks(c, w, rs, 1024 / G);
     batch_check_coupling(c, rs);
     batch_scene_maps(c, S, w.rstart.p, nullptr, nullptr);  // banks of stopped scenes are skipped
-    for (DBuf<double>* q : {&w.bb, &w.rz, &w.rz0, &w.alpha, &w.beta, &w.tol, &w.segout}) q->reserve(S + 1);
+    for (DBuf<double>* q : {&w.bb, &w.rz, &w.rz0, &w.tol, &w.segout}) q->reserve(S + 1);
     for (DBuf<int>* q : {&w.stop, &w.iters, &w.noconv}) q->reserve(S + 1);
     w.ctrl.reserve(C_NUM + 8);
     const long long N = 3LL * c.nb;
@@ -639,7 +650,7 @@ void pcg_solve_batched(Ctx& c, int S, const int* h_row_start, const double* b, d
         hipLaunchKernelGGL((k_bcast<double, double>), dim3(flat_grid(N)), dim3(256), 0, s, N, r64, b);
         SGIPC_LAUNCH_CHECK();
         std::vector<double> bb, rr;
-        hipLaunchKernelGGL((k_bdot<double, double>), dim3(w.nch), dim3(kBT), 0, s, (const int*)w.chunk_row.p, b, b,
+        hipLaunchKernelGGL((k_bdot<double, double>), dim3(w.nch), dim3(kBT), 0, s, (const BatchChunk*)w.chunk.p, b, b,
                            w.part_rr.p);
         SGIPC_LAUNCH_CHECK();
         seg_to_host(c, w, S, w.part_rr.p, bb);
@@ -678,7 +689,7 @@ void pcg_solve_batched(Ctx& c, int S, const int* h_row_start, const double* b, d
             hipLaunchKernelGGL((k_bcast<double, double>), dim3(flat_grid(N)), dim3(256), 0, s, N, r64, b);
             SGIPC_LAUNCH_CHECK();
             spmv64(c, -1.0, x, 1.0, r64);
-            hipLaunchKernelGGL((k_bdot<double, double>), dim3(w.nch), dim3(kBT), 0, s, (const int*)w.chunk_row.p,
+            hipLaunchKernelGGL((k_bdot<double, double>), dim3(w.nch), dim3(kBT), 0, s, (const BatchChunk*)w.chunk.p,
                                (const double*)r64, (const double*)r64, w.part_rr.p);
             SGIPC_LAUNCH_CHECK();
             seg_to_host(c, w, S, w.part_rr.p, rr);
@@ -695,11 +706,11 @@ void pcg_solve_batched(Ctx& c, int S, const int* h_row_start, const double* b, d
     SGIPC_LAUNCH_CHECK();
     spmv64(c, -1.0, x, 1.0, tmp);
     std::vector<double> rr, bb;
-    hipLaunchKernelGGL((k_bdot<double, double>), dim3(w.nch), dim3(kBT), 0, s, (const int*)w.chunk_row.p,
+    hipLaunchKernelGGL((k_bdot<double, double>), dim3(w.nch), dim3(kBT), 0, s, (const BatchChunk*)w.chunk.p,
                        (const double*)tmp, (const double*)tmp, w.part_rr.p);
     SGIPC_LAUNCH_CHECK();
     seg_to_host(c, w, S, w.part_rr.p, rr);
-    hipLaunchKernelGGL((k_bdot<double, double>), dim3(w.nch), dim3(kBT), 0, s, (const int*)w.chunk_row.p, b, b,
+    hipLaunchKernelGGL((k_bdot<double, double>), dim3(w.nch), dim3(kBT), 0, s, (const BatchChunk*)w.chunk.p, b, b,
                        w.part_rr.p);
     SGIPC_LAUNCH_CHECK();
     seg_to_host(c, w, S, w.part_rr.p, bb);

@@ -312,3 +312,32 @@ def test_autotune_then_batched_solve(torch_cuda, five_scenes):
     assert np.linalg.norm(x - x0) <= 1e-3 * np.linalg.norm(x0)
     bn.sys.ctx.call("sgipc_set_schedule", 8, 4)
     bn.set_mode(False)
+
+
+@pytest.mark.parametrize("group,per_graph", [(4, 3), (16, 1), (16, 4)])
+def test_launch_sequence_chunk_sizes(torch_cuda, five_scenes, group, per_graph):
+    """Chunks of 256 and 64 block rows, odd graph lengths and a scene of more
+    chunks than a wavefront has lanes: the sums of each scene are formed by
+    every workgroup from its chunks' partials.  Iteration counts equal those of
+    the default schedule (or the single-system solver); iterates differ by the
+    order of the FP64 sums only (1e-10, as against the oracle above)."""
+    from sgipc import capi, scene
+    from sgipc.system import NewtonSystem
+    print("case: batched launch sequence group", group, "per graph", per_graph, flush=True)
+    _, bn = five_scenes
+    big = NewtonSystem(scene.cube_scene(17, seed=5), "cuda:0", precond=capi.PRECOND_MAS)
+    big.assemble(); big.convert(); big.build_precond()
+    for sysm, rs in ((bn.sys, bn.row_start), (big, [0, big.n])):
+        st0, x0 = _solve_batched(sysm, rs, capi.PRECISION_FP64, 1e-4, 0)
+        sysm.ctx.call("sgipc_set_schedule", group, per_graph)
+        try:
+            st, x = _solve_batched(sysm, rs, capi.PRECISION_FP64, 1e-4, 0)
+        finally:
+            sysm.ctx.call("sgipc_set_schedule", 8, 4)
+        S = len(rs) - 1
+        assert [st[s].iterations for s in range(S)] == [st0[s].iterations for s in range(S)]
+        assert all(st[s].converged for s in range(S))
+        assert np.linalg.norm(x - x0) <= 1e-10 * np.linalg.norm(x0)
+    one = big.solve(tol=1e-4, stop_rule=0)
+    assert one.iterations == st[0].iterations
+    assert np.linalg.norm(big.dx.cpu().numpy() - x) <= 1e-10 * np.linalg.norm(x)

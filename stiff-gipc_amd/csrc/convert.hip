@@ -210,49 +210,68 @@ __global__ void k_merge_write(int nbr, const int* __restrict__ sstart, const int
     }
 }
 
-// value of each merged block: its contact triplets, then its static ones,
-// each run in ascending triplet order
-__global__ void k_merge_values(int K, const int4* __restrict__ desc, const int* __restrict__ dsorted,
-                               const int* __restrict__ ssorted, int sshift, const double* __restrict__ vals,
-                               double* __restrict__ oval) {
-    int u = blockIdx.x * blockDim.x + threadIdx.x;
-    if (u >= K) return;
-    int4 d = desc[u];
-    const int n = d.y + d.w;
-    double acc[9];
-    // groups of four contributions: their ids, then their values, are loaded
-    // before any is added, so the loads overlap; the sum keeps the order
-    // q = 0, 1, ... (bit-identical to a sequential loop)
-    constexpr int kG = 4;
-    for (int q0 = 0; q0 < n; q0 += kG) {
-        int t[kG];
-#pragma unroll
-        for (int j = 0; j < kG; ++j) {
-            const int q = q0 + j;
-            t[j] = q >= n ? -1 : ((q < d.y) ? dsorted[d.x + q] : ssorted[d.z + (q - d.y)] + sshift);
+// Value of each merged block: its contact triplets, then its static ones, each
+// run in ascending triplet order.  A workgroup takes kMergeBlocks blocks and
+// reads their triplets in batches of kMergeBatch into LDS, nine lanes (72
+// contiguous bytes) a triplet; then nine lanes a block add its own in order
+// (bit-identical to a sequential loop).  A diagonal block has some 25 triplets
+// and an off-diagonal one about six, so a lane that fetches for its own block
+// waits for its neighbours most of the time; in a batch every lane always
+// fetches.  Bound by the read of the triplets (461 MB in 72-byte pieces at 640 k
+// tets, a line of which several blocks share): 273 -> 177 us there, 18 -> 6 us at
+// 5000 tets; nine lanes a block without the batches took 379 and 11 us.
+constexpr int kMergeBlocks = 32;               // merged blocks per workgroup
+constexpr int kMergeT = 9 * kMergeBlocks;
+constexpr int kMergeBatch = 256;
+__global__ void __launch_bounds__(kMergeT) k_merge_values(int K, const int4* __restrict__ desc,
+                                                          const int* __restrict__ dsorted,
+                                                          const int* __restrict__ ssorted, int sshift,
+                                                          const double* __restrict__ vals, double* __restrict__ oval) {
+    __shared__ double prod[9 * kMergeBatch];
+    __shared__ int ids[kMergeBatch];
+    __shared__ int4 run[kMergeBlocks];
+    __shared__ int off[kMergeBlocks + 1];      // triplets before each block
+    const int tid = threadIdx.x, w = tid / 9, e = tid - 9 * w, u0 = blockIdx.x * kMergeBlocks;
+    if (tid < 64) {
+        const int4 d = (tid < kMergeBlocks && u0 + tid < K) ? desc[u0 + tid] : make_int4(0, 0, 0, 0);
+        int n = d.y + d.w;
+        for (int o = 1; o < kMergeBlocks; o <<= 1) {
+            const int m = __shfl_up(n, o, 64);
+            if (tid >= o) n += m;
         }
-        double v[kG][9];
-#pragma unroll
-        for (int j = 0; j < kG; ++j)
-            if (t[j] >= 0) {
-                const double* src = vals + 9 * (size_t)t[j];
-#pragma unroll
-                for (int e = 0; e < 9; ++e) v[j][e] = src[e];
-            }
-#pragma unroll
-        for (int j = 0; j < kG; ++j) {
-            if (t[j] < 0) break;
-            if (q0 + j == 0) {
-#pragma unroll
-                for (int e = 0; e < 9; ++e) acc[e] = v[j][e];
-            } else {
-#pragma unroll
-                for (int e = 0; e < 9; ++e) acc[e] += v[j][e];
-            }
+        if (tid < kMergeBlocks) {
+            run[tid] = d;
+            off[tid + 1] = n;
         }
+        if (tid == 0) off[0] = 0;
     }
+    __syncthreads();
+    const int total = off[kMergeBlocks], lo = off[w], hi = off[w + 1];
+    double acc = 0.0;
+    for (int b0 = 0; b0 < total; b0 += kMergeBatch) {
+        const int nb = min(kMergeBatch, total - b0);
+        if (tid < nb) {
+            int k = 0;  // the block of triplet b0 + tid
 #pragma unroll
-    for (int e = 0; e < 9; ++e) oval[9 * (size_t)u + e] = acc[e];
+            for (int step = kMergeBlocks / 2; step > 0; step >>= 1)
+                if (off[k + step] <= b0 + tid) k += step;
+            const int4 d = run[k];
+            const int q = b0 + tid - off[k];
+            ids[tid] = q < d.y ? dsorted[d.x + q] : ssorted[d.z + (q - d.y)] + sshift;
+        }
+        __syncthreads();
+        constexpr int kS = kMergeBatch / kMergeBlocks;
+        double v[kS];
+#pragma unroll
+        for (int j = 0; j < kS; ++j) v[j] = vals[9 * (size_t)ids[min(j * kMergeBlocks + w, nb - 1)] + e];
+#pragma unroll
+        for (int j = 0; j < kS; ++j) prod[9 * (j * kMergeBlocks + w) + e] = v[j];
+        __syncthreads();
+        const int last = min(hi - b0, nb);
+        for (int i = max(lo - b0, 0); i < last; ++i) acc = b0 + i == lo ? prod[9 * i + e] : acc + prod[9 * i + e];
+        __syncthreads();
+    }
+    if (u0 + w < K) oval[9 * (size_t)(u0 + w) + e] = acc;
 }
 
 __global__ void k_copy_back(int K, const int* __restrict__ r, const int* __restrict__ c,
@@ -456,7 +475,7 @@ int bcoo_convert(Ctx& c, long long nt, int nbr) {
                        (const int*)dus, (const int*)ducol, (const int*)durun, (const int*)ustart, orow, ocol, desc);
     SGIPC_LAUNCH_CHECK();
     if (K > 0) {
-        hipLaunchKernelGGL(k_merge_values, dim3(div_up(K, 256)), dim3(256), 0, s, K, (const int4*)desc,
+        hipLaunchKernelGGL(k_merge_values, dim3(div_up(K, kMergeBlocks)), dim3(kMergeT), 0, s, K, (const int4*)desc,
                            (const int*)dsorted, (const int*)P.sorted.p, (int)(s0 - P.s0), (const double*)c.t_vals,
                            oval);
         SGIPC_LAUNCH_CHECK();

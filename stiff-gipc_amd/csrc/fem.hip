@@ -458,19 +458,33 @@ __global__ void __launch_bounds__(128) k_fem_param_adjoint(int T, const double* 
     dlam[t] = s * (J - 1.0) * gc;
 }
 
-// shape[v] += sum over incident tets (ascending tet id) of the tet gradient
-__global__ void k_gather_tet_grad(int n, const int* __restrict__ inc_start, const int* __restrict__ inc_list,
-                                  const double* __restrict__ tet_grad, double* __restrict__ shape) {
-    int v = blockIdx.x * blockDim.x + threadIdx.x;
+// shape[v] += sum over incident tets (ascending tet id) of the tet gradient.
+// Three lanes a vertex, one component each; eight incidences at a time, their
+// ids, then their gradients, loaded before any is added (a loop of dependent
+// loads and adds takes two round trips per incident tet): 59 -> 40 us at 640 k tets, 16 -> 5 us
+// at 5000.
+constexpr int kGatherV = 64;  // vertices per workgroup
+__global__ void __launch_bounds__(3 * kGatherV) k_gather_tet_grad(int n, const int* __restrict__ inc_start,
+                                                                  const int* __restrict__ inc_list,
+                                                                  const double* __restrict__ tet_grad,
+                                                                  double* __restrict__ shape) {
+    const int w = threadIdx.x / 3, k = threadIdx.x - 3 * w, v = blockIdx.x * kGatherV + w;
     if (v >= n) return;
-    double g0 = shape[3 * (size_t)v], g1 = shape[3 * (size_t)v + 1], g2 = shape[3 * (size_t)v + 2];
-    int e = inc_start[v + 1];
-    for (int i = inc_start[v]; i < e; ++i) {
-        int tc = inc_list[i];
-        const double* g = tet_grad + 3 * (size_t)tc;  // 12*t + 3*corner = 3*(4t+corner)
-        g0 += g[0]; g1 += g[1]; g2 += g[2];
+    double g = shape[3 * (size_t)v + k];
+    const int end = inc_start[v + 1];
+    constexpr int U = 8;
+    for (int i = inc_start[v]; i < end; i += U) {
+        int tc[U];
+        double q[U];
+#pragma unroll
+        for (int j = 0; j < U; ++j) tc[j] = inc_list[min(i + j, end - 1)];
+#pragma unroll
+        for (int j = 0; j < U; ++j) q[j] = tet_grad[3 * (size_t)tc[j] + k];  // 12 t + 3 corner = 3 (4 t + corner)
+#pragma unroll
+        for (int j = 0; j < U; ++j)
+            if (i + j < end) g += q[j];
     }
-    shape[3 * (size_t)v] = g0; shape[3 * (size_t)v + 1] = g1; shape[3 * (size_t)v + 2] = g2;
+    shape[3 * (size_t)v + k] = g;
 }
 
 __global__ void k_kinetic(int n, const double* __restrict__ x, const double* __restrict__ xt,
@@ -544,7 +558,7 @@ void fem_assemble(Ctx& c, int T, const double* x, const uint32_t* tets, const do
                        c.t_rows + triplet_offset, c.t_cols + triplet_offset, c.tet_grad.p, c.fem_project);
     SGIPC_LAUNCH_CHECK();
     prof_end(c, PROF_FEM);
-    hipLaunchKernelGGL(k_gather_tet_grad, dim3(div_up(c.fem_n, 256)), dim3(256), 0, c.stream, c.fem_n,
+    hipLaunchKernelGGL(k_gather_tet_grad, dim3(div_up(c.fem_n, kGatherV)), dim3(3 * kGatherV), 0, c.stream, c.fem_n,
                        c.inc_start.p, c.inc_list.p, c.tet_grad.p, shape);
     SGIPC_LAUNCH_CHECK();
 }

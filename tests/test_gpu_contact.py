@@ -118,3 +118,33 @@ def test_convert_plan_reuse_is_bitexact(torch_cuda, oracle, twobox8):
         assert K == len(kr)
         assert np.array_equal(gr, kr) and np.array_equal(gc, kc)
         assert np.array_equal(gv, kv)
+
+
+@pytest.mark.parametrize("rows_used,seed", [(1, 0), (3, 1), (40, 2), (500, 3)])
+def test_convert_long_runs_are_bitexact(torch_cuda, oracle, twobox8, rows_used, seed):
+    """Merged blocks with hundreds to thousands of triplets (a workgroup sums
+    the triplets of 32 blocks in batches of 256), next to blocks with one, from
+    the contact prefix, the static segment or both: every sum in ascending
+    triplet order, bit for bit."""
+    import torch
+    from sgipc.system import NewtonSystem
+    sc, pt, ee = twobox8
+    print("case: convert long runs", rows_used, flush=True)
+    sysm = NewtonSystem(sc, "cuda:0")
+    sysm.setup_contacts(pt, ee)
+    sysm.assemble()
+    nt = 10 * sysm.T + sysm.n + sysm.n_contact_triplets
+    rng = np.random.default_rng(seed)
+    i = rng.integers(0, rows_used, nt); j = rng.integers(0, rows_used, nt)
+    lone = rng.integers(0, nt, nt // 50)                       # a few blocks of their own anywhere
+    i[lone] = rng.integers(0, sysm.n, len(lone)); j[lone] = rng.integers(0, sysm.n, len(lone))
+    R = np.minimum(i, j).astype(np.int32); Cc = np.maximum(i, j).astype(np.int32)
+    V = rng.normal(size=(nt, 9)) * 10.0 ** rng.integers(-6, 7, (nt, 1))
+    sysm.tr[:nt] = torch.tensor(R, device=sysm.tr.device)
+    sysm.tc[:nt] = torch.tensor(Cc, device=sysm.tc.device)
+    sysm.tv[:9 * nt] = torch.tensor(V.reshape(-1), device=sysm.tv.device)
+    K = sysm.convert()
+    kr, kc, kv = oracle.convert(R, Cc, V)
+    gr, gc, gv = sysm.bcoo()
+    assert K == len(kr) and np.array_equal(gr, kr) and np.array_equal(gc, kc)
+    assert np.array_equal(np.asarray(gv).reshape(-1), np.asarray(kv).reshape(-1))

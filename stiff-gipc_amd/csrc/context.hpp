@@ -68,6 +68,7 @@ struct MasState {
     DBuf<int> part_map, real_map;
     DBuf<unsigned> nstart, nnum, nlist;
     DBuf<unsigned> fine_mask, next_mask;
+    DBuf<unsigned char> outer;  // n: the vertex has a neighbour in another node of the level
     DBuf<SlotNode> slot_node;  // M
     DBuf<int> prefix0, psum0, next_prefix, next_psum;
     DBuf<int> level_size;  // 2*(L+2)

@@ -90,12 +90,50 @@ __device__ inline int decode_pair(int4 q, int node_offset, int* v) {
     return cnt;
 }
 
+// Masks ORed into global words by one workgroup: the words [base, base +
+// kOrWin) meet in LDS first, and each that gets a bit costs the workgroup one
+// read and at most one atomic.  Device-scope atomics of the eight XCDs meet in
+// memory, some 40 ns each on one line: with one a wavefront the levels of a few
+// nodes took up to 90 us at 137 k vertices.
+constexpr int kOrT = 512;
+constexpr int kOrWin = 1024;
+struct OrWindow {
+    unsigned* w;  // kOrWin words of LDS
+    int base;
+    __device__ void clear() const {
+        for (int i = threadIdx.x; i < kOrWin; i += kOrT) w[i] = 0u;
+        __syncthreads();
+    }
+    __device__ void add(unsigned* dst, int node, unsigned m) const {
+        const unsigned k = (unsigned)(node - base);
+        if (k < (unsigned)kOrWin) atomicOr(w + k, m);
+        else atomicOr(dst + node, m);
+    }
+    __device__ void flush(unsigned* dst) const {
+        __syncthreads();
+        for (int i = threadIdx.x; i < kOrWin; i += kOrT) {
+            const unsigned m = w[i];
+            if (!m) continue;
+            const unsigned cur = __hip_atomic_load(dst + base + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if ((cur | m) != cur) atomicOr(dst + base + i, m);
+        }
+    }
+};
+
 // level < 0: ids are slots and dst is indexed by vertex; else ids are the
 // level-local coarse ids from coarse_space row (level-1), dst indexed by id.
-__global__ void k_collision(int np, const int4* __restrict__ pairs, int node_offset, int n, int B, int level,
-                            const int* __restrict__ real_map, const int* __restrict__ coarse_space,
-                            unsigned* __restrict__ dst) {
-    int p = blockIdx.x * blockDim.x + threadIdx.x;
+// Coarse levels funnel many pairs onto few nodes: levels of up to kOrWin nodes
+// go through the window.  10 us a level at 137 k vertices with leader rounds of
+// a read and an atomic each, now COLLFIGURES.
+__global__ void __launch_bounds__(kOrT) k_collision(int np, const int4* __restrict__ pairs, int node_offset, int n,
+                                                    int B, int level, const int* __restrict__ ls,
+                                                    const int* __restrict__ real_map,
+                                                    const int* __restrict__ coarse_space, unsigned* __restrict__ dst) {
+    __shared__ unsigned win[kOrWin];
+    const bool few = level >= 0 && ls[2 * level] <= kOrWin;
+    const OrWindow W{win, 0};
+    if (few) W.clear();
+    const int p = blockIdx.x * blockDim.x + threadIdx.x;
     int v[4] = {-1, -1, -1, -1}, cp[4];
     int cnt = (p < np) ? decode_pair(pairs[p], node_offset, v) : 0;
 #pragma unroll
@@ -103,43 +141,33 @@ __global__ void k_collision(int np, const int4* __restrict__ pairs, int node_off
         if (i >= cnt || v[i] < 0 || v[i] >= n) cp[i] = -1;
         else cp[i] = (level < 0) ? real_map[v[i]] : coarse_space[(size_t)(level - 1) * n + v[i]];
     }
+    const int lb = __ffs(B) - 1;
     unsigned msk[4] = {0u, 0u, 0u, 0u};
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
         for (int j = i + 1; j < 4; ++j) {
             if (cp[i] < 0 || cp[j] < 0 || cp[i] == cp[j]) continue;
-            if (cp[i] / B == cp[j] / B) {
-                msk[i] |= 1u << (cp[j] % B);
-                msk[j] |= 1u << (cp[i] % B);
+            if ((cp[i] >> lb) == (cp[j] >> lb)) {
+                msk[i] |= 1u << (cp[j] & (B - 1));
+                msk[j] |= 1u << (cp[i] & (B - 1));
             }
         }
-    // Coarse levels funnel many pairs onto few nodes: merge equal targets
-    // across the wave (a few leader rounds) and skip ORs that add no bit.
+    if (few) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        int addr = (cp[i] >= 0 && msk[i] != 0u) ? (level < 0 ? v[i] : cp[i]) : -1;
-        unsigned m = msk[i];
-        unsigned long long active = __ballot(addr >= 0);
-        for (int round = 0; round < 4 && active; ++round) {
-            int leader = __ffsll((long long)active) - 1;
-            int a = __shfl(addr, leader);
-            bool same = addr >= 0 && addr == a;
-            unsigned mm = same ? m : 0u;
-#pragma unroll
-            for (int off = 32; off > 0; off >>= 1) mm |= __shfl_xor(mm, off);
-            if ((int)(threadIdx.x & 63) == leader) {
-                unsigned cur = __hip_atomic_load(dst + a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                if ((cur | mm) != cur) atomicOr(dst + a, mm);
-            }
-            active &= ~__ballot(same);
-            if (same) addr = -1;
-        }
-        if (addr >= 0) {
-            unsigned cur = __hip_atomic_load(dst + addr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if ((cur | m) != cur) atomicOr(dst + addr, m);
-        }
+        for (int i = 0; i < 4; ++i)
+            if (msk[i]) W.add(dst, cp[i], msk[i]);
+        W.flush(dst);
+        return;
     }
+    unsigned cur[4];  // the four words are read together; an OR that adds no bit is left out
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        cur[i] = msk[i] ? __hip_atomic_load(dst + (level < 0 ? v[i] : cp[i]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+                        : 0u;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        if ((cur[i] | msk[i]) != cur[i]) atomicOr(dst + (level < 0 ? v[i] : cp[i]), msk[i]);
 }
 
 // closure inside each level-0 bank, component count per bank
@@ -166,11 +194,20 @@ __global__ void __launch_bounds__(kTB) k_l0_closure(int M, int B, const int* __r
     }
 }
 
+// sizes of the next level: ls[2*(level+1)] = total comps, ls[2*(level+1)+1] =
+// begin_level + pad(count_level) (Mpad after level 0)
+__device__ inline void set_level_size(int* __restrict__ ls, int level, int total, int B, int first_begin) {
+    ls[2 * (level + 1)] = total;
+    ls[2 * (level + 1) + 1] = level == 0 ? first_begin : ls[2 * level + 1] + (ls[2 * level] + B - 1) / B * B;
+}
+
 __global__ void __launch_bounds__(kTB) k_level1(int M, int Mpad, int n, int B, const int* __restrict__ part_map,
                                                  const unsigned* __restrict__ fine_mask,
                                                  const int* __restrict__ psum0, int* __restrict__ coarse_space,
-                                                 int* __restrict__ going_next, SlotNode* __restrict__ slot_node) {
+                                                 int* __restrict__ going_next, SlotNode* __restrict__ slot_node,
+                                                 const int* __restrict__ total, int* __restrict__ ls) {
     __shared__ unsigned sel[kTB];
+    if (blockIdx.x == 0 && threadIdx.x == 0) set_level_size(ls, 0, *total, B, Mpad);
     int s = blockIdx.x * blockDim.x + threadIdx.x;
     int lane = threadIdx.x % B, bbase = threadIdx.x - lane;
     int v = (s < M) ? part_map[s] : -1;
@@ -190,53 +227,50 @@ __global__ void __launch_bounds__(kTB) k_level1(int M, int Mpad, int n, int B, c
     slot_node[s] = SlotNode{v, pre, fm, 0u};
 }
 
-__global__ void k_set_level_size(int* __restrict__ ls, int level, const int* __restrict__ total, int B,
-                                 int first_begin) {
-    // ls[2*(level+1)] = total comps, ls[2*(level+1)+1] = begin_level + pad(count_level)
-    int cnt_prev = ls[2 * level + 0];
-    int beg_prev = ls[2 * level + 1];
-    ls[2 * (level + 1) + 0] = *total;
-    ls[2 * (level + 1) + 1] = (level == 0) ? first_begin : beg_prev + (cnt_prev + B - 1) / B * B;
-}
-
 // coarse connectivity at `level` (nodes are level-local ids in coarse_space
-// row level-1).  Masks are OR-reduced across the wavefront when every lane
-// targets the same coarse node (the common case on coarse levels, where many
-// vertices share one node), and an atomic is skipped when it would add no bit.
-__global__ void k_lx_masks(int n, int B, int level, const unsigned* __restrict__ nstart,
-                           const unsigned* __restrict__ nnum, const unsigned* __restrict__ nlist,
-                           const int* __restrict__ coarse_space, unsigned* __restrict__ next_mask) {
-    int v = blockIdx.x * blockDim.x + threadIdx.x;
-    bool valid = v < n;
+// row level-1).  Vertices are numbered in bank order, so a workgroup's nodes
+// are few and close together: their masks meet in an LDS window (OrWindow)
+// that begins a little before its first vertex's node.  A vertex whose
+// neighbours are all in its own node has nothing to add on any level above:
+// `outer` marks the others, and the levels after the first look at those only.
+// Per level at 137 k vertices: 20 us with an atomic a wavefront or vertex and
+// all vertices looked at, now LXFIGURES.
+__global__ void __launch_bounds__(kOrT) k_lx_masks(int n, int B, int level, const int* __restrict__ ls,
+                                                   const unsigned* __restrict__ nstart,
+                                                   const unsigned* __restrict__ nnum,
+                                                   const unsigned* __restrict__ nlist,
+                                                   const int* __restrict__ coarse_space,
+                                                   unsigned* __restrict__ next_mask,
+                                                   unsigned char* __restrict__ outer) {
+    __shared__ unsigned win[kOrWin];
+    const int v0 = blockIdx.x * kOrT, v = v0 + threadIdx.x;
+    const bool live = v < n && (level == 1 || outer[v]);
+    if (!__syncthreads_or(live)) return;
     const int* cs = coarse_space + (size_t)(level - 1) * n;
-    int ci = valid ? cs[v] : -1;
-    unsigned msk = 0u;
-    if (valid) {
-        unsigned st = nstart[v], nn = nnum[v];
+    const OrWindow W{win, ls[2 * level] <= kOrWin ? 0 : max(0, cs[v0] - 64)};
+    W.clear();
+    if (live) {
+        const int ci = cs[v], lb = __ffs(B) - 1, bank = ci >> lb;
+        const unsigned st = nstart[v], nn = nnum[v];
+        unsigned msk = 0u;
+        bool out = false;
         for (unsigned i0 = 0; i0 < nn; i0 += kNbrBatch) {  // as in k_l0_masks
             int ids[kNbrBatch], cu[kNbrBatch];
 #pragma unroll
-            for (int k = 0; k < kNbrBatch; ++k) ids[k] = (i0 + k < nn) ? (int)nlist[st + i0 + k] : -1;
+            for (int k = 0; k < kNbrBatch; ++k) ids[k] = (i0 + k < nn) ? (int)nlist[st + i0 + k] : v;
 #pragma unroll
-            for (int k = 0; k < kNbrBatch; ++k) cu[k] = ids[k] >= 0 ? cs[ids[k]] : -1;
+            for (int k = 0; k < kNbrBatch; ++k) cu[k] = cs[ids[k]];
 #pragma unroll
             for (int k = 0; k < kNbrBatch; ++k)
-                if (ids[k] >= 0 && cu[k] / B == ci / B) msk |= 1u << (cu[k] % B);
+                if (cu[k] != ci) {
+                    out = true;
+                    if ((cu[k] >> lb) == bank) msk |= 1u << (cu[k] & (B - 1));
+                }
         }
+        if (level == 1 || !out) outer[v] = out ? 1 : 0;
+        if (msk) W.add(next_mask, ci, msk);
     }
-    int first = __shfl(ci, __ffsll((long long)__ballot(valid)) - 1);
-    bool uniform = __all(!valid || ci == first);
-    if (uniform) {
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) msk |= __shfl_xor(msk, off);
-        if ((threadIdx.x & 63) == __ffsll((long long)__ballot(valid)) - 1 && valid && msk) {
-            unsigned cur = __hip_atomic_load(next_mask + ci, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if ((cur | msk) != cur) atomicOr(next_mask + ci, msk);
-        }
-    } else if (valid && msk) {
-        unsigned cur = __hip_atomic_load(next_mask + ci, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if ((cur | msk) != cur) atomicOr(next_mask + ci, msk);
-    }
+    W.flush(next_mask);
 }
 
 __global__ void __launch_bounds__(kTB) k_lx_closure(int nmax, int B, int level, const int* __restrict__ ls,
@@ -265,7 +299,7 @@ __global__ void __launch_bounds__(kTB) k_lx_closure(int nmax, int B, int level, 
     }
 }
 
-__global__ void __launch_bounds__(kTB) k_lx_renumber(int B, int level, const int* __restrict__ ls,
+__global__ void __launch_bounds__(kTB) k_lx_renumber(int B, int level, int* ls, const int* __restrict__ total,
                                                       unsigned* __restrict__ next_mask,
                                                       const int* __restrict__ next_psum, int* __restrict__ going_next,
                                                       size_t going_cap) {
@@ -274,6 +308,7 @@ __global__ void __launch_bounds__(kTB) k_lx_renumber(int B, int level, const int
     int lane = threadIdx.x % B, bbase = threadIdx.x - lane;
     int number = ls[2 * level + 0], begin = ls[2 * level + 1];
     int pad = (number + B - 1) / B * B;
+    if (c == 0) set_level_size(ls, level, *total, B, 0);  // (this level's words are read only)
     bool valid = c < number;
     unsigned cm = valid ? next_mask[c] : 0u;
     sel[threadIdx.x] = (valid && (cm & ltmask(lane)) == 0u) ? (1u << lane) : 0u;
@@ -287,8 +322,12 @@ __global__ void __launch_bounds__(kTB) k_lx_renumber(int B, int level, const int
     if (g < going_cap) going_next[g] = pre + begin + pad;
 }
 
-__global__ void k_next_table(int n, int level, int* __restrict__ coarse_space, const unsigned* __restrict__ next_mask) {
+// node of every vertex at the next level; clears the masks of that level
+// (`clear`: the buffer the level before this one used)
+__global__ void k_next_table(int n, int level, int* __restrict__ coarse_space, const unsigned* __restrict__ next_mask,
+                             unsigned* __restrict__ clear, int nclear) {
     int v = blockIdx.x * blockDim.x + threadIdx.x;
+    if (v < nclear) clear[v] = 0u;
     if (v >= n) return;
     int nx = coarse_space[(size_t)(level - 1) * n + v];
     coarse_space[(size_t)level * n + v] = (int)next_mask[nx];
@@ -352,6 +391,7 @@ __device__ inline int project_block(int B, int li, int lj, bool same_vertex, con
 // all lanes of a wavefront would aim at the same nine words.
 constexpr int kProjWin1 = 1, kProjWin2 = 1;  // LDS window banks of levels 1 and 2
 constexpr int kProjWinBanks = kProjWin1 + kProjWin2;
+constexpr int kMaxLevels = 6;
 constexpr int kProjWinLevels = 2;
 constexpr int kProjBank16 = 136 * 9;  // doubles per packed 16-vertex bank
 constexpr int kProjTopBanks = 6;      // with the windows: 78 KB of LDS, two workgroups per CU
@@ -395,11 +435,20 @@ __global__ void __launch_bounds__(512) k_project_banked(
             double H[9];
 #pragma unroll
             for (int e = 0; e < 9; ++e) H[e] = vals[9 * (size_t)k + e];
-            const bool dom = dom2 >= 0 && node_of[2 * (size_t)n + r] == dom2 && node_of[2 * (size_t)n + c] == dom2;
+            // both nodes on every level, loaded together (a level at a time
+            // they take a round trip each)
+            int In[kMaxLevels], Jn[kMaxLevels];
+#pragma unroll
+            for (int l = 0; l < kMaxLevels; ++l) {
+                In[l] = node_of[(size_t)min(l, L - 1) * n + r];
+                Jn[l] = node_of[(size_t)min(l, L - 1) * n + c];
+            }
+            const bool dom = dom2 >= 0 && In[2] == dom2 && Jn[2] == dom2;
             const int lend = dom ? 2 : L;  // levels >= 2 of a dominant block: summed below
-            for (int l = 0; l < lend; ++l) {
-                const int I = node_of[(size_t)l * n + r], J = node_of[(size_t)l * n + c];
-                if (I / B != J / B) continue;
+#pragma unroll
+            for (int l = 0; l < kMaxLevels; ++l) {
+                const int I = In[l], J = Jn[l];
+                if (l >= lend || I / B != J / B) continue;
                 const int bank = I / B;
                 double blk[9];
                 const int pidx = project_block(B, I % B, J % B, r == c, H, blk);
@@ -600,34 +649,27 @@ __global__ void k_proj_carry(long long m, int ntiles, const unsigned* __restrict
 }
 
 // top-level bank entries = sum of the per-workgroup partials, fixed order
-// (four interleaved partial sums per entry, combined in order)
+// (four interleaved partial sums per entry, combined in order).  Each sum reads
+// 16 partials ahead of its adds: at 605 workgroups 42 us without, now TOPFIGURES.
 __global__ void __launch_bounds__(256) k_project_top_reduce(const double* __restrict__ scratch, int nwg, int len,
                                                             double* __restrict__ dst) {
     __shared__ double part[4][64];
     const int e = blockIdx.x * 64 + (threadIdx.x & 63), q = threadIdx.x >> 6;
+    constexpr int U = 16;
     double s = 0.0;
     if (e < len)
-        for (int w = q; w < nwg; w += 4) s += scratch[(size_t)w * len + e];
+        for (int w = q; w < nwg; w += 4 * U) {
+            double v[U];
+#pragma unroll
+            for (int k = 0; k < U; ++k) v[k] = scratch[(size_t)min(w + 4 * k, nwg - 1) * len + e];
+#pragma unroll
+            for (int k = 0; k < U; ++k)
+                if (w + 4 * k < nwg) s += v[k];
+        }
     part[q][threadIdx.x & 63] = s;
     __syncthreads();
     if (q == 0 && e < len) dst[e] = ((part[0][threadIdx.x] + part[1][threadIdx.x]) + part[2][threadIdx.x]) +
                                     part[3][threadIdx.x];
-}
-
-// vertex range owned by each level-1 bank (slot-ordered vertex ids)
-__global__ void k_owned_vertices(int nb0, int B, const int* __restrict__ prefix0, const int* __restrict__ psum0,
-                                 const int* __restrict__ part_map, int* __restrict__ vlo, int* __restrict__ vhi) {
-    int cb = blockIdx.x * blockDim.x + threadIdx.x;
-    if (cb >= nb0 || prefix0[cb] <= 0) return;
-    int mn = 0x7fffffff, mx = -1;
-    for (int i = 0; i < B; ++i) {
-        int v = part_map[cb * B + i];
-        if (v >= 0) { mn = min(mn, v); mx = max(mx, v); }
-    }
-    if (mx < 0) return;
-    int f = psum0[cb] / B;
-    atomicMin(vlo + f, mn);
-    atomicMax(vhi + f, mx + 1);
 }
 
 // ---- bank inverse: unpivoted in-place Gauss-Jordan in LDS -------------------
@@ -1282,15 +1324,30 @@ __global__ void __launch_bounds__(kCT) k_mas_solve_top(int L, const int* __restr
     }
 }
 
-// level-0 bank range of each level-1 bank (children of its nodes)
-__global__ void k_l1_ranges(int nb0, int B, const int* __restrict__ prefix0, const int* __restrict__ psum0,
-                            int* __restrict__ lo, int* __restrict__ hi) {
-    int cb = blockIdx.x * blockDim.x + threadIdx.x;
-    if (cb >= nb0 || prefix0[cb] <= 0) return;
-    int f = psum0[cb] / B, e = (psum0[cb] + prefix0[cb] - 1) / B;
+// level-0 bank range of each level-1 bank (children of its nodes), and the
+// vertices [vlo, vhi) of the level-0 banks whose first node it holds (vertex
+// ids in slot order); a lane per slot, one of each bank writes
+__global__ void __launch_bounds__(kTB) k_l1_ranges(int M, int B, const int* __restrict__ prefix0,
+                                                   const int* __restrict__ psum0, const int* __restrict__ part_map,
+                                                   int* __restrict__ lo, int* __restrict__ hi, int* __restrict__ vlo,
+                                                   int* __restrict__ vhi) {
+    const int s = blockIdx.x * kTB + threadIdx.x, cb = s / B;
+    const bool in = s < M;  // (M is a multiple of B)
+    const int v = in ? part_map[s] : -1, first = in ? psum0[cb] : 0, cnt = in ? prefix0[cb] : 0;
+    int mn = v >= 0 ? v : 0x7fffffff, mx = v;
+    for (int off = B / 2; off > 0; off >>= 1) {
+        mn = min(mn, __shfl_xor(mn, off));
+        mx = max(mx, __shfl_xor(mx, off));
+    }
+    if (s % B != 0 || cnt <= 0) return;
+    const int f = first / B, e = (first + cnt - 1) / B;
     for (int b = f; b <= e; ++b) {
         atomicMin(lo + b, cb);
         atomicMax(hi + b, cb + 1);
+    }
+    if (mx >= 0) {
+        atomicMin(vlo + f, mn);
+        atomicMax(vhi + f, mx + 1);
     }
 }
 
@@ -1540,7 +1597,7 @@ int num_levels(int nn, int B) {
         levelSz = (levelSz + B - 1) / B * B;
     }
     nLevel = nLevel + 1;
-    return nLevel > 6 ? 6 : nLevel;
+    return nLevel > kMaxLevels ? kMaxLevels : nLevel;
 }
 
 template <typename V, typename T>
@@ -1628,7 +1685,8 @@ void mas_set_topology(Ctx& c, int n, int node_offset, const unsigned* nstart, co
     if (nlist_len) SGIPC_HIP(hipMemcpy(m.nlist.p, nlist, sizeof(unsigned) * nlist_len, hipMemcpyHostToDevice));
     m.fine_mask.reserve((size_t)n + 1);
     m.slot_node.reserve((size_t)M + 1);
-    m.next_mask.reserve((size_t)n + bank + 1);
+    m.next_mask.reserve(2 * ((size_t)n + bank));
+    m.outer.reserve((size_t)n + 1);
     size_t nbk = (size_t)std::max(M, n) / bank + 2;
     m.prefix0.reserve(nbk);
     m.psum0.reserve(nbk + 1);
@@ -1667,15 +1725,18 @@ void mas_build(Ctx& c, int sub_offset, int sub_nb, const int* pairs, int npairs)
                                         l1hi, vlo, vhi, m.fine_mask.p, m.comp_mask.p, m.slot_node.p, m.going_cap}));
         SGIPC_LAUNCH_CHECK();
     } else {
-        fill<int>(ls, 0, 2LL * (L + 2), s);
-        fill<int>(m.going_next.p, 0, (long long)m.going_cap, s);
+        // the masks of a level: two buffers, the next level's cleared while this one's is read
+        const size_t mask_len = (size_t)n + B;
+        FillRanges f;
+        f.add(ls, 0u, 2LL * (L + 2)).add(m.going_next.p, 0u, (long long)m.going_cap);
+        fill_ranges(f.add(m.next_mask.p, 0u, (long long)mask_len), s);
         // level 0
         hipLaunchKernelGGL(k_l0_masks, dim3(div_up(M, 256)), dim3(256), 0, s, M, B, m.part_map.p, m.real_map.p, m.nstart.p,
                            m.nnum.p, m.nlist.p, m.fine_mask.p);
         SGIPC_LAUNCH_CHECK();
         if (npairs > 0) {
-            hipLaunchKernelGGL(k_collision, dim3(div_up(npairs, 256)), dim3(256), 0, s, npairs, (const int4*)pairs,
-                               m.node_offset, n, B, -1, m.real_map.p, m.coarse_space.p, m.fine_mask.p);
+            hipLaunchKernelGGL(k_collision, dim3(div_up(npairs, kOrT)), dim3(kOrT), 0, s, npairs, (const int4*)pairs,
+                               m.node_offset, n, B, -1, ls, m.real_map.p, m.coarse_space.p, m.fine_mask.p);
             SGIPC_LAUNCH_CHECK();
         }
         hipLaunchKernelGGL(k_l0_closure, dim3(div_up(M, kTB)), dim3(kTB), 0, s, M, B, m.part_map.p, m.fine_mask.p,
@@ -1683,34 +1744,31 @@ void mas_build(Ctx& c, int sub_offset, int sub_nb, const int* pairs, int npairs)
         SGIPC_LAUNCH_CHECK();
         int* tot = c.dev_int.reserve(8);
         exclusive_scan(c, m.prefix0.p, m.psum0.p, M / B, tot + 6, s);
-        hipLaunchKernelGGL(k_set_level_size, dim3(1), dim3(1), 0, s, ls, 0, tot + 6, B, Mpad);
-        SGIPC_LAUNCH_CHECK();
         hipLaunchKernelGGL(k_level1, dim3(div_up(M, kTB)), dim3(kTB), 0, s, M, Mpad, n, B, m.part_map.p, m.fine_mask.p,
-                           m.psum0.p, m.coarse_space.p, m.going_next.p, m.slot_node.p);
+                           m.psum0.p, m.coarse_space.p, m.going_next.p, m.slot_node.p, (const int*)(tot + 6), ls);
         SGIPC_LAUNCH_CHECK();
         const int nmax = n;  // level-local node count never exceeds n
         for (int level = 1; level < L; ++level) {
-            fill<unsigned>(m.next_mask.p, 0u, (long long)nmax + B, s);
-            hipLaunchKernelGGL(k_lx_masks, dim3(div_up(n, 256)), dim3(256), 0, s, n, B, level, m.nstart.p, m.nnum.p,
-                               m.nlist.p, m.coarse_space.p, m.next_mask.p);
+            unsigned* next = m.next_mask.p + (level & 1 ? 0 : mask_len);
+            unsigned* other = m.next_mask.p + (level & 1 ? mask_len : 0);
+            hipLaunchKernelGGL(k_lx_masks, dim3(div_up(n, kOrT)), dim3(kOrT), 0, s, n, B, level, ls, m.nstart.p, m.nnum.p,
+                               m.nlist.p, m.coarse_space.p, next, m.outer.p);
             SGIPC_LAUNCH_CHECK();
             if (npairs > 0) {
-                hipLaunchKernelGGL(k_collision, dim3(div_up(npairs, 256)), dim3(256), 0, s, npairs, (const int4*)pairs,
-                                   m.node_offset, n, B, level, m.real_map.p, m.coarse_space.p, m.next_mask.p);
+                hipLaunchKernelGGL(k_collision, dim3(div_up(npairs, kOrT)), dim3(kOrT), 0, s, npairs, (const int4*)pairs,
+                                   m.node_offset, n, B, level, ls, m.real_map.p, m.coarse_space.p, next);
                 SGIPC_LAUNCH_CHECK();
             }
             int nbk = div_up(nmax, B);
             hipLaunchKernelGGL(k_lx_closure, dim3(div_up((long long)nbk * B, kTB)), dim3(kTB), 0, s, nbk * B, B, level, ls,
-                               m.next_mask.p, m.next_prefix.p, m.comp_mask.p);
+                               next, m.next_prefix.p, m.comp_mask.p);
             SGIPC_LAUNCH_CHECK();
             exclusive_scan(c, m.next_prefix.p, m.next_psum.p, nbk, tot + 6, s);
-            hipLaunchKernelGGL(k_set_level_size, dim3(1), dim3(1), 0, s, ls, level, tot + 6, B, 0);
-            SGIPC_LAUNCH_CHECK();
             hipLaunchKernelGGL(k_lx_renumber, dim3(div_up((long long)nbk * B, kTB)), dim3(kTB), 0, s, B, level, ls,
-                               m.next_mask.p, m.next_psum.p, m.going_next.p, m.going_cap);
+                               (const int*)(tot + 6), next, m.next_psum.p, m.going_next.p, m.going_cap);
             SGIPC_LAUNCH_CHECK();
-            hipLaunchKernelGGL(k_next_table, dim3(div_up(n, 256)), dim3(256), 0, s, n, level, m.coarse_space.p,
-                               m.next_mask.p);
+            hipLaunchKernelGGL(k_next_table, dim3(div_up((long long)mask_len, 256)), dim3(256), 0, s, n, level,
+                               m.coarse_space.p, (const unsigned*)next, other, (int)mask_len);
             SGIPC_LAUNCH_CHECK();
         }
         hipLaunchKernelGGL(k_aggregate, dim3(div_up(n, 256)), dim3(256), 0, s, n, L, m.real_map.p, m.going_next.p,
@@ -1750,11 +1808,8 @@ void mas_build(Ctx& c, int sub_offset, int sub_nb, const int* pairs, int npairs)
             fill_ranges(f, s);
             fill_ranges(g, s);
             if (nb0 > 0) {
-                hipLaunchKernelGGL(k_l1_ranges, dim3(div_up(nb0, 256)), dim3(256), 0, s, nb0, B, m.prefix0.p,
-                                   m.psum0.p, l1lo, l1hi);
-                SGIPC_LAUNCH_CHECK();
-                hipLaunchKernelGGL(k_owned_vertices, dim3(div_up(nb0, 256)), dim3(256), 0, s, nb0, B, m.prefix0.p,
-                                   m.psum0.p, m.part_map.p, vlo, vhi);
+                hipLaunchKernelGGL(k_l1_ranges, dim3(div_up(M, kTB)), dim3(kTB), 0, s, M, B, m.prefix0.p, m.psum0.p,
+                                   m.part_map.p, l1lo, l1hi, vlo, vhi);
                 SGIPC_LAUNCH_CHECK();
             }
         }

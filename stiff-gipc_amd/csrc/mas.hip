@@ -123,8 +123,8 @@ struct OrWindow {
 // level < 0: ids are slots and dst is indexed by vertex; else ids are the
 // level-local coarse ids from coarse_space row (level-1), dst indexed by id.
 // Coarse levels funnel many pairs onto few nodes: levels of up to kOrWin nodes
-// go through the window.  10 us a level at 137 k vertices with leader rounds of
-// a read and an atomic each, now COLLFIGURES.
+// go through the window.  9.9 us a level at 137 k vertices with leader rounds of
+// a read and an atomic each, now 4.4.
 __global__ void __launch_bounds__(kOrT) k_collision(int np, const int4* __restrict__ pairs, int node_offset, int n,
                                                     int B, int level, const int* __restrict__ ls,
                                                     const int* __restrict__ real_map,
@@ -234,7 +234,8 @@ __global__ void __launch_bounds__(kTB) k_level1(int M, int Mpad, int n, int B, c
 // neighbours are all in its own node has nothing to add on any level above:
 // `outer` marks the others, and the levels after the first look at those only.
 // Per level at 137 k vertices: 20 us with an atomic a wavefront or vertex and
-// all vertices looked at, now LXFIGURES.
+// all vertices looked at, now 10 (workgroups of 1024 the same; at 44 k vertices,
+// 43 workgroups then, 10.9 against 7.7).
 __global__ void __launch_bounds__(kOrT) k_lx_masks(int n, int B, int level, const int* __restrict__ ls,
                                                    const unsigned* __restrict__ nstart,
                                                    const unsigned* __restrict__ nnum,
@@ -391,7 +392,6 @@ __device__ inline int project_block(int B, int li, int lj, bool same_vertex, con
 // all lanes of a wavefront would aim at the same nine words.
 constexpr int kProjWin1 = 1, kProjWin2 = 1;  // LDS window banks of levels 1 and 2
 constexpr int kProjWinBanks = kProjWin1 + kProjWin2;
-constexpr int kMaxLevels = 6;
 constexpr int kProjWinLevels = 2;
 constexpr int kProjBank16 = 136 * 9;  // doubles per packed 16-vertex bank
 constexpr int kProjTopBanks = 6;      // with the windows: 78 KB of LDS, two workgroups per CU
@@ -435,20 +435,11 @@ __global__ void __launch_bounds__(512) k_project_banked(
             double H[9];
 #pragma unroll
             for (int e = 0; e < 9; ++e) H[e] = vals[9 * (size_t)k + e];
-            // both nodes on every level, loaded together (a level at a time
-            // they take a round trip each)
-            int In[kMaxLevels], Jn[kMaxLevels];
-#pragma unroll
-            for (int l = 0; l < kMaxLevels; ++l) {
-                In[l] = node_of[(size_t)min(l, L - 1) * n + r];
-                Jn[l] = node_of[(size_t)min(l, L - 1) * n + c];
-            }
-            const bool dom = dom2 >= 0 && In[2] == dom2 && Jn[2] == dom2;
+            const bool dom = dom2 >= 0 && node_of[2 * (size_t)n + r] == dom2 && node_of[2 * (size_t)n + c] == dom2;
             const int lend = dom ? 2 : L;  // levels >= 2 of a dominant block: summed below
-#pragma unroll
-            for (int l = 0; l < kMaxLevels; ++l) {
-                const int I = In[l], J = Jn[l];
-                if (l >= lend || I / B != J / B) continue;
+            for (int l = 0; l < lend; ++l) {
+                const int I = node_of[(size_t)l * n + r], J = node_of[(size_t)l * n + c];
+                if (I / B != J / B) continue;
                 const int bank = I / B;
                 double blk[9];
                 const int pidx = project_block(B, I % B, J % B, r == c, H, blk);
@@ -650,7 +641,7 @@ __global__ void k_proj_carry(long long m, int ntiles, const unsigned* __restrict
 
 // top-level bank entries = sum of the per-workgroup partials, fixed order
 // (four interleaved partial sums per entry, combined in order).  Each sum reads
-// 16 partials ahead of its adds: at 605 workgroups 42 us without, now TOPFIGURES.
+// 16 partials ahead of its adds: at 605 workgroups 42 us without, now 9.
 __global__ void __launch_bounds__(256) k_project_top_reduce(const double* __restrict__ scratch, int nwg, int len,
                                                             double* __restrict__ dst) {
     __shared__ double part[4][64];
@@ -1597,7 +1588,7 @@ int num_levels(int nn, int B) {
         levelSz = (levelSz + B - 1) / B * B;
     }
     nLevel = nLevel + 1;
-    return nLevel > kMaxLevels ? kMaxLevels : nLevel;
+    return nLevel > 6 ? 6 : nLevel;
 }
 
 template <typename V, typename T>

@@ -528,12 +528,11 @@ def main():
     g = os.environ.get("SGIPC_SPMV_G", "8")
     g = g if g in ("4", "8", "16") else "8"   # lanes per block row, as the library reads it
     full32 = os.environ.get("SGIPC_SPMV_FULL32", "1") != "0"   # the library's default for mixed solves
-    if fp32 and full32:
-        kname = "k_spmv_pap_full<%s, float> (PCG SpMV + direction update, row-contiguous FP32 copy)" % g
-    elif fp32:
+    if fp32 and not full32:
         kname = "k_spmv_pap<%s, float, float> (PCG SpMV + direction update, FP32 upper BCOO)" % g
     else:
-        kname = "k_spmv_pap<%s, double, double> (PCG SpMV + direction update, FP64)" % g
+        kname = "k_spmv_pap_full<%s> (PCG SpMV + direction update, grouped copy of both triangles)" % \
+            ("float" if fp32 else "double")
     out = {
         "metric": "Newton solves/sec (assembly + BCOO convert + MAS build + MAS-PCG to 1e-6 true rel. residual)",
         "value": round(r["value"], 4),
@@ -653,8 +652,8 @@ def hybrid(a):
     g = os.environ.get("SGIPC_SPMV_G", "8")
     g = g if g in ("4", "8", "16") else "8"
     full32 = os.environ.get("SGIPC_SPMV_FULL32", "1") != "0"
-    kname = (("k_spmv_pap_full<%s, float>" if full32 else "k_spmv_pap<%s, float, float>") % g) if fp32 else \
-        ("k_spmv_pap<%s, double, double>" % g)
+    kname = "k_spmv_pap<%s, float, float>" % g if fp32 and not full32 else \
+        "k_spmv_pap_full<%s>" % ("float" if fp32 else "double")
     cpu = None
     if not a.no_cpu_baseline:
         sys.path.insert(0, os.path.join(ROOT, "oracle"))

@@ -82,7 +82,7 @@ struct MasState {
     DBuf<int> coarse_table;  // 6*n (itable layout)
     DBuf<int> node_of;       // L*n : global node id of vertex at level l (l=0: slot)
     DBuf<double> bank_upper; // nbanks * npack * 9 (Galerkin, packed upper, col-major blocks)
-    DBuf<double> inv64;      // nbanks * D(D+1)/2 symmetric inverse, upper triangle packed by rows (FP64)
+    DBuf<double> inv64;      // nbanks * D(D+1)/2 symmetric inverse (FP64), in the order of inv_index (bank_solve.hpp)
     DBuf<float> inv32;       // same, FP32
     bool inv64_ok = true;    // inv64 holds the FP64 inverses (not after an FP32-only build)
     DBuf<unsigned short> inv16;  // half storage: S = D^-1 inv D^-1 as FP16 bits, packed like inv64

@@ -288,3 +288,54 @@ def test_zero_rhs_returns_zero(torch_cuda, cube10, mode):
     st2 = sys_.solve(tol=1e-6, stop_rule=1, max_iter=5000, precision=prec)
     assert st2.converged and st2.iterations == ref.iterations
     assert torch_cuda.equal(sys_.dx, x_ref)
+
+
+@pytest.mark.parametrize("cells,hub,mixed", [(1, 7, False), (3, 60, False), (4, 100, True), (10, 1300, False),
+                                             (10, 1300, True), (16, 4500, True), (16, 4500, False)])
+def test_solve_with_rows_of_thousands_of_entries(torch_cuda, cells, hub, mixed):
+    """The SpMV by entries: rows that cross chunk groups of 64 entries and LDS
+    batches of 1024, next to rows with only their diagonal, in systems of one
+    chunk and of many.  A strictly diagonally dominant arrow matrix (dominance
+    2, so the error is at most about the relative residual): solved to 1e-9
+    (FP64) or 1e-6 (FP32 inner solves), compared at ten times that."""
+    import scipy.sparse as sp
+    import scipy.sparse.linalg as spla
+    from sgipc import capi, scene
+    print("case: arrow matrix", cells, hub, mixed, flush=True)
+    sc = scene.cube_scene(cells, seed=2)
+    s = make_system(sc, capi.PRECOND_MAS_FP32 if mixed else capi.PRECOND_MAS)
+    s.assemble()
+    n, rng = sc.n, np.random.default_rng(cells)
+    nt = 10 * s.T + s.n
+    hubs = [0, n // 2] if n > 100 else [0]                     # rows with `hub` couplings each
+    off = {}
+    for h in hubs:
+        for v in rng.choice(n, size=min(hub, n - 1), replace=False):
+            if v != h and len(off) < nt - n:
+                off[(min(h, v), max(h, v))] = 0.5 * rng.normal(size=(3, 3)) / 3
+    A = sp.lil_matrix((3 * n, 3 * n))
+    sums = np.zeros(n)
+    for (i, j), M in off.items():
+        A[3 * i:3 * i + 3, 3 * j:3 * j + 3] = M; A[3 * j:3 * j + 3, 3 * i:3 * i + 3] = M.T
+        w = np.abs(M).sum(); sums[i] += w; sums[j] += w
+    R = [i for i, _ in off] + list(range(n)); Cc = [j for _, j in off] + list(range(n))
+    V = [M.T.reshape(-1) for M in off.values()] + [((1 + 2 * sums[v]) * np.eye(3)).reshape(-1) for v in range(n)]
+    for v in range(n):
+        A[3 * v:3 * v + 3, 3 * v:3 * v + 3] = (1 + 2 * sums[v]) * np.eye(3)
+    k = len(R)
+    R += [0] * (nt - k); Cc += [0] * (nt - k); V += [np.zeros(9)] * (nt - k)    # (the store's count is fixed)
+    dev = s.tr.device
+    s.tr[:nt] = torch_cuda.tensor(np.array(R, np.int32), device=dev)
+    s.tc[:nt] = torch_cuda.tensor(np.array(Cc, np.int32), device=dev)
+    s.tv[:9 * nt] = torch_cuda.tensor(np.array(V).reshape(-1), device=dev)
+    s.convert(); s.build_precond()
+    b = s.b.cpu().numpy()
+    tol = 1e-6 if mixed else 1e-9
+    st = s.solve(tol=tol, stop_rule=capi.STOP_TRUE_REL, max_iter=2000,
+                 precision=capi.PRECISION_MIXED if mixed else capi.PRECISION_FP64)
+    x = s.dx.cpu().numpy()
+    A = A.tocsc()
+    assert st.converged and np.linalg.norm(b - A @ x) <= 1.5 * tol * np.linalg.norm(b)
+    d = A.diagonal()
+    xs = spla.spsolve(A, b)
+    assert np.abs(d * (x - xs)).max() <= 10 * tol * np.linalg.norm(b)

@@ -106,3 +106,21 @@ def test_newton_step_same_bits_with_either_sort(torch_cuda):
     assert len(a[0]) > 0 and a[5] == b[5]
     for u, v in zip(a[:5], b[:5]):
         assert np.array_equal(u, v)
+
+
+@pytest.mark.parametrize("key_bytes,n", [(4, 262143), (4, 262144), (4, 262145), (4, 524288 - 1), (4, 524288 + 2049),
+                                         (8, 262144 + 1023), (8, 524288), (8, 524288 + 4097)])
+def test_own_sort_at_tile_size_limits(torch_cuda, ctx, key_bytes, n):
+    """Tiles of 1024, 2048 and 4096 keys: just below and above the counts where
+    the tile size changes; stable, so equal to numpy's stable sort exactly."""
+    from sgipc import capi
+    torch = torch_cuda
+    print("case: sort tile limit n=%d key_bytes=%d" % (n, key_bytes), flush=True)
+    rng = np.random.default_rng(n)
+    k = rng.integers(0, 1 << 20, size=n).astype(np.uint32 if key_bytes == 4 else np.uint64)
+    vals = np.arange(n, dtype=np.int32)
+    tk = torch.tensor(k.view(np.int32 if key_bytes == 4 else np.int64), device="cuda:0")
+    ko, vo = _sort(ctx, torch, tk, torch.tensor(vals, device="cuda:0"), 20, capi.SORT_OWN)
+    o = np.argsort(k, kind="stable")
+    assert np.array_equal(vo.cpu().numpy(), vals[o])
+    assert np.array_equal(ko.cpu().numpy().view(k.dtype), k[o])

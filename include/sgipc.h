@@ -326,7 +326,12 @@ int sgipc_precond_build(sgipc_ctx* ctx, int kind, int sub_offset, int sub_nb,
                         const int* d_pairs, int n_pairs);
 /* z = M^-1 r; MASPreconditioner::preconditioning (MASPreconditioner.cu:2221-2262) */
 int sgipc_precond_apply(sgipc_ctx* ctx, const double* d_r, double* d_z);
-/* PCG solve of A x = b; PCGSolver::solve (linear_system/solver/pcg_solver.cu:158-267) */
+/* PCG solve of A x = b; PCGSolver::solve (linear_system/solver/pcg_solver.cu:158-267).
+ * The converted values stay in the caller's triplet store: every solve takes A
+ * (sgipc_spmv too) from them as they are at the call, so a shift or scaling
+ * written there needs no other convert (the preconditioner stays as built).
+ * SGIPC_PRECISION_MIXED iterates on an FP32 copy made by the first mixed solve
+ * after a convert and refines on the residual of the current values. */
 int sgipc_solve(sgipc_ctx* ctx, const double* d_b, double* d_x, const sgipc_solve_opts* opts,
                 sgipc_solve_stats* stats);
 

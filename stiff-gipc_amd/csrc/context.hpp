@@ -30,7 +30,7 @@ struct SymBcoo {
     // column, in groups of 64 entries (FullCopy in spmv_sym.hpp)
     DBuf<float> full32;
     DBuf<double> full64;
-    bool full32_ok = false, full64_ok = false;
+    bool full32_ok = false;  // (full64 is made anew by every solve)
 };
 
 // Sort of the static (FEM + mass) triplet segment, built where it started at
@@ -312,8 +312,8 @@ double ground_step_bound(Ctx& c, int m, const unsigned* ids, const double* x, co
 int bcoo_convert(Ctx& c, long long nt, int nblockrows);
 void bsr_build(Ctx& c);
 const float* bsr_values_f32(Ctx& c);
-const float* bsr_full(Ctx& c, float);    // both triangles in entry order, FP32
-const double* bsr_full(Ctx& c, double);  // the same in FP64
+const float* bsr_full(Ctx& c, float);    // both triangles in entry order, FP32 (as converted)
+const double* bsr_full(Ctx& c, double);  // the same in FP64, of the values as they are now
 void spmv64(Ctx& c, double a, const double* x, double b, double* y);
 
 double kinetic_energy(Ctx& c, int n, const double* x, const double* xt, const double* m);

@@ -165,31 +165,38 @@ void bsr_build(Ctx& c) {
                        (const int2*)lref, (const int*)c.uniq_start.p, (const int*)c.t_cols, eptr, ent);
     SGIPC_LAUNCH_CHECK();
     S.valf_ok = false;
-    S.full32_ok = S.full64_ok = false;
+    S.full32_ok = false;
     c.have_bsr = true;
 }
 
 template <typename T>
-static const T* full_copy(Ctx& c, DBuf<T>& buf, bool& ok) {
+static const T* full_copy(Ctx& c, DBuf<T>& buf) {
     SymBcoo& S = c.bsr;
-    // 2K bounds the entries (lower references + upper blocks); whole groups of 64
+    // 2K bounds the entries (lower references + upper blocks; how many blocks
+    // lie on the diagonal only the device knows); whole groups of 64
     T* vf = buf.reserve(((2 * (size_t)S.K + 63) / 64 + 1) * FullCopy<T>::kGroup);
-    if (!ok && S.nb > 0 && S.K > 0) {
+    if (S.nb > 0 && S.K > 0) {
         const int blocks = 8 * std::max(1, std::min((int)div_up(2LL * S.K, 8 * 256), 1024));
         hipLaunchKernelGGL(k_full_copy<T>, dim3(blocks), dim3(256), 0, c.stream, S.nb, (const int*)S.eptr.p,
                            (const int2*)S.ent.p, (const int*)c.t_cols, (const double*)c.t_vals, vf);
         SGIPC_LAUNCH_CHECK();
     }
-    ok = true;
     return vf;
 }
+// Kept until the next convert: the mixed solves' refinement takes its residuals
+// from the converted values themselves.
 const float* bsr_full(Ctx& c, float) {
     if (!c.have_bsr) bsr_build(c);
-    return full_copy<float>(c, c.bsr.full32, c.bsr.full32_ok);
+    SymBcoo& S = c.bsr;
+    if (!S.full32_ok) full_copy<float>(c, S.full32);
+    S.full32_ok = true;
+    return S.full32.p;
 }
+// Made anew by every solve: the values are the caller's, who may have written to
+// them since (nothing else of an FP64 solve would notice).
 const double* bsr_full(Ctx& c, double) {
     if (!c.have_bsr) bsr_build(c);
-    return full_copy<double>(c, c.bsr.full64, c.bsr.full64_ok);
+    return full_copy<double>(c, c.bsr.full64);
 }
 
 // FP32 copy of the BCOO values for the mixed-precision solve

@@ -4,9 +4,11 @@
 // warp row sums plus FP64 atomics for the transposed half).  Here a group of
 // G lanes owns one block row j and sums, in a fixed order, the transposed
 // references A(i,j)^T x_i (i < j) and then the row's own upper blocks
-// A(j,k) x_k, both listed in one per-row entry array.  The values are read in place from the converted BCOO
-// (9 doubles per block, column-major): no atomics, no second copy of the
-// matrix, deterministic.
+// A(j,k) x_k, both listed in one per-row entry array: no atomics,
+// deterministic.  y = a A x + b y, the residuals and the FP64 batched solves
+// read the values in place from the converted BCOO (9 doubles per block,
+// column-major); the single-system PCG, and mixed batched solves, read a copy of
+// both triangles in entry order (FullCopy below).
 #pragma once
 #include "context.hpp"
 

@@ -339,3 +339,31 @@ def test_solve_with_rows_of_thousands_of_entries(torch_cuda, cells, hub, mixed):
     d = A.diagonal()
     xs = spla.spsolve(A, b)
     assert np.abs(d * (x - xs)).max() <= 10 * tol * np.linalg.norm(b)
+
+
+@pytest.mark.parametrize("kind", [0, 1, 2, 3])
+def test_fp64_solve_follows_values_edited_in_place(torch_cuda, cube4, kind):
+    """The converted values live in the caller's store: a diagonal shift or a
+    scaling written there between two solves is the matrix of the next one,
+    without another convert.  Every solve reaches 1e-9 of the matrix as it then
+    is, by the reported residual (half a digit of slack for the recurrence's
+    own drift) and by numpy's."""
+    print("case: values edited in place, precond", kind, flush=True)
+    s = make_system(cube4, kind)
+    s.assemble(); s.convert(); s.build_precond()
+    kr, kc, kv = s.bcoo()
+    diag = torch_cuda.tensor(np.flatnonzero(kr == kc), device=s.dev)
+    v = s.tv[:9 * s.K].view(s.K, 9)
+    shift = float(np.abs(kv[kr == kc][:, [0, 4, 8]]).mean())
+    b = s.b.cpu().numpy()
+    for step in range(4):
+        if step == 3:
+            v *= 0.5
+        elif step:
+            for e in (0, 4, 8):
+                v[diag, e] += shift * step
+        st = s.solve(tol=1e-9, stop_rule=1, max_iter=5000)
+        A = dense_from_bcoo(*s.bcoo(), cube4.n)
+        x = s.dx.cpu().numpy()
+        res = np.linalg.norm(A @ x - b) / np.linalg.norm(b)
+        assert st.converged and res <= 3e-9 and st.rel_residual <= 3e-9, (step, res, st.rel_residual)

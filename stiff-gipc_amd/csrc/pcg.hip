@@ -321,8 +321,9 @@ __global__ void __launch_bounds__(kFT) k_spmv_pap_full(int nb, int R, int nchunk
         const int e0 = er[0], e1 = er[nr];
         const int lo = mine ? er[row] : 0, hi = mine ? er[row + 1] : 0;
         V s0 = 0, s1 = 0, s2 = 0, s3 = 0;
-        // batches start at a whole group of 64 entries
-        for (int b0 = e0 & ~63; b0 < e1; b0 += kFBatch) {
+        // batches start at a whole group of 64 entries; rows without triplets
+        // can leave a chunk with no entry (e0 == e1), where there is none to clamp to
+        for (int b0 = e0 < e1 ? e0 & ~63 : e1; b0 < e1; b0 += kFBatch) {
             // (an index outside the chunk's run is clamped to it; a wavefront
             // past the run does nothing)
 #pragma unroll

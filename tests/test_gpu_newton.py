@@ -1,5 +1,7 @@
 """GPU parity of the HIP Newton-step path against the CPU oracle, through the
 C ABI (libsgipc.so).  Inputs are the seeded synthetic cube scenes."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -367,3 +369,51 @@ def test_fp64_solve_follows_values_edited_in_place(torch_cuda, cube4, kind):
         x = s.dx.cpu().numpy()
         res = np.linalg.norm(A @ x - b) / np.linalg.norm(b)
         assert st.converged and res <= 3e-9 and st.rel_residual <= 3e-9, (step, res, st.rel_residual)
+
+
+_TRAILING = [[125, 126, 127, 128], list(range(125, 136)), list(range(125, 145))]
+_AMONG = [list(range(64, 88)), [0, 1, 2, 3, 4, 5, 6, 7, 140]]
+
+
+@pytest.mark.parametrize("mixed", [False, True])
+@pytest.mark.parametrize("kind,empty", [(k, e) for k in (0, 1) for e in _TRAILING + _AMONG] +
+                         [(2, e) for e in _TRAILING])
+def test_solve_with_rows_without_triplets(torch_cuda, oracle, cube4, kind, mixed, empty):
+    """Block rows that no triplet names, at the end of the system (so that the
+    SpMV's last chunk of eight rows has no entry, one alone or several rows), in
+    whole chunks of the middle and at the front: they stay zero and the others
+    solve the system without them.  (MAS covers the leading rows only, so it is
+    run where the empty ones follow.)"""
+    from sgipc import capi
+    from sgipc.system import _p
+    print("case: rows without triplets", kind, mixed, len(empty), empty[0], flush=True)
+    n = cube4.n
+    ref = oracle_system(oracle, cube4)
+    nb = max(n + len(empty), empty[-1] + 1)
+    rows = np.array([r for r in range(nb) if r not in set(empty)])[:n]      # new row of each old one
+    s = make_system(cube4, kind)
+    R, Cc, V = ref["trip"]
+    nt = len(R)
+    s.tr[:nt] = torch_cuda.tensor(rows[R].astype(np.int32), device=s.dev)
+    s.tc[:nt] = torch_cuda.tensor(rows[Cc].astype(np.int32), device=s.dev)
+    s.tv[:9 * nt] = torch_cuda.tensor(V.reshape(-1), dtype=torch_cuda.float64, device=s.dev)
+    K = C.c_int(0)
+    s.ctx.call("sgipc_convert", nt, nb, C.byref(K))
+    kr, kc, kv = ref["bcoo"]
+    entries = 2 * K.value - n                                               # every old row has its diagonal
+    assert K.value == len(kr) and entries % 64 != 0
+    s.ctx.call("sgipc_precond_build", kind, 0, n if kind == 2 else nb, None, 0)
+    b = np.zeros((nb, 3))
+    b[rows] = ref["b"].reshape(n, 3)
+    bt = torch_cuda.tensor(b.reshape(-1), device=s.dev)
+    xt = torch_cuda.full_like(bt, 7.0)
+    tol = 1e-6 if mixed else 1e-9
+    o = capi.SolveOpts(capi.PRECISION_MIXED if mixed else capi.PRECISION_FP64, capi.STOP_TRUE_REL, tol, 0.3, 5000, 8)
+    st = capi.SolveStats()
+    s.ctx.call("sgipc_solve", _p(bt), _p(xt), C.byref(o), C.byref(st))
+    x = xt.cpu().numpy().reshape(nb, 3)
+    assert not np.any(np.delete(x, rows, axis=0))
+    A = dense_from_bcoo(kr, kc, kv, n)
+    res = np.linalg.norm(A @ x[rows].reshape(-1) - ref["b"]) / np.linalg.norm(ref["b"])
+    # the FP64 recurrence's residual drifts from the true one by rounding (half a digit of slack)
+    assert st.converged and res <= 3 * tol and st.rel_residual <= 3 * tol, (res, st.rel_residual)

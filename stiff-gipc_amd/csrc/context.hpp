@@ -98,6 +98,30 @@ struct MasState {
     DBuf<int> sub_index;     // BCOO block indices in the subsystem range
 };
 
+// First bank of level 3: the fused bank solves leave it and the ones after it to
+// the workgroup that restricts them (all banks are below it with three levels)
+inline int mas_top_bank0(const MasState& m) { return m.L >= 4 ? m.level_size_h[7] / m.bank : m.nbanks; }
+
+// Key of a captured graph: whatever its launches were given, so that a replay is
+// the launch sequence of the call at hand
+struct GraphKey {
+    size_t h = 1469598103934665603ull;
+    void mix(size_t v) { h ^= v + 0x9e3779b97f4a7c15ull + (h << 6) + (h >> 2); }
+    void mix(const void* p) { mix(reinterpret_cast<size_t>(p)); }
+    // The MAS tables and the counts that shape their launches.  mas_top_bank0
+    // among them: with equal totals another contact set can move banks between
+    // level 2 and the levels above.
+    void mix(const MasState& m) {
+        for (int v : {m.nbanks, m.L, m.M, m.n, m.bank, m.nb1, mas_top_bank0(m), (int)m.inv16_ok}) mix((size_t)v);
+        for (const void* p : {(const void*)m.going_next.p, (const void*)m.node_of.p, (const void*)m.level_size.p,
+                              (const void*)m.l1lo.p, (const void*)m.l1hi.p, (const void*)m.comp_mask.p,
+                              (const void*)m.slot_node.p, (const void*)m.inv64.p, (const void*)m.inv32.p,
+                              (const void*)m.inv16.p, (const void*)m.inv16_d.p, (const void*)m.R64.p,
+                              (const void*)m.R32.p, (const void*)m.Z64.p, (const void*)m.Z32.p})
+            mix(p);
+    }
+};
+
 struct PcgGraph {
     hipGraphExec_t exec = nullptr;      // a group of two iterations
     hipGraphExec_t exec_big = nullptr;  // a longer group (single-system PCG), same key

@@ -1997,7 +1997,7 @@ void mas_update_restrict(Ctx& c, double* x, float* r, const float* p, const floa
 template <typename T, bool H>
 static void solve_top_t(Ctx& c, const void* inv, const float* dsc, T* R, T* Z, const int* ctrl, SceneSkip skip) {
     MasState& m = c.mas;
-    const int top_bank0 = m.L >= 4 ? m.level_size_h[7] / m.bank : m.nbanks;
+    const int top_bank0 = mas_top_bank0(m);
     prof_begin(c, PROF_MAS_SOLVE);
     auto launch = [&](auto kern, int nb) {
         hipLaunchKernelGGL(kern, dim3(1 + div_up(top_bank0, kCW * nb)), dim3(kCT), 0, c.stream, m.L,

@@ -576,8 +576,8 @@ struct Engine {
     }
 
     size_t graph_key() const {
-        size_t h = 1469598103934665603ull;
-        auto mix = [&](size_t v) { h ^= v + 0x9e3779b97f4a7c15ull + (h << 6) + (h >> 2); };
+        GraphKey key;
+        auto mix = [&](size_t v) { key.mix(v); };
         const SymBcoo& S = c.bsr;
         mix((size_t)N); mix((size_t)gN); mix((size_t)gS); mix((size_t)G); mix((size_t)rF); mix((size_t)nF); mix((size_t)gF); mix((size_t)gU); mix((size_t)S.nb); mix((size_t)S.K);
         mix((size_t)S.eptr.p); mix((size_t)S.ent.p); mix((size_t)val); mix((size_t)r); mix((size_t)z); mix((size_t)p);
@@ -586,17 +586,8 @@ struct Engine {
         mix((size_t)c.sub_offset); mix((size_t)c.nb); mix((size_t)c.stream);
         mix((size_t)abd_inv(c)); mix((size_t)abd_rows(c)); mix((size_t)vfull);
         mix((size_t)fused); mix((size_t)nRZ);
-        if (mas) {
-            const MasState& m = c.mas;
-            mix((size_t)m.nbanks); mix((size_t)m.L); mix((size_t)m.M); mix((size_t)m.n); mix((size_t)m.bank);
-            mix((size_t)m.nb1); mix((size_t)m.going_next.p); mix((size_t)m.node_of.p); mix((size_t)m.level_size.p);
-            mix((size_t)m.l1lo.p); mix((size_t)m.l1hi.p);
-            mix((size_t)m.comp_mask.p); mix((size_t)m.slot_node.p);
-            mix((size_t)m.inv64.p); mix((size_t)m.inv32.p); mix((size_t)m.R64.p); mix((size_t)m.R32.p);
-            mix((size_t)m.Z64.p); mix((size_t)m.Z32.p);
-            mix((size_t)m.inv16_ok); mix((size_t)m.inv16.p); mix((size_t)m.inv16_d.p);
-        }
-        return h;
+        if (mas) key.mix(c.mas);
+        return key.h;
     }
 
     static constexpr int kBigGroup = 8;  // iterations in the long captured group (even: parities repeat)

@@ -465,8 +465,8 @@ struct BEngine {
     }
 
     size_t key(int per_graph) const {
-        size_t h = 1469598103934665603ull;
-        auto mix = [&](size_t v) { h ^= v + 0x9e3779b97f4a7c15ull + (h << 6) + (h >> 2); };
+        GraphKey k;
+        auto mix = [&](size_t v) { k.mix(v); };
         const SymBcoo& B = c.bsr;
         mix((size_t)N); mix((size_t)S); mix((size_t)nch); mix((size_t)G); mix((size_t)per_graph);
         mix((size_t)rule); mix((size_t)r); mix((size_t)z); mix((size_t)p); mix((size_t)Ap); mix((size_t)x);
@@ -479,13 +479,8 @@ struct BEngine {
                               (const void*)w.ctrl.p, (const void*)w.bank_scene.p})
             mix((size_t)q);
         mix((size_t)c.stream);
-        const MasState& m = c.mas;
-        mix((size_t)m.nbanks); mix((size_t)m.L); mix((size_t)m.M); mix((size_t)m.n); mix((size_t)m.bank);
-        mix((size_t)m.nb1); mix((size_t)m.node_of.p); mix((size_t)m.inv64.p); mix((size_t)m.inv32.p);
-        mix((size_t)m.R64.p); mix((size_t)m.R32.p); mix((size_t)m.Z64.p); mix((size_t)m.Z32.p);
-        mix((size_t)m.going_next.p); mix((size_t)m.level_size.p); mix((size_t)m.l1lo.p); mix((size_t)m.slot_node.p);
-        mix((size_t)m.inv16_ok); mix((size_t)m.inv16.p); mix((size_t)m.inv16_d.p);
-        return h;
+        k.mix(c.mas);
+        return k.h;
     }
 
     void run(PcgGraph& gc, int per_graph) {

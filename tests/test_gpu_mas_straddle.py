@@ -145,3 +145,76 @@ def test_tables_and_apply_on_both_sides_of_the_one_workgroup_limit(torch_cuda, o
     r = np.random.default_rng(4).normal(size=3 * sc.n)
     z, zo = s.precond_apply(r), mas.apply(r, fp32=False)
     assert np.abs(z - zo).max() <= 1e-11 * np.abs(zo).max()
+
+
+def _two_hierarchies():
+    """Two neighbour lists over 512 vertices in 32 banks of two components: 64
+    level-1 nodes each, then 40 and 10 nodes (banks: 3 + 1) or 32 and 32 (2 + 2),
+    so the same number of banks, another first bank of level 3."""
+    def lists(joins):
+        nb = [set() for _ in range(512)]
+        def join(a, b):
+            nb[a].add(b); nb[b].add(a)
+        for v in range(512):
+            if v % 8:
+                join(v - 1, v)                      # level-1 node v // 8
+        for a, b in joins:
+            join(8 * a, 8 * b)
+        num = np.array([len(q) for q in nb], np.uint32)
+        start = np.concatenate([[0], np.cumsum(num)[:-1]]).astype(np.uint32)
+        return start, num, np.array([u for q in nb for u in sorted(q)], np.uint32)
+    wide = [(i, i + 2) for i in range(64) if i % 4 < 2]
+    narrow = [(16 * k, 16 * k + j) for k in range(4) for j in (2, 4, 6, 8, 10, 12)]
+    left = [0, 1, 3, 5, 7, 9, 11, 13, 14, 15]       # a level-1 bank's nodes after these joins, by lowest member
+    node2 = lambda q: 16 * (q // 10) + left[q % 10]
+    pairs2 = [(10, q) for q in range(10)] + [(0, q) for q in range(11, 16)]
+    pairs2 += [(16, q) for q in list(range(20, 30)) + [30, 31]] + [(20, q) for q in (17, 18, 19)]
+    return lists(narrow + [(node2(a), node2(b)) for a, b in pairs2]), lists(wide)
+
+
+@pytest.mark.parametrize("batched", [False, True])
+def test_graphs_follow_the_split_of_the_upper_levels(torch_cuda, batched):
+    """The fused bank solves are captured with the first bank of level 3.  A
+    hierarchy with as many banks in all, but another such bank, is solved on a
+    context that holds the graph of the other one: the iterates are bit for bit
+    those of a context of its own."""
+    import ctypes as C
+    from sgipc import capi, scene
+    from sgipc.system import NewtonSystem, _p
+    print("case: graphs and level splits, batched", batched, flush=True)
+    sc = scene.cube_scene(7, seed=4)
+    ident = np.arange(512, dtype=np.int32)
+    topos = _two_hierarchies()
+
+    def system():
+        s = NewtonSystem(sc, "cuda:0", precond=capi.PRECOND_MAS)
+        s.ctx.call("sgipc_set_deterministic", 1)
+        s.assemble(); s.convert()
+        return s
+
+    def solve(s, topo, precision):
+        ns, nn, nl = topo
+        s.ctx.call("sgipc_set_mas_topology", 512, 0, ns.ctypes.data, nn.ctypes.data, nl.ctypes.data, len(nl),
+                   ident.ctypes.data, 512, ident.ctypes.data, 16)
+        s.build_precond()
+        if batched:
+            st = (capi.SolveStats * 1)()
+            o = capi.SolveOpts(precision, 1, 1e-6, 0.3, 2000, 8)
+            rs = np.array([0, 512], np.int32)
+            s.ctx.call("sgipc_solve_batched", 1, rs.ctypes.data, _p(s.b), _p(s.dx), C.byref(o), st)
+            st = st[0]
+        else:
+            st = s.solve(tol=1e-6, stop_rule=1, precision=precision, max_iter=2000)
+        L, tot = C.c_int(0), C.c_int(0)
+        ls = np.zeros(16, np.int32)
+        s.ctx.call("sgipc_mas_info", C.byref(L), C.byref(tot), ls.ctypes.data)
+        return st.iterations, s.dx.cpu().numpy().copy(), (L.value, tot.value, (ls[2] + 15) // 16), ls[7]
+
+    for precision in (capi.PRECISION_FP64, capi.PRECISION_MIXED):
+        own = [solve(system(), t, precision) for t in topos]
+        assert own[0][2] == own[1][2] == (4, 640, 4) and own[0][3] != own[1][3]
+        assert own[0][0] > 3 and own[1][0] > 3
+        one = system()
+        for k in (0, 1, 0, 1, 1):
+            it, x, _, _ = solve(one, topos[k], precision)
+            assert it == own[k][0] and np.array_equal(x, own[k][1])

@@ -115,7 +115,8 @@ int sgipc_mas_num_levels(int n_nodes, int bank);
 /* FEM mesh (host tets) for the deterministic vertex-gradient gather. */
 int sgipc_set_fem_mesh(sgipc_ctx* ctx, int n_fem, int T, const uint32_t* h_tets);
 /* MAS topology; replaces initPreconditioner_Neighbor + the uploads of
- * StiffGIPC/gl_main.cu:1294-1328 (MASPreconditioner.cu:2264-2302). */
+ * StiffGIPC/gl_main.cu:1294-1328 (MASPreconditioner.cu:2264-2302).
+ * Neighbour ids of 2^31 and above (padding) are skipped. */
 int sgipc_set_mas_topology(sgipc_ctx* ctx, int n_fem, int node_offset, const uint32_t* h_nstart,
                            const uint32_t* h_nnum, const uint32_t* h_nlist, int nlist_len,
                            const int* h_part_map, int map_size, const int* h_real_map, int bank);

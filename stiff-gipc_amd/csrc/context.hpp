@@ -61,6 +61,7 @@ struct MasState {
     int node_offset = 0; // subtracted from contact-pair vertex ids
     int M = 0;           // slot count (bank * parts)
     int nlist_len = 0;   // neighbours listed
+    bool nlist_padded = false;  // some of them ids to skip (top bit set)
     int L = 0;           // levels
     int total = 0;       // clusters over all levels (multiple of bank)
     int nbanks = 0;      // total / bank

@@ -260,6 +260,8 @@ __global__ void __launch_bounds__(kOrT) k_lx_masks(int n, int B, int level, cons
 #pragma unroll
             for (int k = 0; k < kNbrBatch; ++k) ids[k] = (i0 + k < nn) ? (int)nlist[st + i0 + k] : v;
 #pragma unroll
+            for (int k = 0; k < kNbrBatch; ++k) ids[k] = ids[k] < 0 ? v : ids[k];  // (padding)
+#pragma unroll
             for (int k = 0; k < kNbrBatch; ++k) cu[k] = cs[ids[k]];
 #pragma unroll
             for (int k = 0; k < kNbrBatch; ++k)
@@ -1645,8 +1647,11 @@ void mas_set_topology(Ctx& c, int n, int node_offset, const unsigned* nstart, co
         if (sl < 0 || sl >= M || part_map[sl] != v) throw arg_error("MAS real_map/part_map inconsistent");
         if ((long long)nstart[v] + nnum[v] > nlist_len) throw arg_error("MAS neighbour CSR out of range");
     }
-    for (int i = 0; i < nlist_len; ++i)
+    bool padded = false;  // ids with the top bit set are no neighbours
+    for (int i = 0; i < nlist_len; ++i) {
         if ((int)nlist[i] >= n) throw arg_error("MAS neighbour index out of range");
+        padded = padded || (int)nlist[i] < 0;
+    }
     for (int s2 = 0; s2 < M; ++s2)
         if (part_map[s2] >= n) throw arg_error("MAS part_map entry out of range");
     MasState& m = c.mas;
@@ -1659,6 +1664,7 @@ void mas_set_topology(Ctx& c, int n, int node_offset, const unsigned* nstart, co
     m.node_offset = node_offset;
     m.M = M;
     m.nlist_len = nlist_len;
+    m.nlist_padded = padded;
     m.L = num_levels(std::max(M, n), bank);
     int Mpad = (M + bank - 1) / bank * bank;
     m.going_cap = (size_t)Mpad + (size_t)m.L * ((size_t)n + bank) + bank;
@@ -1707,7 +1713,9 @@ void mas_build(Ctx& c, int sub_offset, int sub_nb, const int* pairs, int npairs)
     int* l1hi = m.l1hi.reserve((size_t)nb1_cap + 2);
     int* vlo = m.own_lo.reserve((size_t)nb1_cap + 2);
     int* vhi = m.own_hi.reserve((size_t)nb1_cap + 2);
-    const bool small = n > 0 && n <= kSmallN && M <= kSmallM && m.nlist_len <= kSmallList && npairs <= kSmallPairs;
+    // (its 16-bit lists have no room for padding)
+    const bool small = n > 0 && n <= kSmallN && M <= kSmallM && m.nlist_len <= kSmallList && !m.nlist_padded &&
+                       npairs <= kSmallPairs;
     if (small) {
         hipLaunchKernelGGL(k_small_tables, dim3(1), dim3(kSmallT), 0, s,
                            (SmallTables{M, Mpad, n, B, L, m.node_offset, npairs, nb1_cap, m.nlist_len, m.part_map.p, m.real_map.p,

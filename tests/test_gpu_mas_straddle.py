@@ -218,3 +218,47 @@ def test_graphs_follow_the_split_of_the_upper_levels(torch_cuda, batched):
         for k in (0, 1, 0, 1, 1):
             it, x, _, _ = solve(one, topos[k], precision)
             assert it == own[k][0] and np.array_equal(x, own[k][1])
+
+
+@pytest.mark.parametrize("cells,bank", [(4, 16), (11, 32), (12, 16), (13, 16)])
+def test_padded_neighbour_lists_give_the_same_tables(torch_cuda, cells, bank):
+    """Neighbour ids of 2^31 and above are padding: lists with such ids before,
+    between and after the neighbours (and vertices with nothing else) give the
+    tables of the lists without them, bit for bit, on both sides of the
+    one-workgroup limit; any other id outside the range is refused."""
+    from sgipc import capi, scene
+    from sgipc.capi import SgipcError
+    from sgipc.system import NewtonSystem
+    print("case: padded neighbour lists", cells, bank, flush=True)
+    sc = scene.cube_scene(cells, seed=3, bank=bank)
+    s = NewtonSystem(sc, "cuda:0", precond=capi.PRECOND_MAS)
+    s.assemble(); s.convert()
+    lists = [list(s.nl[a:a + k]) for a, k in zip(s.ns.astype(int), s.nn.astype(int))]
+    lists[sc.n // 2] = []
+
+    def tables(padding, bad=None):
+        rng, out, num = np.random.default_rng(6), [], []
+        for q in lists:
+            q = list(q)
+            if padding:
+                for pad in rng.choice([0xFFFFFFFF, 0x80000000, 0x80000005], size=int(rng.integers(1, 4))):
+                    q.insert(int(rng.integers(0, len(q) + 1)), int(pad))
+            num.append(len(q)); out += q
+        if bad is not None:
+            out[len(out) // 2] = bad
+        num = np.array(num, np.uint32); out = np.array(out, np.uint32)
+        start = np.concatenate([[0], np.cumsum(num)[:-1]]).astype(np.uint32)
+        s.ctx.call("sgipc_set_mas_topology", sc.n, 0, start.ctypes.data, num.ctypes.data, out.ctypes.data, len(out),
+                   s.part_map.ctypes.data, len(s.part_map), s.real_map.ctypes.data, bank)
+        s.build_precond()
+        return s.mas_tables()
+
+    t, p = tables(False), tables(True)
+    assert t["levelnum"] == p["levelnum"] and t["total"] == p["total"]
+    for key in ("level_size", "coarse_space", "fine_mask", "prefix0", "going_next"):
+        assert np.array_equal(t[key], p[key]), key
+    k = t["levelnum"] - 1
+    assert np.array_equal(t["coarse_table"][:, :k], p["coarse_table"][:, :k])
+    for bad in (sc.n, 0x7FFFFFFF):
+        with pytest.raises(SgipcError, match="neighbour index out of range"):
+            tables(False, bad)

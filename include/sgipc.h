@@ -356,7 +356,10 @@ int sgipc_solve_batched(sgipc_ctx* ctx, int n_scenes, const int* h_row_start, co
  * graph launch of the launch sequence and 512/1024 threads per workgroup of
  * the persistent form -- and keeps the fastest for later solves; batched,
  * the fastest sequence and persistent candidates are then timed on whole
- * solves to a 1e-6 true relative residual, which decide.  d_b is only read. */
+ * solves to a 1e-6 true relative residual, which decide.  sgipc_solve's SpMV
+ * goes by matrix entries and has no lanes per row, except mixed with
+ * SGIPC_SPMV_FULL32=0 in the environment: otherwise n_scenes = 0 keeps both
+ * numbers as they are and returns them.  d_b is only read. */
 int sgipc_autotune(sgipc_ctx* ctx, const double* d_b, int n_scenes, const int* h_row_start, int precision,
                    int* h_group, int* h_iters_per_graph);
 /* on != 0: the MAS build sums every coarse-level bank entry in a fixed
@@ -365,7 +368,8 @@ int sgipc_autotune(sgipc_ctx* ctx, const double* d_b, int n_scenes, const int* h
  * bitwise from run to run (slower build).  Default 0.  The reference
  * projects with atomics (MASPreconditioner.cu:1816-2093). */
 int sgipc_set_deterministic(sgipc_ctx* ctx, int on);
-/* Set the schedule directly (group 4, 8 or 16; 1..64 iterations per graph). */
+/* Set the schedule directly (group 4, 8 or 16; 1..64 iterations per graph)
+ * for the batched solver, and the group for any SpMV with lanes per row. */
 int sgipc_set_schedule(sgipc_ctx* ctx, int group, int iters_per_graph);
 /* Batched solver form; no reference counterpart.  persistent = 0: the
  * graph-captured launch sequence above; 1: one persistent launch in which

@@ -718,8 +718,9 @@ namespace sgipc {
 
 // Schedule autotuner: times a fixed number of PCG iterations (unreachable
 // tolerance) for each candidate schedule on the current system and keeps the
-// fastest.  Candidates: lanes per block row in the SpMV (4, 8, 16) and, for
-// the batched solver, iterations captured per graph launch (2, 4, 8) of the
+// fastest.  Candidates: lanes per block row in the SpMV (4, 8, 16; where the
+// SpMV has them: the batched solvers and the upper BCOO's) and, for the batched
+// solver, iterations captured per graph launch (2, 4, 8) of the
 // launch sequence, and (16-vertex banks) the persistent form with 512 or
 // 1024 threads per workgroup.  For the batched solver the fixed-iteration
 // trial only shortlists: the fastest launch sequence and the fastest
@@ -743,10 +744,14 @@ void autotune(Ctx& c, const double* b, int S, const int* h_row_start, int precis
         int group, per_graph, persistent, threads;
     };
     std::vector<Cand> cands;
+    // a single system's SpMV over the copy of both triangles has no lanes per
+    // row: one candidate, the group as it was set (its solve refuses what any
+    // solve refuses)
+    const bool by_entries = S == 0 && (precision == 0 || c.spmv_full32);
     for (int g : {4, 8, 16}) {
         if (S > 0)
             for (int pg : {2, 4, 8}) cands.push_back({g, pg, 0, c.batch_threads});
-        else
+        else if (!by_entries || g == c.spmv_group)
             cands.push_back({g, c.batch_iters_per_graph, 0, c.batch_threads});
     }
     if (S > 0 && c.mas.ready && c.mas.bank == 16)

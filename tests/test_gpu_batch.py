@@ -341,3 +341,28 @@ def test_launch_sequence_chunk_sizes(torch_cuda, five_scenes, group, per_graph):
     one = big.solve(tol=1e-4, stop_rule=0)
     assert one.iterations == st[0].iterations
     assert np.linalg.norm(big.dx.cpu().numpy() - x) <= 1e-10 * np.linalg.norm(x)
+
+
+def test_autotune_of_one_system_keeps_a_group_without_effect(torch_cuda, cube4):
+    """A single system's solve reads the copy of both triangles by entries, so
+    lanes per row change nothing in it: the autotuner leaves the schedule as it
+    was set (a batched solve on the same context uses it), and what it refused
+    it refuses still."""
+    from sgipc import capi
+    from sgipc.capi import SgipcError
+    from sgipc.system import NewtonSystem, _p
+    print("case: autotune of one system", flush=True)
+    s = NewtonSystem(cube4, "cuda:0", precond=capi.PRECOND_MAS)
+    g, pg = C.c_int(0), C.c_int(0)
+
+    def tune(precision):
+        s.ctx.call("sgipc_autotune", _p(s.b), 0, None, precision, C.byref(g), C.byref(pg))
+    with pytest.raises(SgipcError, match="convert first"):
+        tune(capi.PRECISION_FP64)
+    s.assemble(); s.convert()
+    s.build_precond()
+    for group, per_graph in ((4, 2), (16, 3), (8, 4)):
+        for precision in (capi.PRECISION_FP64, capi.PRECISION_MIXED):
+            s.ctx.call("sgipc_set_schedule", group, per_graph)
+            tune(precision)
+            assert (g.value, pg.value) == (group, per_graph)

@@ -88,6 +88,7 @@ int sgipc_ctx_create(int device, sgipc_ctx** out) {
             int v = std::atoi(g);
             if (v == 4 || v == 8 || v == 16) c->spmv_group = v;
         }
+        if (const char* f = std::getenv("SGIPC_SPMV_FULL64")) c->spmv_full64 = std::atoi(f) != 0;
         if (const char* f = std::getenv("SGIPC_SPMV_FULL32")) c->spmv_full32 = std::atoi(f) != 0;
         if (const char* f = std::getenv("SGIPC_MAS_FUSED")) c->mas_fused = std::atoi(f) != 0;
         if (const char* f = std::getenv("SGIPC_SORT")) c->sort_impl = std::string(f) == "rocprim" ? 1 : 0;

@@ -57,6 +57,20 @@ struct DBuf {
         cap = n ? n : 1;
         return p;
     }
+    // null (and no buffer) where the device has not that much memory left
+    T* try_reserve(size_t n) {
+        if (n <= cap && p) return p;
+        release();
+        const size_t want = n ? n : 1;
+        const hipError_t e = hipMalloc((void**)&p, want * sizeof(T));
+        if (e == hipErrorOutOfMemory) {
+            (void)hipGetLastError();
+            return p = nullptr;
+        }
+        SGIPC_HIP(e);
+        cap = want;
+        return p;
+    }
     T* get() const { return p; }
 };
 

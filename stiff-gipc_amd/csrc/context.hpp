@@ -258,6 +258,7 @@ struct Ctx {
     SymBcoo bsr;
     bool have_bsr = false;
     int spmv_group = 8;  // lanes per block row in the batched solvers' SpMV and the upper-BCOO one (env SGIPC_SPMV_G: 4, 8, 16)
+    int spmv_full64 = 1; // FP64: copy of both triangles (env SGIPC_SPMV_FULL64=0, or no memory for it: upper BCOO)
     int spmv_full32 = 1; // mixed precision: FP32 copy of both triangles (env SGIPC_SPMV_FULL32=0: upper BCOO)
     int deterministic = 0;  // 1: MAS projection and barrier gradient summed in a fixed order (bitwise repeatable)
     DBuf<double> grad_scr;               // ordered barrier gradient: per-pair rows (12 doubles per pair)
@@ -338,7 +339,7 @@ int bcoo_convert(Ctx& c, long long nt, int nblockrows);
 void bsr_build(Ctx& c);
 const float* bsr_values_f32(Ctx& c);
 const float* bsr_full(Ctx& c, float);    // both triangles in entry order, FP32 (as converted)
-const double* bsr_full(Ctx& c, double);  // the same in FP64, of the values as they are now
+const double* bsr_full(Ctx& c, double);  // the same in FP64, of the values as they are now (null: no room for it)
 void spmv64(Ctx& c, double a, const double* x, double b, double* y);
 
 double kinetic_energy(Ctx& c, int n, const double* x, const double* xt, const double* m);

@@ -524,11 +524,9 @@ struct Engine {
         if (vfull) {
             hipLaunchKernelGGL((k_spmv_pap_full<V>), dim3(gS), dim3(kFT), 0, s, S.nb, rF, nF, gF, S.eptr.p, vfull,
                                (const V*)z, p, Ap, (const double*)rz_last, (const double*)rz_this, nRZ, part_pap, ctrl);
-        } else if constexpr (sizeof(V) == 4) {
-            if (G == 4) launch(k_spmv_pap<4, MV, V>);
-            else if (G == 16) launch(k_spmv_pap<16, MV, V>);
-            else launch(k_spmv_pap<8, MV, V>);
-        }
+        } else if (G == 4) launch(k_spmv_pap<4, MV, V>);
+        else if (G == 16) launch(k_spmv_pap<16, MV, V>);
+        else launch(k_spmv_pap<8, MV, V>);
         SGIPC_LAUNCH_CHECK();
         prof_end(c, PROF_SPMV);
         if (mas) {
@@ -870,7 +868,9 @@ void pcg_solve(Ctx& c, const double* b, double* x, const SolveOpts& o, SolveStat
                                         mas ? (T*)(fp32mas ? (void*)c.mas.R32.p : (void*)c.mas.R64.p) : nullptr,
                                         mas ? (T*)(fp32mas ? (void*)c.mas.Z32.p : (void*)c.mas.Z64.p) : nullptr,
                                         c.precond_kind == 1 ? w.Dinv.p : nullptr, o.stop_rule};
-            E.use_full(bsr_full(c, double{}));
+            E.G = G;
+            w.xw.reserve(N + 1);  // the true residual's, before the copy takes what is left
+            if (const double* vf = bsr_full(c, double{})) E.use_full(vf);
             hipLaunchKernelGGL((k_copy_cast<double, double>), dim3(gN), dim3(kThreads), 0, s, N, E.r, b);
             SGIPC_LAUNCH_CHECK();
             E.init(o.tol, max_iter);

@@ -169,34 +169,41 @@ void bsr_build(Ctx& c) {
     c.have_bsr = true;
 }
 
+// values of a copy: 2K bounds the entries (lower references + upper blocks; how
+// many blocks lie on the diagonal only the device knows); whole groups of 64
 template <typename T>
-static const T* full_copy(Ctx& c, DBuf<T>& buf) {
-    SymBcoo& S = c.bsr;
-    // 2K bounds the entries (lower references + upper blocks; how many blocks
-    // lie on the diagonal only the device knows); whole groups of 64
-    T* vf = buf.reserve(((2 * (size_t)S.K + 63) / 64 + 1) * FullCopy<T>::kGroup);
+static size_t full_size(const SymBcoo& S) {
+    return ((2 * (size_t)S.K + 63) / 64 + 1) * FullCopy<T>::kGroup;
+}
+template <typename T>
+static void full_copy(Ctx& c, T* vf) {
+    const SymBcoo& S = c.bsr;
     if (S.nb > 0 && S.K > 0) {
         const int blocks = 8 * std::max(1, std::min((int)div_up(2LL * S.K, 8 * 256), 1024));
         hipLaunchKernelGGL(k_full_copy<T>, dim3(blocks), dim3(256), 0, c.stream, S.nb, (const int*)S.eptr.p,
                            (const int2*)S.ent.p, (const int*)c.t_cols, (const double*)c.t_vals, vf);
         SGIPC_LAUNCH_CHECK();
     }
-    return vf;
 }
 // Kept until the next convert: the mixed solves' refinement takes its residuals
 // from the converted values themselves.
 const float* bsr_full(Ctx& c, float) {
     if (!c.have_bsr) bsr_build(c);
     SymBcoo& S = c.bsr;
-    if (!S.full32_ok) full_copy<float>(c, S.full32);
+    float* vf = S.full32.reserve(full_size<float>(S));
+    if (!S.full32_ok) full_copy(c, vf);
     S.full32_ok = true;
-    return S.full32.p;
+    return vf;
 }
 // Made anew by every solve: the values are the caller's, who may have written to
-// them since (nothing else of an FP64 solve would notice).
+// them since (nothing else of an FP64 solve would notice).  Null where it is
+// switched off or does not fit (152 bytes per upper block).
 const double* bsr_full(Ctx& c, double) {
+    if (!c.spmv_full64) return nullptr;
     if (!c.have_bsr) bsr_build(c);
-    return full_copy<double>(c, c.bsr.full64);
+    double* vf = c.bsr.full64.try_reserve(full_size<double>(c.bsr));
+    if (vf) full_copy(c, vf);
+    return vf;
 }
 
 // FP32 copy of the BCOO values for the mixed-precision solve

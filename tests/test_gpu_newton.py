@@ -417,3 +417,25 @@ def test_solve_with_rows_without_triplets(torch_cuda, oracle, cube4, kind, mixed
     res = np.linalg.norm(A @ x[rows].reshape(-1) - ref["b"]) / np.linalg.norm(ref["b"])
     # the FP64 recurrence's residual drifts from the true one by rounding (half a digit of slack)
     assert st.converged and res <= 3 * tol and st.rel_residual <= 3 * tol, (res, st.rel_residual)
+
+
+@pytest.mark.parametrize("kind,group", [(0, 8), (1, 4), (2, 4), (2, 8), (2, 16), (3, 16)])
+def test_fp64_solve_on_the_upper_blocks(torch_cuda, monkeypatch, cube10, kind, group):
+    """Where the entry-order copy does not fit the device (or is switched off) the
+    FP64 solve reads the converted upper blocks in place: the iteration count and
+    iterate of the solve on the copy, but for the order of the row sums (1e-10,
+    as against the oracle above)."""
+    print("case: upper-BCOO FP64 solve, precond", kind, "group", group, flush=True)
+    ref = make_system(cube10, kind)
+    monkeypatch.setenv("SGIPC_SPMV_FULL64", "0")
+    s = make_system(cube10, kind)
+    s.ctx.call("sgipc_set_schedule", group, 4)
+    for q in (ref, s):
+        q.ctx.call("sgipc_set_deterministic", 1)
+        q.assemble(); q.convert(); q.build_precond()
+    for tol, rule in ((1e-4, 0), (1e-30, 0)):
+        st, so = (q.solve(tol=tol, stop_rule=rule, max_iter=12 if tol < 1e-9 else 5000) for q in (s, ref))
+        assert st.iterations == so.iterations and st.converged == so.converged
+        x, xo = s.dx.cpu().numpy(), ref.dx.cpu().numpy()
+        assert np.linalg.norm(x - xo) <= 1e-10 * np.linalg.norm(xo)
+        assert abs(st.rel_residual - so.rel_residual) <= 1e-6 * so.rel_residual

@@ -78,11 +78,22 @@ def copy_calibration(mib):
     print(json.dumps({"copy_calibration_bytes_read": n * 8, "copy_calibration_bytes_written": n * 8}))
 
 
+def spmv_kernel_name(fp32):
+    # the SpMV that the library picks, from the environment that it reads
+    T = "float" if fp32 else "double"
+    if os.environ.get("SGIPC_SPMV_FULL32" if fp32 else "SGIPC_SPMV_FULL64", "1") != "0":
+        return "k_spmv_pap_full<%s> (PCG SpMV + direction update, grouped copy of both triangles)" % T
+    g = os.environ.get("SGIPC_SPMV_G", "8")
+    g = g if g in ("4", "8", "16") else "8"   # lanes per block row
+    return "k_spmv_pap<%s, %s, %s> (PCG SpMV + direction update, upper BCOO)" % (g, T, T)
+
+
 def spmv_alg_bytes(K, nb, fp32):
     # the PCG SpMV kernel (direction update fused): upper BCOO, 9 values
     # (72 B FP64 / 36 B FP32) + 8 B (row, col) per block; per block row z
-    # read once, p and Ap each read and written once.  (The FP32 copy is
-    # stored padded to 48 B per block; the padding is not counted.)
+    # read once, p and Ap each read and written once.  (The copy that the
+    # kernel reads holds both triangles, 40 or 76 B an entry; the minimum counts
+    # the upper one once.)
     vb = 36.0 if fp32 else 72.0
     xb = 12.0 if fp32 else 24.0
     return (vb + 8.0) * K + 5.0 * xb * nb
@@ -499,12 +510,16 @@ def main():
     fp32 = main_mode == "mixed"
     alg = spmv_alg_bytes(sysm.K, sysm.n, fp32)
     achieved = alg / (r["spmv_ms"] * 1e-3) / 1e9
+    kname = spmv_kernel_name(fp32)
+    # stored counters, where they are of the kernel that ran
     traffic = None
     tf = os.path.join(ROOT, "profiles", "spmv_traffic.json")
     if os.path.exists(tf):
         try:
             with open(tf) as f:
-                traffic = json.load(f)[main_mode]["hbm_bytes_per_launch"]
+                rec = json.load(f)[main_mode]
+            if kname.startswith(rec["kernel"]):
+                traffic = rec["hbm_bytes_per_launch"]
         except (OSError, ValueError, KeyError, TypeError):
             traffic = None
 
@@ -525,14 +540,6 @@ def main():
                                  "sample": "%d step(s), %d iterations, %.1f s" % (ssteps, sit, ssecs)},
                "label": "CPU restatement of the reference algorithm (baseline only)", "host": host_cpu()}
 
-    g = os.environ.get("SGIPC_SPMV_G", "8")
-    g = g if g in ("4", "8", "16") else "8"   # lanes per block row, as the library reads it
-    full32 = os.environ.get("SGIPC_SPMV_FULL32", "1") != "0"   # the library's default for mixed solves
-    if fp32 and not full32:
-        kname = "k_spmv_pap<%s, float, float> (PCG SpMV + direction update, FP32 upper BCOO)" % g
-    else:
-        kname = "k_spmv_pap_full<%s> (PCG SpMV + direction update, grouped copy of both triangles)" % \
-            ("float" if fp32 else "double")
     out = {
         "metric": "Newton solves/sec (assembly + BCOO convert + MAS build + MAS-PCG to 1e-6 true rel. residual)",
         "value": round(r["value"], 4),
@@ -576,7 +583,7 @@ def main():
                                         "FETCH_SIZE / WRITE_SIZE runs of this kernel, scaled by a device copy); "
                                         "not measured in this run") if traffic is not None else None,
                      "avg_ms": round(r["spmv_ms"], 5), "launches": r["spmv_calls"], "alg_bytes": alg,
-                     "cache_note": "the SpMV's matrix copy (about 76 MB FP32 / 68 MB FP64) fits MI355X's 256 MB "
+                     "cache_note": "the SpMV's matrix copy (about 70 MB FP32 / 134 MB FP64) fits MI355X's 256 MB "
                                    "Infinity Cache; FETCH_SIZE counts L2 misses, which it may serve instead of HBM"},
         "cpu_baseline": cpu,
         "broad_phase": bp,
@@ -649,11 +656,7 @@ def hybrid(a):
     fp32 = main_mode == "mixed"
     alg = spmv_alg_bytes(s.K, s.nbr, fp32)
     achieved = alg / (r["spmv_ms"] * 1e-3) / 1e9
-    g = os.environ.get("SGIPC_SPMV_G", "8")
-    g = g if g in ("4", "8", "16") else "8"
-    full32 = os.environ.get("SGIPC_SPMV_FULL32", "1") != "0"
-    kname = "k_spmv_pap<%s, float, float>" % g if fp32 and not full32 else \
-        "k_spmv_pap_full<%s>" % ("float" if fp32 else "double")
+    kname = spmv_kernel_name(fp32)
     cpu = None
     if not a.no_cpu_baseline:
         sys.path.insert(0, os.path.join(ROOT, "oracle"))

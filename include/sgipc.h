@@ -332,7 +332,8 @@ int sgipc_precond_apply(sgipc_ctx* ctx, const double* d_r, double* d_z);
  * (sgipc_spmv too) from them as they are at the call, so a shift or scaling
  * written there needs no other convert (the preconditioner stays as built).
  * SGIPC_PRECISION_MIXED iterates on an FP32 copy made by the first mixed solve
- * after a convert and refines on the residual of the current values. */
+ * after a convert and refines on the residual of the current values, which
+ * converges while the two are close; after a large change convert again. */
 int sgipc_solve(sgipc_ctx* ctx, const double* d_b, double* d_x, const sgipc_solve_opts* opts,
                 sgipc_solve_stats* stats);
 

@@ -419,7 +419,9 @@ __device__ inline int xcd_order(int q, int n) {
 // An edge query skips subtrees without an id above its own, and every XCD
 // takes a contiguous range of the queries, so that a node is read into its L2
 // once and not once per XCD.  76,804 queries of two 40^3 boxes: 216 us with
-// the tests in the walk and workgroups in launch order, 150 us so.
+// the tests in the walk and workgroups in launch order, 150 us so (1201
+// wavefronts, 1.8 per CU on average over the launch; 79 % of the L2 requests
+// hit).
 template <int PASS>
 __global__ void __launch_bounds__(kQT) k_query(Trees T, Query Q) {
     __shared__ unsigned stack[kStack * kQT];

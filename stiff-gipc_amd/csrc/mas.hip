@@ -12,8 +12,9 @@
 // Table semantics are identical to the reference (integer, bit-exact); the
 // reference's warp-synchronous 16-lane-bank tricks become explicit LDS stages
 // with block barriers (a bank is a quarter of a wave64).  The restriction is
-// a deterministic per-bank component sum (no FP atomics); the apply is a
-// bank-per-workgroup dense GEMV on the symmetric inverse.
+// a deterministic per-bank component sum (no FP atomics); the apply is a dense
+// product with the symmetric inverse, a wavefront per 16-vertex bank (from
+// registers, bank_solve.hpp) or a workgroup per 32-vertex one.
 #include "context.hpp"
 #include <rocprim/device/device_radix_sort.hpp>
 #include <utility>
@@ -380,7 +381,7 @@ __device__ inline int project_block(int B, int li, int lj, bool same_vertex, con
 // Galerkin projection for 16-vertex banks when vertex ids follow slot order:
 // workgroup b owns the vertices whose level-1 node lies in level-1 bank b,
 // i.e. the contiguous BCOO rows [vlo_b, vhi_b).  Level 0 targets are unique
-// (plain stores).  Level-1 and level-2 targets accumulate in one-bank LDS
+// (read and added to without atomics; they were zeroed before).  Level-1 and level-2 targets accumulate in one-bank LDS
 // windows (the first owned vertex's banks, which hold nearly every target)
 // flushed once; the top levels (>= top_lvl, at most kProjTopBanksMax banks)
 // accumulate in LDS and are written as per-workgroup partials, summed
@@ -1043,10 +1044,10 @@ __device__ inline void restrict_bank(int b, int B, int L, int beg1, const SlotNo
 }
 
 // Multilevel restriction R_l = sum of children, levels 0 to 2 in one launch.
-// Workgroup b owns level-1 bank b: it gathers the level-0 slots of every
-// level-0 bank holding one of its children (reading the residual r through
-// part_map, writing R_0 for the banks whose first child lands in b), forms
-// its level-1 sums, and from them the level-2 nodes (whose children always
+// Workgroup b owns level-1 bank b: it goes through the level-0 slots of every
+// level-0 bank holding one of its children (slot_node), takes the residual r of
+// those whose level-1 node lies in b (they alone are read, and written to R_0,
+// here), forms its level-1 sums, and from them the level-2 nodes (whose children always
 // lie in one level-1 bank).  Sum orders are those of the level-by-level
 // component sums, so results do not depend on the schedule.
 template <typename V, typename T>
@@ -1352,9 +1353,11 @@ __global__ void __launch_bounds__(kTB) k_l1_ranges(int M, int B, const int* __re
 // lists (16-bit), the masks and the vertices' nodes of the current level live
 // in LDS, a phase ends with a barrier, and only the tables go to memory.
 // Latency-bound: 20 us at 125 vertices and 59 us at 1331, where the launches
-// it replaces (about 40) took 90 and 150 us of a step.  Above 2048 vertices
-// (two per thread) one CU is too few: 369 us against 170 at 5488 vertices, with
-// the lists read from memory because they no longer fit LDS.
+// it replaces (about 40) took 90 and 150 us of a step.  A whole build, this
+// launch against those: 76 and 140 us at 125 vertices, 94 and 152 at 512, 120 and
+// 164 at 1000, 128 and 167 at 1331, 161 and 175 at 1728, 172 and 188 at 2000.
+// Above 2048 vertices (two per thread) one CU is too few: 369 us against 170 at
+// 5488 vertices, with the lists read from memory because they no longer fit LDS.
 constexpr int kSmallT = 1024;
 constexpr int kSmallN = 2048;
 constexpr int kSmallM = 4096;

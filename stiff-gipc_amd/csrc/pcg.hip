@@ -261,8 +261,11 @@ __global__ void __launch_bounds__(kThreads) k_simple_precond_dot(long long N, co
 // (70 MB) 20.3 -> 17.7 us, FP64 (134 MB; the upper BCOO has 68 MB, but a
 // scattered 72-byte gather per transposed block) 37.3 -> 28.6 us, where a plain
 // read of as many bytes takes about 12 and 21 us; at 525 block rows 8.9 ->
-// 4.9 us.  Several entries in flight per thread were slower (more registers,
-// fewer wavefronts): 21.3 and 22.6 us for two and four against 19.8 us.
+// 4.9 us.  Counted there: 81 MB and 155 MB past L2, 30 % and 24 % of the L2
+// requests hit (the gathers of z), 14 and 11 wavefronts per CU on average over
+// a launch, 8 % of the LDS cycles are bank conflicts.  Several entries in flight
+// per thread were slower (more registers, fewer wavefronts): 21.3 and 22.6 us
+// for two and four against 19.8 us.
 constexpr int kFT = 256;          // threads
 constexpr int kFRows = 72;        // block rows per chunk, at most (three components each, of 256 threads)
 constexpr int kFBatch = 1024;     // entries per LDS batch
@@ -475,10 +478,17 @@ struct Engine {
     const V* vfull = nullptr;
     int rF = 1, nF = 1, gF = 1;
     // Rows per chunk: at least 8, so that small systems spread over many
-    // workgroups (one entry per thread), and more once there are 1920 chunks,
-    // seven or eight resident workgroups per CU, up to 72 (at 137 k rows, 42,
-    // 54, 64, 72 and 85 rows: 20.8, 20.0, 21.1, 18.8 and 19.8 us in FP32, the
-    // same order in FP64).
+    // workgroups (one entry per thread), and more once there are 1920 chunks, 7.5
+    // workgroups per CU (8 fit by registers in FP32, 6 in FP64), up to 72.  Per
+    // launch, FP64 / FP32, the rule's own number first:
+    //   1,331 rows:   8: 4.6 / 4.8 us, 4: 5.3 / 5.4, 32: 5.2 / 5.4, 72: 6.9 / 6.5
+    //   19,683 rows: 11: 8.6 / 7.1, 16: 7.0 / 6.7, 32: 6.7 / 6.6, 72: 7.5 / 7.1
+    //   43,904 rows: 23: 13.4 / 7.8, 32: 10.7 / 7.4, 48: 10.5 / 7.0, 72: 10.5 / 7.3
+    //   137,842 rows: 72: 26.1 / 15.6, 42: 29.0 / 17.9, 54: 26.0 / 17.1, 64: 26.2 / 18.6, 85: 28.4 / 16.2
+    //   265,302 rows: 72: 48.0 / 26.7, 48: 48.9 / 25.6, 64: 49.5 / 27.9, 85: 50.7 / 27.3
+    // so it is within 4 % of the best at both ends, and up to 28 % off it in
+    // FP64 between 20 k and 44 k rows, where larger chunks do better.  (Solves
+    // without a preconditioner: the matrix stays in the Infinity Cache.)
     void use_full(const V* vf) {
         vfull = vf;
         rF = std::max(8, std::min(kFRows, (int)div_up(c.nb, 1920)));
@@ -673,7 +683,7 @@ struct Engine {
             // Keep two groups of iterations queued ahead of the device and
             // follow its published progress in pinned memory: the device never
             // waits for the host, and at most two groups run past the stop
-            // (their kernels return at once).  Groups are kBigGroup
+            // (their kernels read their first data and store nothing).  Groups are kBigGroup
             // iterations long (one graph launch and one publication per
             // group) while the convergence rate seen in the publications
             // predicts more than that many iterations to go, two iterations

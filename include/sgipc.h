@@ -358,10 +358,11 @@ int sgipc_solve_batched(sgipc_ctx* ctx, int n_scenes, const int* h_row_start, co
  * the persistent form -- and keeps the fastest for later solves; batched,
  * the fastest sequence and persistent candidates are then timed on whole
  * solves to a 1e-6 true relative residual, which decide.  sgipc_solve's SpMV
- * goes by matrix entries and has no lanes per row, unless the environment has
- * SGIPC_SPMV_FULL64=0 (FP64) or SGIPC_SPMV_FULL32=0 (mixed): otherwise
- * n_scenes = 0 keeps both numbers as they are and returns them.  d_b is only
- * read. */
+ * goes by matrix entries and has no lanes per row, except FP64 where a copy of
+ * the matrix would not stay cached (some 200,000 to 360,000 block rows) and with
+ * SGIPC_SPMV_FULL64=0 (FP64) or SGIPC_SPMV_FULL32=0 (mixed) in the environment:
+ * otherwise n_scenes = 0 keeps both numbers as they are and returns them.  d_b
+ * is only read. */
 int sgipc_autotune(sgipc_ctx* ctx, const double* d_b, int n_scenes, const int* h_row_start, int precision,
                    int* h_group, int* h_iters_per_graph);
 /* on != 0: the MAS build sums every coarse-level bank entry in a fixed

@@ -258,7 +258,8 @@ struct Ctx {
     SymBcoo bsr;
     bool have_bsr = false;
     int spmv_group = 8;  // lanes per block row in the batched solvers' SpMV and the upper-BCOO one (env SGIPC_SPMV_G: 4, 8, 16)
-    int spmv_full64 = 1; // FP64: copy of both triangles (env SGIPC_SPMV_FULL64=0, or no memory for it: upper BCOO)
+    int spmv_full64 = -1; // FP64: copy of both triangles, 1 where it fits the device, 0 never (upper BCOO), -1 by
+                          // fp64_on_copy (env SGIPC_SPMV_FULL64: 0, 1)
     int spmv_full32 = 1; // mixed precision: FP32 copy of both triangles (env SGIPC_SPMV_FULL32=0: upper BCOO)
     int deterministic = 0;  // 1: MAS projection and barrier gradient summed in a fixed order (bitwise repeatable)
     DBuf<double> grad_scr;               // ordered barrier gradient: per-pair rows (12 doubles per pair)
@@ -335,11 +336,38 @@ double ground_energy(Ctx& c, int m, const unsigned* ids, const double* x, const 
 double ground_step_bound(Ctx& c, int m, const unsigned* ids, const double* x, const double* dir,
                          const double* normal, double offset, double slack);
 
+// Whether the FP64 PCG iterates on the copy of both triangles or on the upper
+// BCOO in place.  The copy's SpMV is faster (contiguous reads) but streams twice
+// the bytes, and an iteration's data otherwise stays in the 256 MB Infinity Cache:
+// in place where the copy would take it past kPcgCached bytes and the upper blocks
+// would not.  rest: an iteration's bytes besides the matrix (inverses, vectors).
+// Per iteration, copy / in place, cubes of one body: MAS 132,651 rows 60.6 / 67.5
+// us, 157,464: 68.2 / 71.3, 185,193: 91.4 / 91.3, 226,981: 109.5 / 107.7, 262,144:
+// 120.0 / 122.4; FP32 apply 185,193: 67.3 / 70.8, 226,981: 87.7 / 79.6, 262,144:
+// 98.1 / 96.0, 300,763: 114.3 / 117.7; block Jacobi 226,981: 68.2 / 69.3, 262,144:
+// 76.7 / 74.9, 300,763: 98.3 / 88.6, 357,911: 114.5 / 110.9, 493,039: 147.4 /
+// 156.3; the copy is made in 0.1 to 0.15 ms there.
+constexpr double kPcgCached = 300e6;
+inline bool fp64_copy_pays(double K, double nb, double rest) {
+    const double entries = 2.0 * K - nb;  // (every row has its diagonal block)
+    return !(76.0 * entries + rest > kPcgCached && 72.0 * K + 8.0 * entries + rest <= kPcgCached);
+}
+inline bool fp64_on_copy(const Ctx& c) {
+    if (c.spmv_full64 >= 0) return c.spmv_full64 != 0;
+    double rest = 120.0 * c.nb;  // r, z, p, Ap, x
+    if (c.precond_kind == 1) rest += 72.0 * c.nb;
+    if (c.precond_kind >= 2) {
+        const double D = 3.0 * c.mas.bank, T = c.precond_kind == 3 ? 4.0 : 8.0;
+        rest += T * (c.mas.nbanks * (D * (D + 1.0) / 2.0) + 6.0 * c.mas.total);  // inverses, R and Z
+    }
+    return fp64_copy_pays(c.K, c.nb, rest);
+}
+
 int bcoo_convert(Ctx& c, long long nt, int nblockrows);
 void bsr_build(Ctx& c);
 const float* bsr_values_f32(Ctx& c);
 const float* bsr_full(Ctx& c, float);    // both triangles in entry order, FP32 (as converted)
-const double* bsr_full(Ctx& c, double);  // the same in FP64, of the values as they are now (null: no room for it)
+const double* bsr_full(Ctx& c, double);  // the same in FP64, of the values as they are now (null: iterate on the upper BCOO)
 void spmv64(Ctx& c, double a, const double* x, double b, double* y);
 
 double kinetic_energy(Ctx& c, int n, const double* x, const double* xt, const double* m);

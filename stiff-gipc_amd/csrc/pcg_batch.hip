@@ -747,7 +747,7 @@ void autotune(Ctx& c, const double* b, int S, const int* h_row_start, int precis
     // a single system's SpMV over the copy of both triangles has no lanes per
     // row: one candidate, the group as it was set (its solve refuses what any
     // solve refuses)
-    const bool by_entries = S == 0 && (precision == 0 ? c.spmv_full64 : c.spmv_full32);
+    const bool by_entries = S == 0 && (precision == 0 ? fp64_on_copy(c) : c.spmv_full32 != 0);
     for (int g : {4, 8, 16}) {
         if (S > 0)
             for (int pg : {2, 4, 8}) cands.push_back({g, pg, 0, c.batch_threads});

@@ -196,10 +196,11 @@ const float* bsr_full(Ctx& c, float) {
     return vf;
 }
 // Made anew by every solve: the values are the caller's, who may have written to
-// them since (nothing else of an FP64 solve would notice).  Null where it is
-// switched off or does not fit (152 bytes per upper block).
+// them since (nothing else of an FP64 solve would notice).  Null where the upper
+// blocks in place are the better choice, or where it does not fit (152 bytes per
+// upper block).
 const double* bsr_full(Ctx& c, double) {
-    if (!c.spmv_full64) return nullptr;
+    if (!fp64_on_copy(c)) return nullptr;
     if (!c.have_bsr) bsr_build(c);
     double* vf = c.bsr.full64.try_reserve(full_size<double>(c.bsr));
     if (vf) full_copy(c, vf);

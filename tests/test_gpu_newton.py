@@ -426,6 +426,7 @@ def test_fp64_solve_on_the_upper_blocks(torch_cuda, monkeypatch, cube10, kind, g
     iterate of the solve on the copy, but for the order of the row sums (1e-10,
     as against the oracle above)."""
     print("case: upper-BCOO FP64 solve, precond", kind, "group", group, flush=True)
+    monkeypatch.setenv("SGIPC_SPMV_FULL64", "1")
     ref = make_system(cube10, kind)
     monkeypatch.setenv("SGIPC_SPMV_FULL64", "0")
     s = make_system(cube10, kind)
@@ -439,3 +440,26 @@ def test_fp64_solve_on_the_upper_blocks(torch_cuda, monkeypatch, cube10, kind, g
         x, xo = s.dx.cpu().numpy(), ref.dx.cpu().numpy()
         assert np.linalg.norm(x - xo) <= 1e-10 * np.linalg.norm(xo)
         assert abs(st.rel_residual - so.rel_residual) <= 1e-6 * so.rel_residual
+
+
+def test_fp64_solve_where_the_copy_leaves_the_cache(torch_cuda, monkeypatch):
+    """300,763 rows under block Jacobi, where the solve chooses the blocks in
+    place: twenty iterations are those on the copy and in place when either is
+    forced, up to the order of the row sums."""
+    from sgipc import scene
+    print("case: FP64 solve at 300,763 rows", flush=True)
+    sc = scene.cube_scene(66, seed=1)
+    xs = []
+    for force in ("1", "0", None):
+        if force is None:
+            monkeypatch.delenv("SGIPC_SPMV_FULL64")
+        else:
+            monkeypatch.setenv("SGIPC_SPMV_FULL64", force)
+        s = make_system(sc, 1)
+        s.assemble(); s.convert(); s.build_precond()
+        st = s.solve(tol=1e-30, stop_rule=1, max_iter=21)
+        assert st.iterations == 21
+        xs.append(s.dx.cpu().numpy().copy())
+        del s
+    assert np.linalg.norm(xs[1] - xs[0]) <= 1e-10 * np.linalg.norm(xs[0])
+    assert np.array_equal(xs[2], xs[1])

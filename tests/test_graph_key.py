@@ -1,6 +1,7 @@
-"""Keys of the captured PCG graphs: two MAS hierarchies that launch differently
-have different keys.  The key is host code of the library's own header; a small
-program here compiles it (host side only) and prints keys of made-up tables."""
+"""Host code of the library's own header, compiled here (host side only) into
+small programs: the keys of the captured PCG graphs (two MAS hierarchies that
+launch differently have different keys) and the rule by which an FP64 solve
+takes the copy of its matrix or the blocks in place."""
 import os
 import shutil
 import subprocess
@@ -36,22 +37,56 @@ int main() {
 """
 
 
-def test_graph_keys_tell_hierarchies_apart(tmp_path):
+def _rows(tmp_path, text):
     hipcc = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
     if not (os.path.exists(hipcc) or shutil.which(hipcc)):
         pytest.skip("no hipcc")
-    src = tmp_path / "key.hip"
-    src.write_text(SRC)
-    exe = tmp_path / "key"
+    src = tmp_path / "prog.hip"
+    src.write_text(text)
+    exe = tmp_path / "prog"
     p = subprocess.run([hipcc, "-std=c++17", "-O1", "--offload-arch=gfx950", "--offload-host-only", "-x", "hip",
                         "-I", os.path.join(ROOT, "stiff-gipc_amd", "csrc"), str(src), "-o", str(exe)],
                        capture_output=True, text=True, timeout=120)
     assert p.returncode == 0, p.stderr[-2000:]
     out = subprocess.run([str(exe)], capture_output=True, text=True, timeout=60)
     assert out.returncode == 0, out.stderr
-    rows = [list(map(int, ln.split())) for ln in out.stdout.split("\n") if ln]
-    a, b, again, mask, hi = rows
+    return [list(map(int, ln.split())) for ln in out.stdout.split("\n") if ln]
+
+
+def test_graph_keys_tell_hierarchies_apart(tmp_path):
+    a, b, again, mask, hi = _rows(tmp_path, SRC)
     assert a[:2] == b[:2] == [40, 4] and a[2] != b[2]       # the same totals, another boundary
     assert a[3] != b[3]
     assert again == a
     assert len({a[3], mask[3], hi[3]}) == 3
+
+
+RULE = r"""
+#include "context.hpp"
+#include <cstdio>
+using namespace sgipc;
+int main() {
+    // rows, upper blocks, preconditioner, and its banks and nodes
+    const double rows[][2] = {{125, 665}, {132651, 905301}, {185193, 1267281}, {226981, 1555561}, {300763, 2065141},
+                              {357911, 2460221}, {531441, 3661281}, {2e7, 1.4e8}};
+    for (auto& q : rows)
+        for (int kind : {0, 1, 2, 3})
+            for (int force : {-1, 0, 1}) {
+                Ctx c;
+                c.nb = (int)q[0]; c.K = (int)q[1]; c.precond_kind = kind; c.spmv_full64 = force;
+                c.mas.bank = 16; c.mas.nbanks = (int)(q[0] / 13.3); c.mas.total = 16 * c.mas.nbanks;
+                std::printf("%d %d %d %d\n", c.nb, kind, force, (int)fp64_on_copy(c));
+            }
+}
+"""
+
+
+def test_fp64_copy_rule(tmp_path):
+    """The copy wherever it stays cached and wherever neither does; in place
+    between, from some 200 k to 360 k rows depending on what else an iteration
+    streams; a switch that is set decides alone."""
+    got = {(n, kind, force): on for n, kind, force, on in _rows(tmp_path, RULE)}
+    in_place = {(185193, 2), (226981, 3), (300763, 0), (300763, 1), (357911, 0), (357911, 1)}
+    for (n, kind, force), on in got.items():
+        want = force if force >= 0 else int((n, kind) not in in_place)
+        assert on == want, (n, kind, force, on)

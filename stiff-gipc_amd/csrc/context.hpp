@@ -155,6 +155,8 @@ struct BatchWork {
     DBuf<BatchChunk> chunk;                         // nch
     DBuf<int> scene_chunk;                          // S + 1
     DBuf<double> part_pap, part_rr, part_rz;        // one partial per chunk
+    DBuf<double> fold;                              // their sums per scene (r.z, p.Ap, r.r), where fold_on
+    bool fold_on = false;
     DBuf<double> bb, rz, rz0, tol, segout;  // per scene
     DBuf<int> stop, iters, noconv;                  // per scene
     DBuf<int> ctrl, bad, rstart;                    // C_* words; coupling check counter; row starts

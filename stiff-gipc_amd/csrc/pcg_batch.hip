@@ -10,7 +10,8 @@
 // rows for the SpMV with G lanes per row); one workgroup per chunk writes one
 // partial per dot product, and every wavefront that needs a scene's sum adds
 // its partials in chunk order (deterministic, no FP atomics; the same value
-// everywhere), so no launch only sums.  A stopped scene's rows are left
+// everywhere), so no launch only sums -- except where scenes have hundreds of
+// chunks (kFoldWork).  A stopped scene's rows are left
 // untouched by every later kernel.  The iteration sequence
 //   SpMV (Ap, p.Ap) -> alpha; x, r update (r.r) -> MAS restrict + bank solve
 //   -> collect (z, r.z) -> stop test, beta; p update
@@ -38,6 +39,38 @@ __device__ inline double wave_sum_partials(const double* __restrict__ part, int 
     double v = 0.0;
     for (int i = lo + lane; i < hi; i += 64) v += part[i];
     return __shfl(wave_sum(v), 0, 64);  // (the tree ends in the first lane)
+}
+
+// The same sum in the same order, sixteen partials of a lane in flight: for the
+// one wavefront that sums a scene's partials for all of its chunks
+__device__ inline double wave_sum_partials_ahead(const double* __restrict__ part, int lo, int hi) {
+    constexpr int U = 16;
+    const int lane = threadIdx.x & 63;
+    double v = 0.0;
+    for (int i = lo + lane; i < hi; i += 64 * U) {
+        double q[U];
+#pragma unroll
+        for (int k = 0; k < U; ++k) q[k] = part[min(i + 64 * k, hi - 1)];
+#pragma unroll
+        for (int k = 0; k < U; ++k)
+            if (i + 64 * k < hi) v += q[k];
+    }
+    return __shfl(wave_sum(v), 0, 64);
+}
+
+// Sums of every scene's partials, one wavefront a scene (BEngine::fold)
+__global__ void __launch_bounds__(64) k_bfold(const int* __restrict__ scene_chunk, const int* __restrict__ sstop,
+                                              const double* __restrict__ pa, double* __restrict__ fa,
+                                              const double* __restrict__ pb, double* __restrict__ fb,
+                                              const int* __restrict__ ctrl) {
+    const int s = blockIdx.x;
+    if (ctrl[C_STOP] || sstop[s]) return;
+    const int lo = scene_chunk[s], hi = scene_chunk[s + 1];
+    const double a = wave_sum_partials_ahead(pa, lo, hi), b = pb ? wave_sum_partials_ahead(pb, lo, hi) : 0.0;
+    if (threadIdx.x == 0) {
+        fa[s] = a;
+        if (pb) fb[s] = b;
+    }
 }
 
 // Ap = A p on the chunk's rows, partial p.Ap per chunk
@@ -121,20 +154,23 @@ __global__ void __launch_bounds__(1024) k_bspmv_full(const BatchChunk* __restric
 // sums its scene's partials of r.z and p.Ap for alpha; the scene's first chunk
 // keeps the old r.z for k_bpupdate.  Bound by dependent round trips, like the
 // two kernels below: the vectors are in flight while the partials are summed.
+// (Where the scenes have too many chunks for that, fold_* hold the sums.)
 // With alpha here and the stop test and beta in k_bpupdate, an iteration of 48
 // scenes has six launches instead of eight: 49.4 -> 40.5 us.
 template <typename V>
 __global__ void __launch_bounds__(kBT) k_bupdate(const BatchChunk* __restrict__ chunk, double* __restrict__ x,
                                                  V* __restrict__ r, const V* __restrict__ p, const V* __restrict__ Ap,
                                                  const double* __restrict__ part_rz,
-                                                 const double* __restrict__ part_pap, double* __restrict__ rz,
+                                                 const double* __restrict__ part_pap,
+                                                 const double* __restrict__ fold_rz,
+                                                 const double* __restrict__ fold_pap, double* __restrict__ rz,
                                                  const int* __restrict__ sstop, double* __restrict__ part,
                                                  int* __restrict__ ctrl) {
     __shared__ double sh[kBT / 64];
     const BatchChunk c = chunk[blockIdx.x];
     const int stopped = ctrl[C_STOP], ended = sstop[c.scene];
-    const double rzv = wave_sum_partials(part_rz, c.c0, c.c1);
-    const double pap = wave_sum_partials(part_pap, c.c0, c.c1);
+    const double rzv = fold_rz ? fold_rz[c.scene] : wave_sum_partials(part_rz, c.c0, c.c1);
+    const double pap = fold_rz ? fold_pap[c.scene] : wave_sum_partials(part_pap, c.c0, c.c1);
     constexpr int U = 2;
     const long long i1 = 3LL * c.r1;
     long long i = 3LL * c.r0 + threadIdx.x;
@@ -227,13 +263,15 @@ constexpr int kCTicket = C_NUM + 1;  // workgroups of the start-up scalars done
 template <typename V>
 __global__ void __launch_bounds__(kBT) k_bpupdate(const BatchChunk* __restrict__ chunk, const V* __restrict__ z,
                                                   V* __restrict__ p, const double* __restrict__ part_rr,
-                                                  const double* __restrict__ part_rz, BScal q, int rule,
+                                                  const double* __restrict__ part_rz,
+                                                  const double* __restrict__ fold_rr,
+                                                  const double* __restrict__ fold_rz, BScal q, int rule,
                                                   int* __restrict__ ctrl) {
     const BatchChunk c = chunk[blockIdx.x];
     const int s = c.scene;
     const int stopped = ctrl[C_STOP], ended = q.stop[s], k = ctrl[C_ITER] - 1, maxit = ctrl[C_MAXIT];
-    const double rr = wave_sum_partials(part_rr, c.c0, c.c1);
-    const double rzn = wave_sum_partials(part_rz, c.c0, c.c1);
+    const double rr = fold_rr ? fold_rr[s] : wave_sum_partials(part_rr, c.c0, c.c1);
+    const double rzn = fold_rr ? fold_rz[s] : wave_sum_partials(part_rz, c.c0, c.c1);
     const double rz = q.rz[s], tol = q.tol[s], ref = rule == 0 ? q.rz0[s] : q.bb[s];
     constexpr int U = 2;
     const long long i1 = 3LL * c.r1;
@@ -385,6 +423,18 @@ struct BEngine {
     int rule;
     const float* vfull = nullptr;  // mixed: row-contiguous FP32 copy of both triangles (else the upper BCOO)
 
+    // Per-scene sums by launches of their own instead of by every wavefront that
+    // needs one (build_chunks decides; the same bits)
+    double *fold_rz() { return w.fold_on ? w.fold.p : nullptr; }
+    double *fold_pap() { return w.fold_on ? w.fold.p + S : nullptr; }
+    double *fold_rr() { return w.fold_on ? w.fold.p + 2 * (size_t)S : nullptr; }
+    void fold(const double* pa, double* fa, const double* pb, double* fb) {
+        if (!w.fold_on) return;
+        hipLaunchKernelGGL(k_bfold, dim3(S), dim3(64), 0, c.stream, (const int*)w.scene_chunk.p, (const int*)w.stop.p,
+                           pa, fa, pb, fb, (const int*)w.ctrl.p);
+        SGIPC_LAUNCH_CHECK();
+    }
+
     BScal scal() {
         return BScal{w.bb.p, w.rz.p, w.rz0.p, w.tol.p, w.segout.p, w.stop.p, w.iters.p, w.noconv.p};
     }
@@ -437,13 +487,17 @@ struct BEngine {
             else launch(k_bspmv<8, MV, V>);
         }
         SGIPC_LAUNCH_CHECK();
+        fold(w.part_pap.p, fold_pap(), nullptr, nullptr);
         hipLaunchKernelGGL((k_bupdate<V>), dim3(nch), dim3(kBT), 0, s, (const BatchChunk*)w.chunk.p, x, r,
-                           (const V*)p, (const V*)Ap, (const double*)w.part_rz.p, (const double*)w.part_pap.p, w.rz.p,
+                           (const V*)p, (const V*)Ap, (const double*)w.part_rz.p, (const double*)w.part_pap.p,
+                           (const double*)fold_rz(), (const double*)fold_pap(), w.rz.p,
                            (const int*)w.stop.p, w.part_rr.p, w.ctrl.p);
         SGIPC_LAUNCH_CHECK();
         precond();
+        fold(w.part_rr.p, fold_rr(), w.part_rz.p, fold_rz());
         hipLaunchKernelGGL((k_bpupdate<V>), dim3(nch), dim3(kBT), 0, s, (const BatchChunk*)w.chunk.p, (const V*)z, p,
-                           (const double*)w.part_rr.p, (const double*)w.part_rz.p, scal(), rule, w.ctrl.p);
+                           (const double*)w.part_rr.p, (const double*)w.part_rz.p, (const double*)fold_rr(),
+                           (const double*)fold_rz(), scal(), rule, w.ctrl.p);
         SGIPC_LAUNCH_CHECK();
     }
 
@@ -460,6 +514,7 @@ struct BEngine {
         scalars(B_INIT_BB, w.part_rr.p);
         precond();
         scalars(B_INIT_RZ, w.part_rz.p);
+        fold(w.part_rz.p, fold_rz(), nullptr, nullptr);
         hipLaunchKernelGGL((k_bcast<V, V>), dim3(flat_grid(N)), dim3(256), 0, s, N, p, (const V*)z);
         SGIPC_LAUNCH_CHECK();
     }
@@ -476,7 +531,8 @@ struct BEngine {
                               (const void*)w.part_pap.p, (const void*)w.part_rr.p, (const void*)w.part_rz.p,
                               (const void*)w.bb.p, (const void*)w.rz.p, (const void*)w.rz0.p, (const void*)w.tol.p, (const void*)w.segout.p,
                               (const void*)w.stop.p, (const void*)w.iters.p, (const void*)w.noconv.p,
-                              (const void*)w.ctrl.p, (const void*)w.bank_scene.p})
+                              (const void*)w.ctrl.p, (const void*)w.bank_scene.p,
+                              (const void*)(w.fold_on ? w.fold.p : nullptr)})
             mix((size_t)q);
         mix((size_t)c.stream);
         k.mix(c.mas);
@@ -529,20 +585,34 @@ void seg_to_host(Ctx& c, BatchWork& w, int S, const double* part, std::vector<do
     SGIPC_HIP(hipStreamSynchronize(c.stream));
 }
 
+// Every wavefront of a scene sums the scene's partials itself, which saves two
+// launches an iteration and costs reads in proportion to the square of the
+// scene's chunks: with more than kFoldWork of those squares over all scenes the
+// sums get their launches.  Sixty FP64 iterations, by every wavefront / by
+// launches: 48 scenes of 18 k squares 4.36 / 4.62 ms; one scene of 112 k 3.37 /
+// 3.28; 16 scenes of 233 k 14.8 / 15.0; one scene of 269 k 5.88 / 5.62, of 387 k
+// 4.28 / 3.94, of 1.08 M 5.86 / 5.19, of 34.7 M (753,571 rows) 37.6 / 21.1; 256
+// scenes of 1.05 M 41.7 / 41.1.
+constexpr long long kFoldWork = 250000;
+
 // chunk table: scenes cut into chunks of at most `rows` block rows
 void build_chunks(Ctx& c, BatchWork& w, const std::vector<int>& rs, int rows) {
     const int S = (int)rs.size() - 1;
     std::vector<BatchChunk> chunk;
     std::vector<int> schunk(S + 1, 0);
+    long long squares = 0;
     for (int s = 0; s < S; ++s) {
         const int c0 = (int)chunk.size(), c1 = c0 + (rs[s + 1] - rs[s] + rows - 1) / rows;
         schunk[s] = c0;
+        squares += (long long)(c1 - c0) * (c1 - c0);
         for (int r0 = rs[s]; r0 < rs[s + 1]; r0 += rows)
             chunk.push_back(BatchChunk{r0, std::min(r0 + rows, rs[s + 1]), s, c0, c1});
     }
     const int nch = (int)chunk.size();
     schunk[S] = nch;
     w.nch = nch;
+    w.fold_on = squares > kFoldWork;
+    if (w.fold_on) w.fold.reserve(3 * (size_t)S);
     w.chunk.reserve(nch + 1);
     w.scene_chunk.reserve(S + 1);
     if (nch) SGIPC_HIP(hipMemcpy(w.chunk.p, chunk.data(), sizeof(BatchChunk) * nch, hipMemcpyHostToDevice));

@@ -366,3 +366,46 @@ def test_autotune_of_one_system_keeps_a_group_without_effect(torch_cuda, cube4):
             s.ctx.call("sgipc_set_schedule", group, per_graph)
             tune(precision)
             assert (g.value, pg.value) == (group, per_graph)
+
+
+@pytest.mark.parametrize("mixed", [False, True])
+def test_scene_of_hundreds_of_chunks(torch_cuda, mixed):
+    """A scene of some 36,000 rows beside small ones: its sums are formed by
+    every wavefront with 128 rows a chunk and by launches of their own with 64
+    (more than 500 chunks).  FP64: the same iteration counts, and after some ten
+    iterations the same iterates up to the order of the sums (1e-10, as for the
+    chunk sizes above).  Mixed: every scene reaches the tolerance of its FP64
+    residual.  A scene with a zero right-hand side stays zero, a budget ends
+    every scene, and a repeated solve repeats bitwise."""
+    from sgipc import capi, scene
+    from sgipc.system import NewtonSystem
+    print("case: batched scene of hundreds of chunks, mixed", mixed, flush=True)
+    scs = scene.batch_scenes(3, 9, 150, 400) + scene.batch_scenes(1, 5, 36000, 36001)
+    u, rs = scene.union_scene(scs)
+    assert (-(-np.diff(rs) // 64)).max() > 500 and (-(-np.diff(rs) // 128)).max() < 500
+    s = NewtonSystem(u, "cuda:0", precond=capi.PRECOND_MAS)
+    s.ctx.call("sgipc_set_deterministic", 1)      # (one preconditioner for every run of this test)
+    s.assemble(); s.convert(); s.build_precond()
+    s.b[3 * rs[1]:3 * rs[2]] = 0.0
+    prec, S = (capi.PRECISION_MIXED if mixed else capi.PRECISION_FP64), len(scs)
+    tol = 1e-6 if mixed else 1e-4
+    for t, rule, max_iter in ((tol, int(mixed), 3000), (1e-30, 1, 9)):
+        st, x = {}, {}
+        for group in (8, 16, 16):
+            s.ctx.call("sgipc_set_schedule", group, 4)
+            r, xg = _solve_batched(s, rs, prec, t, rule, max_iter)
+            q = [(r[i].iterations, r[i].converged) for i in range(S)]
+            if group in st:
+                assert st[group] == q and np.array_equal(x[group], xg)
+            st[group], x[group] = q, xg
+            assert q[1] == (0, 1) and not np.any(xg[3 * rs[1]:3 * rs[2]])
+            if max_iter == 9:
+                assert all(q[i] == (9, 0) for i in (0, 2, 3)), q
+            else:
+                assert all(c for _, c in q), q
+                if mixed:
+                    assert all(r[i].rel_residual <= tol for i in range(S))
+        if not mixed:
+            assert st[8] == st[16], (st[8], st[16])
+            d = np.linalg.norm(x[8] - x[16]) / np.linalg.norm(x[8])
+            assert d <= 1e-10, d

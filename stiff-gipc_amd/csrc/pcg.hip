@@ -268,6 +268,7 @@ __global__ void __launch_bounds__(kThreads) k_simple_precond_dot(long long N, co
 // for two and four against 19.8 us.
 constexpr int kFT = 256;          // threads
 constexpr int kFRows = 72;        // block rows per chunk, at most (three components each, of 256 threads)
+constexpr int kFRowsBodies = 24;  // the same with affine bodies
 constexpr int kFBatch = 1024;     // entries per LDS batch
 constexpr int kFChunks = 4096;    // workgroups (p.Ap partials), at most
 
@@ -489,9 +490,17 @@ struct Engine {
     // so it is within 4 % of the best at both ends, and up to 28 % off it in
     // FP64 between 20 k and 44 k rows, where larger chunks do better.  (Solves
     // without a preconditioner: the matrix stays in the Infinity Cache.)
+    // The rows of affine bodies come first and have hundreds of entries (about 250
+    // for 64 bodies in columns), and a chunk's entries pass through one workgroup a
+    // batch at a time, its rows summed by g lanes: 72 such rows took longer than all
+    // the others.  With bodies a chunk has at most 24 rows.  An iteration of FP64
+    // / mixed, with 8, 16, 24, 32 and 72 rows: 214,477 rows, 64 bodies 135 / 76, 118
+    // / 68, 114 / 65, 120 / 70 and 161 / 98 us; 106,117 rows 62 / 49, 55 / 43, 53 /
+    // 45, 54 / 43 and 69 / 56; 360,637 rows 207 / 140, 181 / 119, 175 / 119, 190 /
+    // 129 and 272 / 201.
     void use_full(const V* vf) {
         vfull = vf;
-        rF = std::max(8, std::min(kFRows, (int)div_up(c.nb, 1920)));
+        rF = std::max(8, std::min(c.abd.nb > 0 ? kFRowsBodies : kFRows, (int)div_up(c.nb, 1920)));
         nF = (int)div_up(c.nb, rF);
         gF = 1;
         while (gF < 64 && 2 * gF * 3 * rF <= kFT) gF *= 2;

@@ -215,3 +215,30 @@ def test_newton_solve_converges(torch_cuda):
     for b in range(s.nb):
         Am = q[b, 3:].reshape(3, 3)
         assert np.abs(Am @ Am.T - np.eye(3)).max() < 1e-6
+
+
+@pytest.mark.parametrize("mixed", [False, True])
+def test_large_slab_under_bodies(torch_cuda, monkeypatch, mixed):
+    """64 bodies on a slab of 56 k rows: rows of hundreds of entries, several to a
+    chunk of the SpMV by entries, next to short ones.  The solve on the copy
+    and the one on the upper blocks reach the tolerance of the true residual,
+    which is formed on the blocks in place, and repeat bitwise."""
+    from sgipc import capi, scene
+    from sgipc.hybrid import HybridSystem
+    print("case: bodies on a large slab, mixed", mixed, flush=True)
+    hs = scene.hybrid_scene(cells=(60, 14, 60), lattice=4)
+    for copy in ("1", "0"):
+        monkeypatch.setenv("SGIPC_SPMV_FULL32" if mixed else "SGIPC_SPMV_FULL64", copy)
+        s = HybridSystem(hs, "cuda:0", precond=capi.PRECOND_MAS)
+        assert s.detect() > 0 and s.nbr > 46080
+        s.ctx.call("sgipc_set_deterministic", 1)
+        s.ctx.call("sgipc_set_inner_tol", 1e-4)
+        kw = dict(tol=1e-6, stop_rule=capi.STOP_TRUE_REL, max_iter=5000,
+                  precision=capi.PRECISION_MIXED if mixed else capi.PRECISION_FP64)
+        st = s.newton_step(**kw)
+        x = s.dx.clone()
+        # the FP64 recurrence's residual drifts from the true one by rounding (half a digit of slack)
+        assert st.converged and st.rel_residual <= 3e-6, st.rel_residual
+        again = s.solve(**kw)
+        assert again.iterations == st.iterations and torch_cuda.equal(s.dx, x)
+        del s

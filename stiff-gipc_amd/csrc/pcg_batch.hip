@@ -157,7 +157,7 @@ __global__ void __launch_bounds__(1024) k_bspmv_full(const BatchChunk* __restric
 // (Where the scenes have too many chunks for that, fold_* hold the sums.)
 // With alpha here and the stop test and beta in k_bpupdate, an iteration of 48
 // scenes has six launches instead of eight: 49.4 -> 40.5 us.
-template <typename V>
+template <typename V, bool FOLD>
 __global__ void __launch_bounds__(kBT) k_bupdate(const BatchChunk* __restrict__ chunk, double* __restrict__ x,
                                                  V* __restrict__ r, const V* __restrict__ p, const V* __restrict__ Ap,
                                                  const double* __restrict__ part_rz,
@@ -169,8 +169,8 @@ __global__ void __launch_bounds__(kBT) k_bupdate(const BatchChunk* __restrict__ 
     __shared__ double sh[kBT / 64];
     const BatchChunk c = chunk[blockIdx.x];
     const int stopped = ctrl[C_STOP], ended = sstop[c.scene];
-    const double rzv = fold_rz ? fold_rz[c.scene] : wave_sum_partials(part_rz, c.c0, c.c1);
-    const double pap = fold_rz ? fold_pap[c.scene] : wave_sum_partials(part_pap, c.c0, c.c1);
+    const double rzv = FOLD ? fold_rz[c.scene] : wave_sum_partials(part_rz, c.c0, c.c1);
+    const double pap = FOLD ? fold_pap[c.scene] : wave_sum_partials(part_pap, c.c0, c.c1);
     constexpr int U = 2;
     const long long i1 = 3LL * c.r1;
     long long i = 3LL * c.r0 + threadIdx.x;
@@ -260,7 +260,7 @@ constexpr int kCTicket = C_NUM + 1;  // workgroups of the start-up scalars done
 // same decision from the same sums; the scene's first chunk writes it, and the
 // last scene to stop sets the stop word.  (A chunk that starts later and sees
 // its scene stopped would have left p alone as well.)
-template <typename V>
+template <typename V, bool FOLD>
 __global__ void __launch_bounds__(kBT) k_bpupdate(const BatchChunk* __restrict__ chunk, const V* __restrict__ z,
                                                   V* __restrict__ p, const double* __restrict__ part_rr,
                                                   const double* __restrict__ part_rz,
@@ -270,8 +270,8 @@ __global__ void __launch_bounds__(kBT) k_bpupdate(const BatchChunk* __restrict__
     const BatchChunk c = chunk[blockIdx.x];
     const int s = c.scene;
     const int stopped = ctrl[C_STOP], ended = q.stop[s], k = ctrl[C_ITER] - 1, maxit = ctrl[C_MAXIT];
-    const double rr = fold_rr ? fold_rr[s] : wave_sum_partials(part_rr, c.c0, c.c1);
-    const double rzn = fold_rr ? fold_rz[s] : wave_sum_partials(part_rz, c.c0, c.c1);
+    const double rr = FOLD ? fold_rr[s] : wave_sum_partials(part_rr, c.c0, c.c1);
+    const double rzn = FOLD ? fold_rz[s] : wave_sum_partials(part_rz, c.c0, c.c1);
     const double rz = q.rz[s], tol = q.tol[s], ref = rule == 0 ? q.rz0[s] : q.bb[s];
     constexpr int U = 2;
     const long long i1 = 3LL * c.r1;
@@ -488,16 +488,24 @@ struct BEngine {
         }
         SGIPC_LAUNCH_CHECK();
         fold(w.part_pap.p, fold_pap(), nullptr, nullptr);
-        hipLaunchKernelGGL((k_bupdate<V>), dim3(nch), dim3(kBT), 0, s, (const BatchChunk*)w.chunk.p, x, r,
-                           (const V*)p, (const V*)Ap, (const double*)w.part_rz.p, (const double*)w.part_pap.p,
-                           (const double*)fold_rz(), (const double*)fold_pap(), w.rz.p,
-                           (const int*)w.stop.p, w.part_rr.p, w.ctrl.p);
+        auto update = [&](auto kern) {
+            hipLaunchKernelGGL(kern, dim3(nch), dim3(kBT), 0, s, (const BatchChunk*)w.chunk.p, x, r, (const V*)p,
+                               (const V*)Ap, (const double*)w.part_rz.p, (const double*)w.part_pap.p,
+                               (const double*)fold_rz(), (const double*)fold_pap(), w.rz.p, (const int*)w.stop.p,
+                               w.part_rr.p, w.ctrl.p);
+        };
+        if (w.fold_on) update(k_bupdate<V, true>);
+        else update(k_bupdate<V, false>);
         SGIPC_LAUNCH_CHECK();
         precond();
         fold(w.part_rr.p, fold_rr(), w.part_rz.p, fold_rz());
-        hipLaunchKernelGGL((k_bpupdate<V>), dim3(nch), dim3(kBT), 0, s, (const BatchChunk*)w.chunk.p, (const V*)z, p,
-                           (const double*)w.part_rr.p, (const double*)w.part_rz.p, (const double*)fold_rr(),
-                           (const double*)fold_rz(), scal(), rule, w.ctrl.p);
+        auto direction = [&](auto kern) {
+            hipLaunchKernelGGL(kern, dim3(nch), dim3(kBT), 0, s, (const BatchChunk*)w.chunk.p, (const V*)z, p,
+                               (const double*)w.part_rr.p, (const double*)w.part_rz.p, (const double*)fold_rr(),
+                               (const double*)fold_rz(), scal(), rule, w.ctrl.p);
+        };
+        if (w.fold_on) direction(k_bpupdate<V, true>);
+        else direction(k_bpupdate<V, false>);
         SGIPC_LAUNCH_CHECK();
     }
 
